@@ -67,13 +67,9 @@ def ring_table(num_points_approx: int, radius: float):
     points_per_ring, radii, div_angle = _ring_counts(num_points_approx, radius)
     n = int(points_per_ring.sum())
     ring_first = np.concatenate([[0], np.cumsum(points_per_ring)[:-1]]).astype(np.int64)
-    seg = [0]
-    for length in points_per_ring:
-        nxt = seg[-1] + int(length) + 1
-        if nxt >= n:
-            break
-        seg.append(nxt)
-    return radii.astype(np.float64), div_angle.astype(np.float64), ring_first, np.array(seg, np.int64), n
+    seg = np.concatenate([[0], np.cumsum(points_per_ring + 1)]).astype(np.int64)
+    seg = seg[: max(1, int(np.searchsorted(seg, n)))]  # the restarts before point n
+    return radii.astype(np.float64), div_angle.astype(np.float64), ring_first, seg, n
 
 
 def _dtype_code(dtype) -> int:
@@ -87,12 +83,14 @@ def _dtype_code(dtype) -> int:
 def device_rings(num_points_approx: int, radius: float, kind: int, offset_xy, device, dtype=torch.float64):
     """(x, y, dx, dy) device tensors of a ring source generated on the GPU."""
     radii, steps, ring_first, seg_first, n = ring_table(num_points_approx, radius)
-    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
-    tr, ts, trf, tsf = t(radii), t(steps), t(ring_first), t(seg_first)
+    # the four tables (8-byte entries) in one buffer: one copy to the device
+    parts = (radii, steps, ring_first, seg_first)
+    table = torch.from_numpy(np.concatenate([p.view(np.int64) for p in parts])).to(device)
+    tr, ts, trf, tsf = table.data_ptr() + 8 * np.cumsum([0] + [len(p) for p in parts[:3]])
     out = [torch.empty(n, dtype=dtype, device=device) for _ in range(4)]
-    st = _lib.load().tg_source_rings(tr.data_ptr(), ts.data_ptr(), trf.data_ptr(), len(radii), tsf.data_ptr(),
-                                     len(seg_first), n, kind, float(offset_xy[0]), float(offset_xy[1]),
-                                     _dtype_code(dtype), *[o.data_ptr() for o in out], _lib.stream_ptr(device))
+    st = _lib.load().tg_source_rings(int(tr), int(ts), int(trf), len(radii), int(tsf), len(seg_first), n, kind,
+                                     float(offset_xy[0]), float(offset_xy[1]), _dtype_code(dtype),
+                                     *[o.data_ptr() for o in out], _lib.stream_ptr(device))
     _lib.check(st, "tg_source_rings")
     return out
 
@@ -182,7 +180,7 @@ class Source(HasParamsMixin):
         if device is None:
             device = torch.device("cuda") if torch.cuda.is_available() else torch.device("cpu")
         device = torch.device(device)
-        if device.type == "cuda" and self._device_kind is not None and (random or ring_table(num, 1.0)[4] > 1):
+        if device.type == "cuda" and self._device_kind is not None and (random or _ring_counts(num, 1.0)[0].sum() > 1):
             off = self.offset_xy
             if random:
                 x, y, dx, dy = device_disc(max(1, int(num)), self._disc_radius(), self._device_kind, off, device,
