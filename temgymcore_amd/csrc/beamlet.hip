@@ -431,6 +431,13 @@ __global__ __launch_bounds__(256) void beamlet_moment_kernel(const tg_beamlet_co
   }
 }
 
+// The chain rule of one beamlet (blockIdx.x, lane) along one direction
+// (blockIdx.y): a forward-mode pass of the coefficient algebra.  Bound: the
+// latency of a few thousand dependent f64 instructions (divisions, square
+// roots, sincos), so the 31 directions of a beamlet run side by side: 2,048
+// beamlets take 15 us, where all directions in one lane kept 32 wavefronts
+// busy for 268 us.  The direction is uniform over a workgroup, so its seeds
+// are scalar selects.
 __global__ __launch_bounds__(64) void beamlet_grad_kernel(const double* __restrict__ params, int64_t n,
                                                           const double* __restrict__ abcd, int64_t abcd_stride,
                                                           int32_t mode, double m0, double m1, double m2, double m3,
@@ -461,38 +468,38 @@ __global__ __launch_bounds__(64) void beamlet_grad_kernel(const double* __restri
   G[5] = S0;
   const double ar = p[5], ai = p[6];
   double* gp = grad_params + i * TG_BEAMLET_NPARAM;
-  gp[5] = S0.re;   // u = amp exp(Phi'): dL/d amp_re = Re sum W exp(Phi')
-  gp[6] = -S0.im;  //                    dL/d amp_im = Re(i sum W exp(Phi'))
-  gp[13] = gp[14] = gp[15] = 0.0;
   // directions: parameter columns 0-4 and 7-12, then ray-transfer entries 0-19
-  const int n_dir = prop ? 11 + 20 : 11;
-  for (int q = 0; q < n_dir; ++q) {
-    const int col = q < 5 ? q : (q < 11 ? q + 2 : -1);
-    const int ent = q < 11 ? -1 : q - 11;
-    dual pd[13], Td[25];
-#pragma unroll
-    for (int k = 0; k < 13; ++k) pd[k] = dual(p[k], k == col ? 1.0 : 0.0);
-    if (prop) {
-#pragma unroll
-      for (int e = 0; e < 25; ++e) Td[e] = dual(T[e], e == ent ? 1.0 : 0.0);
+  const int q = blockIdx.y;
+  if (q == 0) {
+    gp[5] = S0.re;   // u = amp exp(Phi'): dL/d amp_re = Re sum W exp(Phi')
+    gp[6] = -S0.im;  //                    dL/d amp_im = Re(i sum W exp(Phi'))
+    gp[13] = gp[14] = gp[15] = 0.0;
+    if (grad_abcd) {
+      for (int e = prop ? 20 : 0; e < 25; ++e) grad_abcd[i * 25 + e] = 0.0;
     }
-    cx<dual> d6[6];
-    phi_coefficients<dual>(pd, Td, mode, m, mk(dual(1.0), dual(0.0)), d6);
-    double sr = 0.0, si = 0.0;  // sum_k G_k dc_k
+  }
+  const int col = q < 5 ? q : (q < 11 ? q + 2 : -1);
+  const int ent = q < 11 ? -1 : q - 11;
+  dual pd[13], Td[25];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      sr += G[k].re * d6[k].re.t - G[k].im * d6[k].im.t;
-      si += G[k].re * d6[k].im.t + G[k].im * d6[k].re.t;
-    }
-    const double g = ar * sr - ai * si;  // Re[amp sum_k G_k dc_k]
-    if (col >= 0)
-      gp[col] = g;
-    else if (grad_abcd)
-      grad_abcd[i * 25 + ent] = g;
+  for (int k = 0; k < 13; ++k) pd[k] = dual(p[k], k == col ? 1.0 : 0.0);
+  if (prop) {
+#pragma unroll
+    for (int e = 0; e < 25; ++e) Td[e] = dual(T[e], e == ent ? 1.0 : 0.0);
   }
-  if (grad_abcd) {
-    for (int e = prop ? 20 : 0; e < 25; ++e) grad_abcd[i * 25 + e] = 0.0;
+  cx<dual> d6[6];
+  phi_coefficients<dual>(pd, Td, mode, m, mk(dual(1.0), dual(0.0)), d6);
+  double sr = 0.0, si = 0.0;  // sum_k G_k dc_k
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    sr += G[k].re * d6[k].re.t - G[k].im * d6[k].im.t;
+    si += G[k].re * d6[k].im.t + G[k].im * d6[k].re.t;
   }
+  const double g = ar * sr - ai * si;  // Re[amp sum_k G_k dc_k]
+  if (col >= 0)
+    gp[col] = g;
+  else
+    grad_abcd[i * 25 + ent] = g;
 }
 
 int splits_for(int64_t n, int64_t H, int64_t W) {
@@ -669,7 +676,9 @@ extern "C" int tg_beamlet_backward(const double* params, int64_t n, const double
   hipLaunchKernelGGL(beamlet_moment_kernel, dim3((unsigned)tg::cdiv(n, kBeamletsPerMomentBlock)), dim3(256), 0, s,
                      unit, n, (int32_t)height, (int32_t)width, w, moments);
   TG_LAUNCH_CHECK("beamlet_moment_kernel launch");
-  hipLaunchKernelGGL(beamlet_grad_kernel, dim3((unsigned)tg::cdiv(n, 64)), dim3(64), 0, s, params, n, abcd,
+  // the 20 ray-transfer directions only where their gradient is wanted
+  const unsigned n_dir = grad_abcd != nullptr ? 31 : 11;
+  hipLaunchKernelGGL(beamlet_grad_kernel, dim3((unsigned)tg::cdiv(n, 64), n_dir), dim3(64), 0, s, params, n, abcd,
                      abcd_stride, mode, pix2m[0], pix2m[1], pix2m[2], pix2m[3], pix2m[4], pix2m[5], (int32_t)height,
                      (int32_t)width, unit, moments, grad_params, grad_abcd);
   TG_LAUNCH_CHECK("beamlet_grad_kernel launch");

@@ -189,3 +189,24 @@ def test_backward_rejects_bad_arguments(device):
         beamlet_field(params, grid, MODE_PROPAGATED, one, 5)
     with pytest.raises(ValueError, match=r"shape \[n, 16\]"):
         beamlet_field(params[:, :15], grid, MODE_INPUT)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 200])
+def test_parameter_gradient_without_the_matrix_gradient(device, n):
+    """The parameter directions alone (a shared matrix whose gradient is not
+    wanted) give the bits they have beside the ray-transfer directions, and
+    every beamlet's row is the one it has in a batch of its own."""
+    rng = np.random.default_rng(90 + n)
+    p = torch.from_numpy(_rays(n, rng)).to(device)
+    T = np.eye(5)
+    T[0, 2] = T[1, 3] = 1e-3
+    A = torch.from_numpy(T).to(device)
+    grid = Detector(z=1e-3, pixel_size=(3e-8, 3e-8), shape=(33, 47))
+    g = torch.from_numpy((rng.normal(size=(33, 47)) + 1j * rng.normal(size=(33, 47))).astype(np.complex64)).to(device)
+    both, gT = beamlet_backward(p, grid, MODE_PROPAGATED, g, A, 0, want_abcd=True)
+    alone, none = beamlet_backward(p, grid, MODE_PROPAGATED, g, A, 0)
+    assert none is None and gT.shape == (n, 25)
+    torch.testing.assert_close(alone, both, rtol=0, atol=0)
+    last, last_T = beamlet_backward(p[n - 1:].contiguous(), grid, MODE_PROPAGATED, g, A, 0, want_abcd=True)
+    torch.testing.assert_close(last[0], both[n - 1], rtol=0, atol=0)
+    torch.testing.assert_close(last_T[0], gT[n - 1], rtol=0, atol=0)
