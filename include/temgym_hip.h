@@ -226,6 +226,15 @@ typedef struct tg_stem_geometry {
 int tg_stem_forward(const tg_stem_geometry* g, const double* params, const float* image, float* coords,
                     float* values, float* image4d, void* stream);
 
+/* The simulated 4D dataset alone: image4d [S, det_h, det_w] f32 (camera
+ * length 0) is overwritten, every pixel once, with the deposit that
+ * tg_stem_forward accumulates.  Detector rows hold at most
+ * tg_stem_dataset_max_width() pixels (wider: TG_EINVAL, use
+ * tg_stem_forward on a cleared image). */
+int32_t tg_stem_dataset_max_width(void);
+int tg_stem_dataset(const tg_stem_geometry* geom, const double* params, const float* image, float* image4d,
+                    void* stream);
+
 /* Descan / geometry fit, forward and adjoint in one pass over the targets.
  *   targets  [n_cam, S, J, 2] f32 target detector coordinates
  *   workspace tg_stem_fit_workspace(g) bytes of f64: starts with the

@@ -47,6 +47,8 @@ class StemGeometry(ctypes.Structure):
 _P = ctypes.c_void_p
 _lib.register_signatures({
     "tg_stem_forward": (ctypes.c_int, [ctypes.POINTER(StemGeometry), _P, _P, _P, _P, _P, _P]),
+    "tg_stem_dataset_max_width": (ctypes.c_int32, []),
+    "tg_stem_dataset": (ctypes.c_int, [ctypes.POINTER(StemGeometry), _P, _P, _P, _P]),
     "tg_stem_fit_workspace": (ctypes.c_int64, [ctypes.POINTER(StemGeometry)]),
     "tg_stem_fit": (ctypes.c_int, [ctypes.POINTER(StemGeometry), _P, _P, _P, _P, _P]),
     "tg_stem_backproject": (ctypes.c_int, [ctypes.POINTER(StemGeometry), _P, _P, ctypes.c_int32, _P, _P, _P]),
@@ -255,10 +257,6 @@ def stem_forward(model: STEMModel, params: torch.Tensor | None = None, sample: t
             if (not isinstance(t, torch.Tensor) or tuple(t.shape) != shapes[name] or t.dtype != torch.float32
                     or not t.is_cuda or not t.is_contiguous()):
                 raise ValueError(f"out[{name!r}] must be a contiguous device float32 tensor of shape {shapes[name]}")
-    if image4d:
-        # the kernel adds every ray's deposit into the image: it starts from
-        # zero on every call (a fill kernel, so the call stays graph-capturable)
-        res["image4d"].zero_()
     if (values or image4d) and sample is None:
         raise ValueError("a sample image is needed for values / image4d")
     if sample is not None:
@@ -266,10 +264,22 @@ def stem_forward(model: STEMModel, params: torch.Tensor | None = None, sample: t
             raise ValueError(f"sample must be a device float32 tensor of shape {tuple(model.sample_shape)}")
         sample = sample.contiguous()
     g = model.geometry()
-    st = lib.tg_stem_forward(ctypes.byref(g), params.data_ptr(), _ptr(sample), _ptr(res.get("coords") if coords else None),
-                             _ptr(res.get("values") if values else None),
-                             _ptr(res.get("image4d") if image4d else None), _lib.stream_ptr(device))
-    _lib.check(st, "tg_stem_forward")
+    stream = _lib.stream_ptr(device)
+    if image4d and g.det_w <= lib.tg_stem_dataset_max_width():
+        # the dataset is written by a kernel of its own, every pixel once
+        st = lib.tg_stem_dataset(ctypes.byref(g), params.data_ptr(), _ptr(sample), _ptr(res["image4d"]), stream)
+        _lib.check(st, "tg_stem_dataset")
+        image4d = False
+    elif image4d:
+        # very wide detectors: deposited with atomics onto a cleared image (a
+        # fill kernel, so the call stays graph-capturable)
+        res["image4d"].zero_()
+    if coords or values or image4d:
+        st = lib.tg_stem_forward(ctypes.byref(g), params.data_ptr(), _ptr(sample),
+                                 _ptr(res.get("coords") if coords else None),
+                                 _ptr(res.get("values") if values else None),
+                                 _ptr(res.get("image4d") if image4d else None), stream)
+        _lib.check(st, "tg_stem_forward")
     return res
 
 

@@ -447,3 +447,73 @@ def test_fit_terms_are_the_per_scan_position_shares(device):
     rows = terms.cpu().numpy()
     assert np.all(np.abs(rows.sum(axis=1) - out.cpu().numpy()) <= 1e-12 * np.abs(rows).sum(axis=1) + 1e-300)
     assert np.all(rows[-1] >= 0)
+
+
+@pytest.mark.parametrize("det_shape, n_side, rot", [
+    ((1, 1), 8, 0.0), ((7, 5), 30, 0.0), ((250, 253), 62, 0.0), ((64, 256), 64, 0.0), ((33, 257), 20, 0.0),
+    ((3, 8192), 64, 0.0), ((2, 8193), 64, 0.0), ((97, 101), 2, 0.0), ((120, 131), 46, 33.0), ((128, 60), 64, 90.0)])
+def test_dataset_bands_vs_forward_deposit(device, det_shape, n_side, rot):
+    """The dataset kernel (bands of rows in LDS, written once) on detectors that
+    do not divide into its bands, misaligned rows, one-row bands, the width
+    past which the deposit goes through memory, and rotated detectors (whose
+    rows mix both slopes): the deposit of the same call's coordinates and
+    values, within one f32 rounding of each term (a pixel's terms are added in
+    any order); buffers that held other numbers are overwritten."""
+    import ctypes
+
+    model, sample = stem.reference_workload(n_cam=1, scan_shape=(3, 5), det_shape=det_shape, n_side=n_side,
+                                            det_pixel=6e-4 / det_shape[0])
+    sample_t = torch.from_numpy(sample).to(device)
+    params = stem.params_tensor(model, device)
+    g = model.geometry()
+    if rot:
+        R_ = np.deg2rad(rot)
+        rows = np.array(g.det_m).reshape(2, 3)
+        c = np.array([(det_shape[0] - 1) / 2, (det_shape[1] - 1) / 2])
+        lin = np.array([[np.cos(R_), np.sin(R_)], [-np.sin(R_), np.cos(R_)]]) @ rows[:, :2]
+        g.det_m[:] = np.column_stack([lin, c]).reshape(-1).tolist()
+    res = stem.stem_forward(model, params, sample_t, coords=True, values=True)
+    img = torch.full((model.n_scan,) + det_shape, float("nan"), device=device)
+    lib = stem._lib.load()
+    wide = det_shape[1] > lib.tg_stem_dataset_max_width()
+    st = lib.tg_stem_dataset(ctypes.byref(g), params.data_ptr(), sample_t.data_ptr(), img.data_ptr(),
+                             stem._lib.stream_ptr(device))
+    assert st == (-1 if wide else 0)
+    if wide:
+        img = stem.stem_forward(model, params, sample_t, coords=False, image4d=True)["image4d"]
+    xy = res["coords"].double().cpu().numpy()[0]
+    v = res["values"].double().cpu().numpy()
+    m = np.array(g.det_m)
+    py = np.rint((m[0] * xy[..., 1] + m[1] * xy[..., 0]) + m[2])
+    px = np.rint((m[3] * xy[..., 1] + m[4] * xy[..., 0]) + m[5])
+    ok = (py >= 0) & (py < det_shape[0]) & (px >= 0) & (px < det_shape[1])
+    s = np.broadcast_to(np.arange(model.n_scan)[:, None], ok.shape)
+    ref, size, n = np.zeros(img.shape), np.zeros(img.shape), np.zeros(img.shape)
+    at = (s[ok], py[ok].astype(int), px[ok].astype(int))
+    np.add.at(ref, at, v[ok])
+    np.add.at(size, at, np.abs(v[ok]))
+    np.add.at(n, at, 1)
+    assert ok.any()
+    assert np.all(np.abs(img.double().cpu().numpy() - ref) <= 2.0 ** -24 * n * size)
+
+
+def test_dataset_of_undefined_parameters_bins_to_pixel_zero(device):
+    """NaN detector positions cast to pixel (0, 0), as the forward's binning
+    does: each position's whole sum lies there (256 values within pi, added in
+    any order: 256 roundings of at most 256 pi 2^-24)."""
+    model, sample = stem.reference_workload(n_cam=1, scan_shape=(1, 2), n_side=16, det_shape=(40, 300))
+    params = stem.params_tensor(model, device)
+    params[0] = float("nan")
+    img = stem.stem_forward(model, params, torch.from_numpy(sample).to(device), coords=False, image4d=True)["image4d"]
+    ref = torch.zeros_like(img)
+    g = model.geometry()
+    import ctypes
+
+    sample_t = torch.from_numpy(sample).to(device)
+    st = stem._lib.load().tg_stem_forward(ctypes.byref(g), params.data_ptr(), sample_t.data_ptr(), None, None,
+                                          ref.data_ptr(), stem._lib.stream_ptr(device))
+    assert st == 0
+    torch.cuda.synchronize()
+    assert img[:, 0, 0].abs().min() > 0  # every ray's value, on pixel (0, 0)
+    assert (img[:, 1:].abs().sum() + img[:, 0, 1:].abs().sum()) == 0
+    assert (img - ref).abs().max() <= 2 * 256 * 256 * np.pi * 2.0 ** -24
