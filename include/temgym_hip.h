@@ -130,6 +130,46 @@ typedef struct tg_bin_spec {
  * Ray-count 0 is a no-op. */
 int tg_ray_program_run(const tg_program* prog, const tg_bin_spec* bin, void* stream);
 
+/* A column of standard elements over rays held as contiguous arrays: the
+ * program such a model compiles to, element by element (the same operations,
+ * each rounded once to the dtype; immediates rounded to it on the host).  A
+ * step is an optional drift  x += dx d, y += dy d (and pathlength += d with
+ * TG_STEP_DRIFT_PATH), then its element. */
+#define TG_MAX_STEP 64
+enum tg_step_kind {
+  TG_STEP_NONE = 0,    /* the drift alone                                           */
+  TG_STEP_LENS = 1,    /* dx = -x/p0 + dx (likewise y), path -= (x^2 + y^2)/p1      */
+  TG_STEP_DEFLECT = 2, /* path = path + dx x + dy y, then dx += p0, dy += p1        */
+  TG_STEP_ROTATE = 3,  /* (x, y) and (dx, dy) by p0 = cos, p1 = sin                 */
+  TG_STEP_SHIFT = 4,   /* x += p0, y += p1, dx += p2, dy += p3                      */
+  TG_STEP_BIPRISM = 5  /* path = path + dx x + dy y, then dx += sign(x) p0          */
+};
+enum tg_step_flag { TG_STEP_DRIFT = 1, TG_STEP_DRIFT_PATH = 2 };
+
+typedef struct tg_step {
+  int32_t kind, flags;
+  double d, p[4];
+} tg_step;
+
+typedef struct tg_column {
+  int32_t dtype;          /* tg_dtype of every array                              */
+  int32_t n_step;
+  int64_t n;              /* number of rays                                       */
+  const void* in[5];      /* x, y, dx, dy, pathlength (NULL: uniform)             */
+  void* out[5];           /* the same fields after the column (NULL: not stored)  */
+  double pathlength;      /* uniform pathlength where in[4] is NULL               */
+  tg_step step[TG_MAX_STEP];
+} tg_column;
+
+/* Run `column` over its rays; optionally bin the final x, y (the register and
+ * uniform fields of `bin` are ignored; unit weights only).  `workspace` (16-byte
+ * aligned, tg_ray_column_workspace bytes; may be NULL) serves many rays on a
+ * detector too large for one workgroup's LDS, which are counted in two passes;
+ * without it they are counted with memory atomics, to the same result. */
+int64_t tg_ray_column_workspace(int64_t n, int64_t height, int64_t width, int32_t acc_dtype);
+int tg_ray_column_run(const tg_column* column, const tg_bin_spec* bin, void* workspace, int64_t workspace_bytes,
+                      void* stream);
+
 /* Number of compute units of the current device (cached per device). */
 int32_t tg_device_cu_count(void);
 

@@ -65,6 +65,25 @@ class Program(ctypes.Structure):
     ]
 
 
+# Columns of standard elements: step kinds and flags (tg_step_kind, tg_step_flag)
+TG_MAX_STEP = 64
+STEP_NONE, STEP_LENS, STEP_DEFLECT, STEP_ROTATE, STEP_SHIFT, STEP_BIPRISM = range(6)
+STEP_DRIFT, STEP_DRIFT_PATH = 1, 2
+
+
+class Step(ctypes.Structure):
+    _fields_ = [("kind", ctypes.c_int32), ("flags", ctypes.c_int32), ("d", ctypes.c_double),
+                ("p", ctypes.c_double * 4)]
+
+
+class Column(ctypes.Structure):
+    _fields_ = [
+        ("dtype", ctypes.c_int32), ("n_step", ctypes.c_int32), ("n", ctypes.c_int64),
+        ("in_", ctypes.c_void_p * 5), ("out", ctypes.c_void_p * 5), ("pathlength", ctypes.c_double),
+        ("step", Step * TG_MAX_STEP),
+    ]
+
+
 class BinSpec(ctypes.Structure):
     _fields_ = [
         ("enabled", ctypes.c_int32), ("acc_dtype", ctypes.c_int32),
@@ -87,6 +106,9 @@ _SIGNATURES: dict[str, tuple] = {
     "tg_tune_get": (ctypes.c_int, [ctypes.c_int32, ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int32)]),
     "tg_tune_clear": (ctypes.c_int, []),
     "tg_ray_program_run": (ctypes.c_int, [ctypes.POINTER(Program), ctypes.POINTER(BinSpec), ctypes.c_void_p]),
+    "tg_ray_column_workspace": (ctypes.c_int64, [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64, ctypes.c_int32]),
+    "tg_ray_column_run": (ctypes.c_int, [ctypes.POINTER(Column), ctypes.POINTER(BinSpec), ctypes.c_void_p,
+                                         ctypes.c_int64, ctypes.c_void_p]),
     "tg_hbm_read_probe": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int32,
                                          ctypes.c_void_p]),
 }

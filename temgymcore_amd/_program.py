@@ -522,7 +522,7 @@ def _live_instrs(trace: Trace, live_out: set):
     return kept, needed
 
 
-def _compile_segments(trace: Trace, out_vids: list, keep_vids: list, shape: tuple):
+def _compile_segments(trace: Trace, out_vids: list, keep_vids: list, shape: tuple, given: dict | None = None):
     """Compile one shape group, splitting it into several programs when it
     exceeds one program's instruction, register, slot or output limits.
 
@@ -541,8 +541,8 @@ def _compile_segments(trace: Trace, out_vids: list, keep_vids: list, shape: tupl
         # more outputs than one program stores: the first ones get programs
         # of their own, whose results later programs read instead of recomputing
         head, out_vids = out_vids[:_lib.TG_MAX_SLOT], out_vids[_lib.TG_MAX_SLOT:]
-        p, comp, pc = _compile_segments(trace, head, [], shape)
-        prog, outs, keepalive = prepare(trace, comp, None)
+        p, comp, pc = _compile_segments(trace, head, [], shape, given)
+        prog, outs, keepalive = prepare(trace, comp, None, given)
         prefixes += p + [(prog, None, keepalive + list(outs.values()))]
         prefix_comps += pc + [(comp, outs)]
         _bind_slots(trace, outs)
@@ -573,7 +573,7 @@ def _compile_segments(trace: Trace, out_vids: list, keep_vids: list, shape: tupl
         if chosen is None:
             raise NotImplementedError("ray program cannot be split into programs that fit the kernel's limits")
         stores, comp = chosen
-        prog, outs, keepalive = prepare(trace, comp, None)
+        prog, outs, keepalive = prepare(trace, comp, None, given)
         prefixes.append((prog, None, keepalive + list(outs.values())))
         prefix_comps.append((comp, outs))
         _bind_slots(trace, outs)
@@ -613,8 +613,9 @@ def _slot_strides(t: torch.Tensor, shape: tuple) -> tuple[list, bool]:
     return st, contig
 
 
-def prepare(trace: Trace, comp: Compiled, bin_spec: _lib.BinSpec | None = None):
-    """Allocate outputs and fill the C program struct for one compiled group.
+def prepare(trace: Trace, comp: Compiled, bin_spec: _lib.BinSpec | None = None, given: dict | None = None):
+    """Allocate outputs (those not in `given`: value id -> tensor) and fill the
+    C program struct for one compiled group.
 
     Returns (Program, outputs: value id -> tensor, keep-alive tensors)."""
     shape = tuple(comp.shape)
@@ -647,7 +648,9 @@ def prepare(trace: Trace, comp: Compiled, bin_spec: _lib.BinSpec | None = None):
     prog.n_out = len(comp.outputs)
     for k, (v, r) in enumerate(comp.outputs):
         odt = trace.vdtype[v]
-        o = torch.empty(shape, dtype=odt, device=trace.device)
+        o = given.get(v) if given else None
+        if o is None:
+            o = torch.empty(shape, dtype=odt, device=trace.device)
         outs[v] = o
         prog.out[k] = o.data_ptr()
         prog.out_reg[k] = r
@@ -656,6 +659,7 @@ def prepare(trace: Trace, comp: Compiled, bin_spec: _lib.BinSpec | None = None):
         bin_spec.x_reg, bin_spec.y_reg = comp.bin_regs
     # what the struct's pointers were bound to (for PlanCache templates)
     prog.bound_slots = [s for s, _ in comp.slots]
+    prog.slot_values = trace.slot_value
     prog.bound_outputs = [(v, shape, trace.vdtype[v]) for v, _ in comp.outputs]
     return prog, outs, keep
 
@@ -666,18 +670,34 @@ class Plan:
     Launching re-runs the same kernels on the same input and output buffers
     (inputs may be refilled in place between launches).  ``launch()`` costs one
     C call per program, so a plan is also what a HIP graph capture records.
+
+    A model that is a column of standard elements launches its ``column``
+    (tg_ray_column_run); ``programs``, the register programs of the same model,
+    are then compiled when first asked for.
     """
 
-    def __init__(self, trace: Trace, programs: list, out_ray, acc=None):
+    def __init__(self, trace: Trace, programs, out_ray, acc=None):
         self.trace = trace
-        self.programs = programs  # list of (Program, BinSpec | None, keepalive)
+        self._programs = programs  # list of (Program, BinSpec | None, keepalive), or the function that compiles them
         self.out_ray = out_ray
         self.acc = acc
         self.extra_out: list = []
+        self.column = None  # (Column, BinSpec | None, ColumnMatch)
+
+    @property
+    def programs(self) -> list:
+        if callable(self._programs):
+            self._programs = self._programs()
+        return self._programs
 
     def launch(self, stream: int | None = None):
         lib = _lib.load()
         st = _lib.stream_ptr(self.trace.device) if stream is None else stream
+        if self.column is not None:
+            col, spec, _ = self.column
+            _lib.check(_run_column(lib, col, spec, _column_workspace(lib, col, spec), self.trace.device, st),
+                       "tg_ray_column_run")
+            return self.out_ray
         for prog, spec, _ in self.programs:
             status = lib.tg_ray_program_run(ctypes.byref(prog), ctypes.byref(spec) if spec is not None else None, st)
             _lib.check(status, "tg_ray_program_run")
@@ -688,41 +708,15 @@ class Plan:
 # user-facing drivers
 # --------------------------------------------------------------------------
 
-def build_plan(trace: Trace, sym_ray, bin_request=None, extra_rays=()) -> Plan:
-    """Compile the trace into launchable programs and the output ray.
-
-    bin_request: (BinSpec, x, y) with x, y the symbolic final positions, or None.
-    extra_rays: more symbolic rays of the same trace computed by the same
-    launches (e.g. derivative rays); rebuilt into ``plan.extra_out``.
-    """
-    rays = [sym_ray] + list(extra_rays)
-    fields = {(i, f.name): getattr(r, f.name) for i, r in enumerate(rays) for f in dataclasses.fields(r)}
-    stored: dict = {}
-    for name, v in fields.items():
-        if isinstance(v, Sym):
-            if v.tr is not trace:
-                raise ValueError("output holds a per-ray value of a different trace")
-            stored[name] = v.vid
-    # values that are unchanged inputs are returned as the input arrays
-    direct = {name: vid for name, vid in stored.items() if vid in trace.value_slot}
-    computed = {name: vid for name, vid in stored.items() if name not in direct}
-    groups: dict[tuple, list] = {}
-    for name, vid in computed.items():
-        groups.setdefault(_shape_of(trace, vid), []).append(vid)
-    bin_shape = None
-    keep: list[int] = []
-    if bin_request is not None:
-        _, bx, by = bin_request
-        kv = [v.vid for v in (bx, by) if isinstance(v, Sym)]
-        bin_shape = tuple(torch.broadcast_shapes(*[_shape_of(trace, v) for v in kv])) if kv else (1,)
-        groups.setdefault(bin_shape, [])
-        keep = kv
+def _compile_programs(trace: Trace, groups: dict, bin_request, bin_shape, keep: list, given: dict | None = None):
+    """The launchable programs of the shape groups (shape -> value ids to
+    store): ([(Program, BinSpec | None, keepalive)], value id -> tensor)."""
     results: dict[int, torch.Tensor] = {}
     programs = []
     for shape, vids in groups.items():
         uniq = list(dict.fromkeys(vids))
         is_bin = bin_request is not None and shape == bin_shape
-        prefixes, comp, prefix_comps = _compile_segments(trace, uniq, keep if is_bin else [], shape)
+        prefixes, comp, prefix_comps = _compile_segments(trace, uniq, keep if is_bin else [], shape, given)
         programs.extend(prefixes)
         for _, outs in prefix_comps:  # outputs stored by a prefix program
             results.update(outs)
@@ -737,9 +731,53 @@ def build_plan(trace: Trace, sym_ray, bin_request=None, extra_rays=()) -> Plan:
             if not isinstance(by, Sym):
                 spec.y_uniform = _uniform_as(by, comp.dtype)
             comp.bin_regs = (xr, yr)
-        prog, outs, keepalive = prepare(trace, comp, spec)
+        prog, outs, keepalive = prepare(trace, comp, spec, given)
         results.update(outs)
         programs.append((prog, spec, keepalive))
+    return programs, results
+
+
+def build_plan(trace: Trace, sym_ray, bin_request=None, extra_rays=(), sym_in=None) -> Plan:
+    """Compile the trace into launchable programs and the output ray.
+
+    bin_request: (BinSpec, x, y) with x, y the symbolic final positions, or None.
+    extra_rays: more symbolic rays of the same trace computed by the same
+    launches (e.g. derivative rays); rebuilt into ``plan.extra_out``.
+    sym_in: the symbolic ray the trace started from, where the whole trace maps
+    it to sym_ray (a column of standard elements is recognised from it).
+    """
+    rays = [sym_ray] + list(extra_rays)
+    fields = {(i, f.name): getattr(r, f.name) for i, r in enumerate(rays) for f in dataclasses.fields(r)}
+    stored: dict = {}
+    for name, v in fields.items():
+        if isinstance(v, Sym):
+            if v.tr is not trace:
+                raise ValueError("output holds a per-ray value of a different trace")
+            stored[name] = v.vid
+    # values that are unchanged inputs are returned as the input arrays
+    direct = {name: vid for name, vid in stored.items() if vid in trace.value_slot}
+    computed = {name: vid for name, vid in stored.items() if name not in direct}
+    column = None
+    if sym_in is not None and not extra_rays:
+        from ._column import match
+
+        column = match(trace, sym_in, sym_ray, bin_request)
+    groups: dict[tuple, list] = {}
+    for name, vid in computed.items():
+        groups.setdefault(column.shape if column else _shape_of(trace, vid), []).append(vid)
+    bin_shape = None
+    keep: list[int] = []
+    if bin_request is not None:
+        _, bx, by = bin_request
+        kv = [v.vid for v in (bx, by) if isinstance(v, Sym)]
+        bin_shape = tuple(torch.broadcast_shapes(*[_shape_of(trace, v) for v in kv])) if kv else (1,)
+        groups.setdefault(bin_shape, [])
+        keep = kv
+    if column is not None:
+        buf, results = _column_outputs(column, trace.device)
+        programs = lambda: _compile_programs(trace, groups, bin_request, bin_shape, keep, results)[0]  # noqa: E731
+    else:
+        programs, results = _compile_programs(trace, groups, bin_request, bin_shape, keep)
     out_vals: list[dict] = [{} for _ in rays]
     field_src = []  # the primary ray's fields: ("slot", s) | ("vid", v) | ("value", v)
     for (i, name), v in fields.items():
@@ -758,7 +796,47 @@ def build_plan(trace: Trace, sym_ray, bin_request=None, extra_rays=()) -> Plan:
     plan = Plan(trace, programs, _rebuild(sym_ray, out_vals[0]))
     plan.extra_out = [_rebuild(r, vals) for r, vals in zip(rays[1:], out_vals[1:])]
     plan.field_src = field_src
+    if column is not None:
+        col = _lib.Column.from_buffer_copy(column.struct)
+        for k, s in enumerate(column.slots):
+            if s is not None:
+                col.in_[k] = trace.slot_tensors[s].data_ptr()
+            if column.out_vids[k] is not None:
+                col.out[k] = results[column.out_vids[k]].data_ptr()
+        plan.column = (col, None if bin_request is None else bin_request[0], column)
+        plan.recipe = (groups, bin_request, bin_shape, keep)
     return plan
+
+
+def _column_workspace(lib, col, spec) -> int:
+    """Bytes of scratch memory a column's binning takes (0: none)."""
+    return 0 if spec is None else lib.tg_ray_column_workspace(col.n, spec.height, spec.width, spec.acc_dtype)
+
+
+def _run_column(lib, col, spec, ws_bytes: int, device, stream) -> int:
+    """Launch a column; its scratch memory comes from torch's stream-ordered
+    allocator (on the launch's stream) and is given back once the launch is
+    enqueued."""
+    if not ws_bytes:
+        return lib.tg_ray_column_run(ctypes.byref(col), None if spec is None else ctypes.byref(spec), None, 0, stream)
+    if stream == _lib.stream_ptr(device):
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
+    else:
+        with torch.cuda.stream(torch.cuda.ExternalStream(stream, device=device)):
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
+    return lib.tg_ray_column_run(ctypes.byref(col), ctypes.byref(spec), ws.data_ptr(), ws_bytes, stream)
+
+
+def _column_outputs(column, device):
+    """One allocation for a column's outputs, every row on a 16-byte boundary
+    (the kernel's wide stores): (buffer [rows, row], value id -> tensor)."""
+    vids = [v for v in column.out_vids if v is not None]
+    n = column.struct.n
+    buf = torch.empty((len(vids), column.row), dtype=column.dtype, device=device)
+    rows = (buf if column.row == n else buf.narrow(1, 0, n)).unbind(0)
+    if len(column.shape) != 1:
+        rows = [r.view(column.shape) for r in rows]
+    return buf, dict(zip(vids, rows))
 
 
 def _materialize(trace: Trace, sym_ray, bin_request=None):
@@ -779,7 +857,7 @@ def plan_fn(fn: Callable, ray, bin_request_fn: Callable | None = None) -> Plan:
     sym_in = trace.symbolize(ray)
     sym_out = fn(sym_in)
     req = bin_request_fn(sym_out) if bin_request_fn is not None else None
-    return build_plan(trace, sym_out, req)
+    return build_plan(trace, sym_out, req, sym_in=sym_in)
 
 
 def apply_fn(fn: Callable, ray, bin_request_fn: Callable | None = None):
@@ -900,10 +978,25 @@ def _structure_key(obj, leaves: list, seen: dict):
     raise Uncacheable(t.__name__)
 
 
+def _without_arrays(trace: Trace) -> Trace:
+    """A copy of a trace that compiles to the same programs and holds none of
+    its arrays (shapes, strides and dtypes only)."""
+    bare = Trace(torch.device("meta"))
+    bare.instrs, bare.n_values = trace.instrs, trace.n_values
+    bare.deps, bare.vdtype = trace.deps, trace.vdtype
+    for t, src, v in zip(trace.slot_tensors, trace.slot_source, trace.slot_value):
+        if src is not None:  # an input, not a buffer between programs
+            bare.value_slot[v] = len(bare.slot_tensors)
+            bare.slot_tensors.append(torch.empty_strided(t.shape, t.stride(), dtype=t.dtype, device="meta"))
+            bare.slot_source.append(None)
+            bare.slot_value.append(v)
+    return bare
+
+
 class _PlanTemplate:
     """The compiled programs of one cache key with their pointers unbound."""
 
-    __slots__ = ("device", "programs", "fields", "ray_type", "convert")
+    __slots__ = ("device", "_programs", "fields", "ray_type", "convert", "column")
 
     def __init__(self, plan: Plan, leaves: list):
         trace = plan.trace
@@ -924,14 +1017,21 @@ class _PlanTemplate:
             else:
                 raise Uncacheable("an input array is not reachable from the call's arguments")
         self.device = trace.device
-        self.programs = []
-        for prog, spec, _ in plan.programs:
-            groups: dict = {}
-            for k, (vid, shape, dt) in enumerate(prog.bound_outputs):
-                groups.setdefault((tuple(shape), dt), []).append((k, vid))
-            self.programs.append((_lib.Program.from_buffer_copy(prog),
-                                  None if spec is None else _lib.BinSpec.from_buffer_copy(spec),
-                                  [slot_src[s] for s in prog.bound_slots], list(groups.items())))
+        self.column = None
+        if plan.column is not None:
+            # (the register programs are compiled when asked for, from a copy of
+            # the trace that holds no arrays)
+            _, spec, match = plan.column
+            self.column = [match, None if spec is None else _lib.BinSpec.from_buffer_copy(spec),
+                           [None if s is None else slot_src[s][1] for s in match.slots], None]
+            bare = _without_arrays(trace)
+            groups, request, bin_shape, keep = plan.recipe
+            if request is not None:
+                request = (_lib.BinSpec.from_buffer_copy(request[0]), *(Sym(bare, v.vid) for v in request[1:]))
+            self._programs = lambda: self._unbound(_compile_programs(bare, groups, request, bin_shape, keep)[0],
+                                                   slot_src)
+        else:
+            self._programs = self._unbound(plan.programs, slot_src)
         self.fields = []
         for name, (kind, x) in plan.field_src:
             if kind == "slot":
@@ -950,6 +1050,25 @@ class _PlanTemplate:
             else:
                 raise Uncacheable(type(x).__name__)
         self.ray_type = type(plan.out_ray)
+
+    @staticmethod
+    def _unbound(programs, slot_src):
+        out = []
+        for prog, spec, _ in programs:
+            groups: dict = {}
+            for k, (vid, shape, dt) in enumerate(prog.bound_outputs):
+                groups.setdefault((tuple(shape), dt), []).append((k, vid))
+            # slots past the inputs are buffers of earlier programs
+            binds = [slot_src[s] if s < len(slot_src) else ("vid", prog.slot_values[s]) for s in prog.bound_slots]
+            out.append((_lib.Program.from_buffer_copy(prog),
+                        None if spec is None else _lib.BinSpec.from_buffer_copy(spec), binds, list(groups.items())))
+        return out
+
+    @property
+    def programs(self) -> list:
+        if callable(self._programs):
+            self._programs = self._programs()
+        return self._programs
 
     def bind(self, leaves: list, acc: torch.Tensor | None):
         """Copies of the programs with this call's arrays and fresh outputs
@@ -998,8 +1117,52 @@ class _PlanTemplate:
                 vals[name] = x
         return bound, _rebuild_type(self.ray_type, vals), (inputs, outs)
 
+    def _launch_column(self, leaves: list, acc: torch.Tensor | None, stream: int):
+        match, spec_t, in_leaves, ws_bytes = self.column
+        dev = self.device
+        inputs = {i: to_device_tensor(leaves[i], dev) if i in self.convert else leaves[i]
+                  for i in in_leaves if i is not None}
+        col = _lib.Column.from_buffer_copy(match.struct)
+        ptrs = col.in_
+        for k, i in enumerate(in_leaves):
+            if i is not None:
+                ptrs[k] = inputs[i].data_ptr()
+        outs = {}
+        if match.n_out:
+            buf, outs = _column_outputs(match, dev)
+            at, ptrs = buf.data_ptr(), col.out
+            for k, v in enumerate(match.out_vids):
+                if v is not None:
+                    ptrs[k] = at
+                    at += match.row_bytes
+        spec = None
+        if spec_t is not None:
+            spec = _lib.BinSpec.from_buffer_copy(spec_t)
+            spec.acc = acc.data_ptr()
+        lib = _lib.load()
+        if ws_bytes is None:
+            ws_bytes = self.column[3] = _column_workspace(lib, col, spec)
+        st = _run_column(lib, col, spec, ws_bytes, dev, stream)
+        if st != 0:
+            _lib.check(st, "tg_ray_column_run")
+        vals = {}
+        for name, kind, x in self.fields:
+            if kind == "vid":
+                vals[name] = outs[x]
+            elif kind == "input":
+                t = inputs.get(x)
+                vals[name] = t if t is not None else (
+                    to_device_tensor(leaves[x], dev) if x in self.convert else leaves[x])
+            elif kind == "leaf":
+                vals[name] = leaves[x]
+            else:
+                vals[name] = x
+        return _rebuild_type(self.ray_type, vals)
+
     def launch(self, leaves: list, acc: torch.Tensor | None, stream: int):
         """Bind this call's arrays and fresh outputs, launch, return the output ray."""
+        if self.column is not None:
+            return self._launch_column(leaves, acc, stream)
         run = _lib.load().tg_ray_program_run
         bound, out_ray, _ = self.bind(leaves, acc)
         for prog, spec in bound:

@@ -13,8 +13,8 @@
 //   * the program is a kernel argument (kernarg segment -> scalar loads), so
 //     opcode dispatch is a uniform scalar branch and never diverges;
 //   * registers are named VGPRs selected through uniform switches (no scratch);
-//   * binning of small detectors (<= 32768 bins of int counts) goes through
-//     an LDS-privatised histogram of packed 16-bit counters (two bins per
+//   * binning of detectors up to kLdsBins (int counts) goes through an
+//     LDS-privatised histogram of packed 16-bit counters (two bins per
 //     32-bit word; a workgroup bins at most 65535 rays, so a counter never
 //     carries into its neighbour), flushed once per workgroup with
 //     device-scope atomics; larger detectors and float accumulators use
@@ -24,15 +24,15 @@
 // sequence evaluated elementwise on the CPU.
 #include <algorithm>
 
-#include "tg_common.hpp"
+#include "ray_common.hpp"
 
 namespace {
+
+using namespace tgr;
 
 constexpr int kThreads = 256;
 // the program and binning spec travel by value in the kernel-argument segment
 static_assert(sizeof(tg_program) + sizeof(tg_bin_spec) <= 4096, "ray program exceeds the kernel-argument limit");
-constexpr int64_t kLdsBins = 32768;
-constexpr int64_t kMaxRaysPerGroup = 65535;
 // input slots whose loads are issued together (one memory round trip);
 // strided slots carry 64-bit offsets per ray, so they go two at a time
 template <bool CONTIG>
@@ -86,12 +86,6 @@ struct RegFile<T, TG_MAX_REG> {
 };
 static_assert((TG_MAX_REG & (TG_MAX_REG - 1)) == 0, "TG_MAX_REG must be a power of two");
 
-template <typename T>
-__device__ __forceinline__ T sign_of(T a) {
-  if (a != a || a == T(0)) return a;
-  return a > T(0) ? T(1) : T(-1);
-}
-
 __device__ __forceinline__ int64_t slot_offset(int64_t lin, const int64_t (&shape)[TG_MAX_DIM],
                                                const int64_t (&stride)[TG_MAX_DIM]) {
   const int64_t i3 = lin % shape[3];
@@ -103,49 +97,16 @@ __device__ __forceinline__ int64_t slot_offset(int64_t lin, const int64_t (&shap
   return i0 * stride[0] + i1 * stride[1] + i2 * stride[2] + i3 * stride[3];
 }
 
-// Pixel index of one position; -1 when it falls outside the detector.
-__device__ __forceinline__ int64_t bin_index(const tg_bin_spec& B, double y, double x) {
-  // Same operation order as apply_transformation's T @ [y, x, 1]
-  // (reference coordinate_transforms.py:104-140), in f64.
-  const double fy = __dadd_rn(__dadd_rn(__dmul_rn(B.m[0], y), __dmul_rn(B.m[1], x)), B.m[2]);
-  const double fx = __dadd_rn(__dadd_rn(__dmul_rn(B.m[3], y), __dmul_rn(B.m[4], x)), B.m[5]);
-  // jnp.round is round-half-to-even; rint uses the default RNE mode.
-  const int32_t iy = tg::xla_f64_to_i32(rint(fy));
-  const int32_t ix = tg::xla_f64_to_i32(rint(fx));
-  if (iy < 0 || iy >= B.height || ix < 0 || ix >= B.width) return -1;
-  return (int64_t)iy * B.width + ix;
-}
-
-template <typename T>
-__device__ __forceinline__ void global_deposit(const tg_bin_spec& B, int64_t p, T w) {
-  switch (B.acc_dtype) {
-    case 0:
-      atomicAdd((int32_t*)B.acc + p, 1);
-      break;
-    case 1:
-      atomicAdd((unsigned long long*)B.acc + p, 1ull);
-      break;
-    case 2:
-      unsafeAtomicAdd((float*)B.acc + p, (float)w);
-      break;
-    default:
-      unsafeAtomicAdd((double*)B.acc + p, (double)w);
-      break;
-  }
-}
-
 // BIN: 0 = no binning, 1 = LDS-privatised integer histogram, 2 = global atomics.
 // NT: workgroup size (LDS-histogram launches use 1024 so that 16 wavefronts
 // share one private histogram and fewer flushes hit the same global bins).
 template <typename T, int R, bool CONTIG, int BIN, int NT, int NREG, bool MIXED>
 __global__ __launch_bounds__(NT) void ray_program_kernel(const tg_program P, const tg_bin_spec B) {
   constexpr int kThreads = NT;
-  extern __shared__ int32_t lds_hist[];
+  extern __shared__ __align__(16) int32_t lds_hist[];
   const int64_t n = P.n;
-  int64_t hw = 0;
   if constexpr (BIN == 1) {
-    hw = B.height * B.width;
-    for (int64_t i = threadIdx.x; i < (hw + 1) / 2; i += kThreads) lds_hist[i] = 0;
+    lds_clear<kThreads>(lds_hist, (int)(B.height * B.width));
     __syncthreads();
   }
   const int64_t chunk = (int64_t)kThreads * R;
@@ -322,7 +283,7 @@ __global__ __launch_bounds__(NT) void ray_program_kernel(const tg_program P, con
         const int64_t p = bin_index(B, (double)yv[u], (double)xv[u]);
         if (p < 0) continue;
         if constexpr (BIN == 1) {
-          atomicAdd(&lds_hist[p >> 1], 1 << (16 * (int)(p & 1)));
+          lds_deposit(lds_hist, p);
         } else {
           global_deposit<T>(B, p, wv[u]);
         }
@@ -331,20 +292,7 @@ __global__ __launch_bounds__(NT) void ray_program_kernel(const tg_program P, con
   }
   if constexpr (BIN == 1) {
     __syncthreads();
-    for (int64_t i = threadIdx.x; i < (hw + 1) / 2; i += kThreads) {
-      const uint32_t w = (uint32_t)lds_hist[i];
-      if (w == 0) continue;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int32_t c = (int32_t)((w >> (16 * h)) & 0xffffu);
-        const int64_t bin = 2 * i + h;
-        if (c == 0 || bin >= hw) continue;
-        if (B.acc_dtype == 0)
-          atomicAdd((int32_t*)B.acc + bin, c);
-        else
-          atomicAdd((unsigned long long*)B.acc + bin, (unsigned long long)(int64_t)c);
-      }
-    }
+    lds_flush<kThreads>(B, lds_hist, 0, (int)(B.height * B.width));
   }
 }
 
@@ -372,7 +320,9 @@ int launch(const tg_program& P, const tg_bin_spec& B, hipStream_t stream) {
     const int64_t min_grid = tg::cdiv(P.n, (kMaxRaysPerGroup / chunk) * chunk);
     if (grid < min_grid) grid = min_grid;
   }
-  const size_t lds = (BIN == 1) ? (size_t)((B.height * B.width + 1) / 2) * sizeof(int32_t) : 0;
+  const size_t lds = (BIN == 1) ? (size_t)lds_words(B.height * B.width) * sizeof(int32_t) : 0;
+  const int st = allow_lds((const void*)ray_program_kernel<T, R, CONTIG, BIN, kThreads, NREG, MIXED>, lds);
+  if (st != TG_OK) return st;
   hipLaunchKernelGGL((ray_program_kernel<T, R, CONTIG, BIN, kThreads, NREG, MIXED>), dim3((unsigned)grid), dim3(kThreads),
                      lds, stream, P, B);
   TG_LAUNCH_CHECK("ray_program_kernel launch");
