@@ -679,18 +679,20 @@ def bench_beamlet(steps: int, warmup: int):
     evals_per_s = evaluated / (ms_per_step * 1e-3)
     matrix = tuned_path == autotune.BEAMLET_PATH_AUTO and _all_separable(rec_bytes)
     if matrix:
-        # the matrix-core product computes whole 64x64 tiles: 8 flops (one
-        # complex multiply-add) per (beamlet, pixel) of every tile its cutoff box meets
+        # the matrix-core product computes whole 128x128 tiles; a real product
+        # is three f16 ones (high and low halves): 24 flops per complex
+        # multiply-add, for each (beamlet, pixel) of every tile its cutoff
+        # ellipse meets
         tile_pairs = _tile_pair_count(rec_bytes, n, H, W)
-        achieved = 8 * tile_pairs / (sum_ms * 1e-3)
-        roof = {"bound": "mfma", "achieved": achieved / 1e12, "peak": 157.3, "unit": "TFLOP/s",
-                "frac": achieved / 157.3e12, "traffic": None, "flops_per_pair": 8, "tile_pairs": tile_pairs,
+        achieved = 24 * tile_pairs / (sum_ms * 1e-3)
+        roof = {"bound": "mfma", "achieved": achieved / 1e12, "peak": 2516.6, "unit": "TFLOP/s",
+                "frac": achieved / 2516.6e12, "traffic": None, "flops_per_pair": 24, "tile_pairs": tile_pairs,
                 "timed_kernels": "tg_beamlet_sum (path flags + beamlet_sum_sep_kernel + slice sums), HIP events",
-                "peak_note": "MI355X dense FP32 matrix peak (v_mfma_f32_32x32x2f32)",
+                "peak_note": "MI355X dense f16 matrix peak (v_mfma_f32_32x32x16_f16)",
                 "mfma_util_percent": _profiled("beamlet_sum_sep_kernel-beamlet_131072_1024sq.md",
                                                "mfma_util_percent"),
-                "mfma_source": "profiles/beamlet_sum_sep_kernel-beamlet_131072_1024sq.md (MfmaUtil PMC); the "
-                               "factor evaluation's vector instructions do not overlap the f32 MFMAs on gfx950"}
+                "mfma_source": "profiles/beamlet_sum_sep_kernel-beamlet_131072_1024sq.md (MFMA busy cycles); the "
+                               "factor evaluation's vector instructions take the rest of the issue slots"}
     else:
         flops_per_eval = 14  # two complex f32 products (6 each) + complex accumulate (2)
         achieved = flops_per_eval * evaluated / (sum_ms * 1e-3)
@@ -718,7 +720,7 @@ def bench_beamlet(steps: int, warmup: int):
                 "autotune": {"beamlet_path": {1: "auto", 2: "valu"}[tuned_path],
                              "path_candidate_ms": {{1: "auto", 2: "valu"}[k]: v for k, v in path_ms.items()},
                              "beamlet_splits": tuned_splits, "candidate_ms": tune_ms,
-                             "tile_shape": _shape_name(tuned_shape) if tuned_shape else "64x64 (matrix cores)",
+                             "tile_shape": _shape_name(tuned_shape) if tuned_shape else "128x128 (matrix cores)",
                              "tile_shape_ms": {_shape_name(k): v for k, v in shape_ms.items()}}},
         roofline=roof,
         cpu_baseline=cpu,
@@ -739,11 +741,11 @@ def _all_separable(coef_bytes):
                 and np.all(phi[:, 0] < 0) and np.all(phi[:, 4] < 0))
 
 
-def _tile_pair_count(coef_bytes, n, H, W, tile=64):
-    """(beamlet, pixel) pairs of the 64x64 tiles each separable beamlet's
+def _tile_pair_count(coef_bytes, n, H, W, tile=128):
+    """(beamlet, pixel) pairs of the 128x128 tiles each separable beamlet's
     cutoff ellipse meets (the matrix-core tile sum's list test: the tile's
     pixel centre nearest the centre inside u^2 + gamma v^2 <= beta, in f32),
-    4096 per tile."""
+    16384 per tile."""
     import numpy as np
 
     rec = np.frombuffer(coef_bytes, dtype=np.dtype(_COEF_DTYPE))

@@ -32,6 +32,8 @@
 //   dL/dtheta = Re[amp sum_k G_k dc_k/dtheta]
 // with dc_k/dtheta from forward-mode dual numbers through the same
 // coefficient algebra (one pass per parameter and ray-transfer entry).
+#include <utility>
+
 #include "beamlet_common.hpp"
 
 namespace {
@@ -75,32 +77,72 @@ __device__ __forceinline__ bool separable(const tg_beamlet_coef& c) {
 // |Ey| <= the peak.  One axis is
 //   exp(q2 (p - cen)^2 + g + i (q1 p^2 + l1 p + c0)).
 struct SepAxis {
-  double q2, q1, l1, c0, cen, g;
+  float q2l, gl;  // q2 and g times log2(e)
+  double q1, l1, c0, cen;
 };
-struct SepParams {
-  SepAxis x, y;
-};
-static_assert(sizeof(SepParams) == 96, "SepParams layout");
 
-__device__ __forceinline__ SepParams sep_params(const tg_beamlet_coef& c) {
-  SepParams q;
+// The factors of n beamlets, 96 bytes each: what every tile reads (the cutoff
+// ellipse cx, cy, gamma, beta, then gl and the x factor's q2l), the x
+// factors (gl = c0 = 0 left out), the y factors.
+struct SepTables {
+  float4* cull;
+  float2* peak;   // gl, q2l of x
+  double* x;      // 4 a beamlet: (q2l, -), q1, l1, cen
+  double* y;      // 5 a beamlet: (q2l, gl), q1, l1, c0, cen
+};
+constexpr int64_t kSepBytes = 96;
+constexpr double kLog2e = 1.4426950408889634;
+
+__host__ __device__ inline SepTables sep_tables(void* p, int64_t n) {
+  SepTables t;
+  t.cull = (float4*)p;
+  t.peak = (float2*)(t.cull + n);
+  t.x = (double*)(t.peak + n);
+  t.y = t.x + 4 * n;
+  return t;
+}
+
+__device__ __forceinline__ double two_floats(float lo, float hi) {
+  return __hiloint2double(__float_as_int(hi), __float_as_int(lo));
+}
+
+__device__ __forceinline__ void store_sep(const SepTables& t, int64_t i, const tg_beamlet_coef& c) {
   const double ar = c.phi[0], cr = c.phi[4];
   const double cx = -c.phi[6] / (2.0 * ar), cy = -c.phi[8] / (2.0 * cr);
-  q.x = {ar, c.phi[1], c.phi[7], 0.0, cx, 0.0};
-  q.y = {cr, c.phi[5], c.phi[9], c.phi[11], cy, c.phi[10] - ar * cx * cx - cr * cy * cy};
-  return q;
+  const float qx = (float)(ar * kLog2e), qy = (float)(cr * kLog2e);
+  const float gl = (float)((c.phi[10] - ar * cx * cx - cr * cy * cy) * kLog2e);
+  t.cull[i] = make_float4(c.cx, c.cy, c.gamma, c.beta);
+  t.peak[i] = make_float2(gl, qx);
+  double* x = t.x + 4 * i;
+  x[0] = two_floats(qx, 0.0f);
+  x[1] = c.phi[1];
+  x[2] = c.phi[7];
+  x[3] = cx;
+  double* y = t.y + 5 * i;
+  y[0] = two_floats(qy, gl);
+  y[1] = c.phi[5];
+  y[2] = c.phi[9];
+  y[3] = c.phi[11];
+  y[4] = cy;
+}
+
+__device__ __forceinline__ SepAxis load_sep(const SepTables& t, int64_t i, bool y_axis) {
+  const double* p = y_axis ? t.y + 5 * i : t.x + 4 * i;
+  const double q = p[0];
+  return {__int_as_float(__double2loint(q)), __int_as_float(__double2hiint(q)), p[1], p[2],
+          y_axis ? p[3] : 0.0, p[y_axis ? 4 : 3]};
 }
 
 // flags[blockIdx.x]: some beamlet of this workgroup's share is not separable
-// (or force_valu); par[i]: the factors of beamlet i when it is separable.
+// (or force_valu); tab[i]: the factors of beamlet i when it is separable.
 __global__ __launch_bounds__(256) void sep_flag_kernel(const tg_beamlet_coef* __restrict__ coef, int64_t n,
                                                        int32_t force_valu, int32_t* __restrict__ flags,
-                                                       SepParams* __restrict__ par) {
+                                                       SepTables tab) {
   int bad = force_valu;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n && !force_valu; i += (int64_t)gridDim.x * 256) {
     const tg_beamlet_coef& c = coef[i];
     if (separable(c))
-      par[i] = sep_params(c);
+      store_sep(tab, i, c);
     else
       bad = 1;
   }
@@ -131,46 +173,99 @@ __global__ __launch_bounds__(kThreads) void beamlet_sum_kernel(const tg_beamlet_
 // ---------------------------------------------------------------------------
 // Separable beamlets on the matrix cores.  A tile is the complex matrix
 // product  T[m][n] = sum_k Ey_k(ty0 + m) Ex_k(tx0 + n)  over the beamlets whose
-// cutoff box meets it: three real f32 MFMA products per k (sep_mfma).
-// Wave w owns the 32x32 block at rows 32 (w / 2), columns
-// 32 (w % 2) of the 64x64 tile.  The factors of kSepK beamlets at a time are
-// staged in LDS, double-buffered: a wave evaluates chunk c + 1 into one
-// buffer while issuing chunk c's products from the other, one barrier per
-// chunk.  (On gfx950 the vector instructions and the f32 MFMAs of a SIMD do
-// not execute concurrently -- measured: their times add, also across waves
-// -- so the evaluation's instruction count is what it costs.)  Each thread
-// evaluates one 16-pixel segment of one factor directly, without branches:
-//   exp2(q2' (p - cen)^2 + g') (cos, sin)(2 pi theta(p)),
+// cutoff ellipse meets it, K = beamlets.
+//
+// Precision.  A factor value is held as two f16, x = h + l (l the rounding of
+// h, itself rounded: 22 bits, no less than the 16 phasor steps behind a value
+// carry), and a real product is ah bh + ah bl + al bh in f32 accumulators (what
+// is left out is below 2^-22 |a b|).  f16 has few exponents, so the factors are
+// scaled: each x factor by the power of two that takes its largest value in
+// the tile to [2^14, 2^15), and the y factor, amplitude included, by the rest,
+// so that no term exceeds 2^28 times 2^exp_now, the largest term met so far in
+// the tile.  A list block with larger terms rescales the sums first (an exact
+// power of two).  Parts of a factor below 2^-39 of its largest value in the
+// tile are lost, far below the f32 rounding of that value.  Against complex128,
+// norm of the error over norm of the field, 131,072 beamlets on 1024^2: 3.9e-6
+// (f32 products: 4.2e-6; both are the phasor recurrence's error).
+//
+// Rate.  12 v_mfma_f32_32x32x16_f16 take 16 beamlets of a 32x32 block, 25
+// cycles a beamlet, where f32 products (three v_mfma_f32_32x32x2_f32 a pair)
+// take 96.  And vector instructions run beside f16 MFMAs, which they do not
+// beside f32 ones (register-only chains, two wavefronts a SIMD: 8 FMAs beside
+// each MFMA cost 33 -> 44 cycles in f16, 67 -> 103 in f32).  (Three bf16 parts,
+// six products, 24 bits: 3.75 ms where f16 takes 2.45.)
+//
+// A workgroup owns a 128x128 tile, a wave 2x2 of its 32x32 blocks: evaluating
+// a factor costs about as much as its products, and a wider tile uses a value
+// more often.  131,072 beamlets on 1024^2: 2.45 ms, 64x64 tiles (one block a
+// wave) 3.06 ms; 20,000 on 512^2: 398 and 496 us; on images of one tile the two
+// differ by less than the launch's host work, so there is one tile shape.
+// 16 beamlets a chunk go through two LDS buffers, one barrier a chunk: beside
+// its products of chunk c every lane evaluates one 16-pixel segment of one
+// factor of chunk c + 1, a pixel between every three products (at raised
+// priority: a wave between its loads would otherwise hold up the matrix cores'
+// next instruction; 2.57 -> 2.45 ms), with chunk c + 2's parameters in flight.
+// A lane's beamlet is k = lane & 15; lanes k and k + 1 exchange a component
+// (DPP) so that the even lane packs both real parts and the odd one both
+// imaginary parts: the operand layout wants consecutive beamlets side by side.
+// A pixel's 16 beamlets take 32 bytes, with 64 more after every 16 pixels and
+// 32 between the arrays: stores of a wavefront meet 64 banks, operand reads
+// (16 bytes a lane) are contiguous.
+//
+// A segment's value is  exp2(q2' (p - cen)^2 + g') (cos, sin)(2 pi theta(p)),
 //   theta(p0 + j) = theta0 + j A + j^2 B   (revolutions),
 // theta0 being the segment start's phase reduced in double-double.  theta0,
 // A and B are reduced modulo one revolution as 32-bit fixed-point fractions
 // (exact whatever the size of the linear and quadratic phase terms; an f32
 // sum theta0 + jA + j^2 B lost 1e-5 revolutions on strongly curved
 // input-plane beamlets), and seed a unit-phasor recurrence (two transcendental
-// pairs per segment instead of a sine and cosine per value).  Parameters are
-// loaded one chunk ahead of their use.
+// pairs per segment instead of a sine and cosine per value).
+//
+// 131,072 beamlets, 1024^2, 4 sigma, the whole sum: 4.64 ms with f32 products,
+// now 2.4 ms (tile sum 2.25, slices 0.105).  Bound: vector issue (63% of the
+// cycles, 520 instructions a chunk) and the matrix cores (46%) together, at
+// the 1.9 GHz that this mix runs at.
 // ---------------------------------------------------------------------------
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
 
-constexpr int kSepK = 32;          // beamlets per LDS chunk (the product's K)
-constexpr int kSepSeg = 16;        // pixels per generated segment
-constexpr int kSepRow = kTileW + 1;  // LDS row pitch (float2): a bank offset per beamlet row
-constexpr int kSepBlock = 2048;    // beamlets per list build
-constexpr double kLog2e = 1.4426950408889634;
-static_assert(kTileW == 64 && kTileH == 64 && kThreads == 256 && kThreads >= kFlagBlocks &&
-                  kSepK * 2 * (kTileW / kSepSeg) == kThreads && kSepSeg == kSepK / 2 &&
-                  kSepBlock % kThreads == 0,
-              "the matrix-core tile sum assumes 64x64 tiles, four waves, one segment per thread and one "
-              "segment value per k pair");
+constexpr int kMxK = 16;           // beamlets per MFMA
+constexpr int kMxSeg = 16;         // pixels per evaluated segment
+constexpr int kMxBlock = 1024;     // beamlets per list build
+constexpr int kMxScale = 14;       // factors are held times 2^14 and at most 2^15: their low halves stay normal
 
-// The axis record (q2, q1), (l1, c0), (cen, g) of beamlet i.
-__device__ __forceinline__ void load_axis(const SepParams* __restrict__ par, int64_t i, int axis, double2& v0,
-                                          double2& v1, double2& v2) {
-  const double2* src = reinterpret_cast<const double2*>(par + i) + 3 * axis;
-  v0 = src[0];
-  v1 = src[1];
-  v2 = src[2];
+// A TW x TH tile, KC beamlets a chunk, BM x BN 32x32 blocks a wave: LDS layout
+// and workgroup.
+template <int TW_, int TH_, int KC_, int BM_, int BN_>
+struct MxTile {
+  static constexpr int TW = TW_, TH = TH_, KC = KC_, BM = BM_, BN = BN_;
+  static constexpr int kPix = TW + TH;  // x pixels, then y pixels
+  static constexpr int kWaves = TW * TH / (1024 * BM * BN), kThreads = 64 * kWaves;
+  // dwords (two beamlets each) of one component of one split part, and of the
+  // four of them for one MFMA's beamlets
+  static constexpr int kPart = kPix * (kMxK / 2) + kPix / 16 * 16 + 8;
+  static constexpr int kStep = 4 * kPart;
+  static constexpr int kBuffer = KC / kMxK * kStep;
+  static_assert(TW % (32 * BN) == 0 && TH % (32 * BM) == 0 && TW % 64 == 0 && kPart % 64 == 8 && kStep % 64 == 32,
+                "whole blocks; stores of a wavefront on 64 banks");
+  static_assert(KC * kPix / kMxSeg == kThreads, "one segment a lane");
+};
+
+using SepTile = MxTile<128, 128, 16, 2, 2>;
+
+constexpr int kNoExp = -(1 << 24);  // no beamlet met yet
+
+__device__ __forceinline__ int wave_max_i32(int v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
+  return v;
 }
+
+// dword offset of a pixel's row within a part
+constexpr int kBlockRow = 32 * (kMxK / 2) + 32;  // 32 pixels further
+__device__ __forceinline__ int mx_row(int pix) { return pix * (kMxK / 2) + (pix >> 4) * 16; }
 
 // Evaluation state of one 16-pixel segment starting at pixel p0: the
 // log2-scaled envelope, evaluated directly, and the unit phasor
@@ -185,9 +280,12 @@ struct SegGen {
   float t0, q2l, gl;
 };
 
-// r (revolutions, |r| < 2^52) modulo one, in 2^-32 units
+// r (revolutions, |r| < 2^52) modulo one, in 2^-32 units, rounded to nearest:
+// the low word of the fraction times 2^32 plus 1.5 2^52 (a conversion to a
+// 64-bit integer takes about ten instructions)
 __device__ __forceinline__ uint32_t fixed_revolutions(double r) {
-  return (uint32_t)(int64_t)rint((r - rint(r)) * 4294967296.0);
+  const double f = fma(r - rint(r), 4294967296.0, 6755399441055744.0);
+  return (uint32_t)__double2loint(f);
 }
 
 // exp(2 pi i u 2^-32)
@@ -196,21 +294,25 @@ __device__ __forceinline__ float2 phasor(uint32_t u) {
   return make_float2(__builtin_amdgcn_cosf(t), __builtin_amdgcn_sinf(t));
 }
 
-__device__ __forceinline__ SegGen seg_setup(double2 v0, double2 v1, double2 v2, double p0, bool valid) {
-  const double q2 = v0.x, q1 = v0.y, l1 = v1.x, c0 = v1.y, cen = v2.x, g = v2.y;
+// exponent: added to the envelope's log2.  swap: the values come out as (im,
+// re): z with its parts exchanged, stepped by the conjugate ratios.
+__device__ __forceinline__ SegGen seg_setup(const SepAxis& v, double p0, float exponent, bool valid, bool swap) {
   // theta(p0 + j) = theta0 + j A + j^2 B  (revolutions)
-  const double x = fma(fma(q1, p0, l1), p0, c0);
+  const double x = fma(fma(v.q1, p0, v.l1), p0, v.c0);
   const double hi = x * kInv2PiHi;
   const double theta0 = (hi - rint(hi)) + fma(x, kInv2PiLo, fma(x, kInv2PiHi, -hi));
-  const uint32_t a = fixed_revolutions(fma(2.0 * q1, p0, l1) * kInv2PiHi);
-  const uint32_t b = fixed_revolutions(q1 * kInv2PiHi);
+  const uint32_t a = fixed_revolutions(fma(2.0 * v.q1, p0, v.l1) * kInv2PiHi);
+  const uint32_t b = fixed_revolutions(v.q1 * kInv2PiHi);
   SegGen s;
-  s.z = phasor(fixed_revolutions(theta0));
-  s.r = phasor(a + b);  // theta(1) - theta(0) = A + B
-  s.k = phasor(2u * b);  // second difference 2 B
-  s.t0 = (float)(p0 - cen);
-  s.q2l = (float)(q2 * kLog2e);
-  s.gl = valid ? (float)(g * kLog2e) : -INFINITY;
+  // (quarter turn minus theta: (sin, cos); minus a phase: the conjugate)
+  const uint32_t flip = swap ? 0xffffffffu : 0u;
+  const uint32_t t = fixed_revolutions(theta0);
+  s.z = phasor(swap ? 0x40000000u - t : t);
+  s.r = phasor(((a + b) ^ flip) - flip);  // theta(1) - theta(0) = A + B
+  s.k = phasor(((2u * b) ^ flip) - flip);  // second difference 2 B
+  s.t0 = (float)(p0 - v.cen);
+  s.q2l = v.q2l;
+  s.gl = valid ? v.gl + exponent : -INFINITY;
   return s;
 }
 
@@ -224,151 +326,235 @@ __device__ __forceinline__ float2 seg_next(SegGen& s, int j) {
   return v;
 }
 
-// One k pair of the complex product a b (a = Ey_k(m), b = Ex_k(n): this
-// lane's operands) in three real products (Gauss): p1 += a.re b.re,
-// p2 += a.im b.im, p3 += (a.re + a.im)(b.re + b.im); then Re = p1 - p2 and
-// Im = p3 - (p1 + p2).  Three MFMAs per k pair instead of four (no vector
-// instruction and MFMA of one SIMD run together, so the two adds cost far
-// less than the fourth product).
-__device__ __forceinline__ void sep_mfma(float2 a, float2 b, floatx16& p1, floatx16& p2, floatx16& p3) {
-  p1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, p1, 0, 0, 0);
-  p2 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, p2, 0, 0, 0);
-  p3 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x + a.y, b.x + b.y, p3, 0, 0, 0);
+// Two values rounded to f16, packed (first in the low half), and what the
+// rounding left of them (one mixed-precision instruction each).
+__device__ __forceinline__ uint32_t take_f16(float& u, float& v) {
+  const f16x2 p = __builtin_convertvector((floatx2){u, v}, f16x2);
+  const uint32_t w = __builtin_bit_cast(uint32_t, p);
+  asm("v_fma_mix_f32 %0, %1, -1.0, %0 op_sel_hi:[1,0,0]" : "+v"(u) : "v"(w));
+  asm("v_fma_mix_f32 %0, %1, -1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(v) : "v"(w));
+  return w;
 }
 
-__global__ __launch_bounds__(kThreads) void beamlet_sum_sep_kernel(const tg_beamlet_coef* __restrict__ coef,
-                                                                   const SepParams* __restrict__ par, int64_t n,
-                                                                   int64_t H, int64_t W, int32_t ntx, int32_t ntiles,
-                                                                   int32_t nsplit, const int32_t* __restrict__ flags,
-                                                                   float2* __restrict__ ws) {
-  __shared__ int32_t list[kSepBlock];
-  __shared__ int32_t wave_cnt[kWaves];
-  __shared__ float2 fac[2][2][kSepK][kSepRow];  // [buffer][x: Ex_k(tx0 + n), y: Ey_k(ty0 + m)][k][pixel]
+// Pixel j of a segment: lanes k (even) and k + 1 exchange their second
+// components; high and low get the halves of both beamlets' real parts (even
+// lane) or imaginary parts (odd lane, whose values come as (im, re)).
+__device__ __forceinline__ void mx_pack(float2 v, bool odd, uint32_t& high, uint32_t& low) {
+  const float got = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v.y), 0xB1, 0xF, 0xF, true));  // lane ^ 1
+  float a = odd ? got : v.x, b = odd ? v.x : got;
+  high = take_f16(a, b);
+  low = __builtin_bit_cast(uint32_t, __builtin_convertvector((floatx2){a, b}, f16x2));
+}
+
+// Operands of one component: its high and low halves.
+struct MxOperand {
+  f16x8 h, l;
+};
+
+template <int PART>
+__device__ __forceinline__ MxOperand mx_load(const uint32_t* src) {
+  return {*reinterpret_cast<const f16x8*>(src), *reinterpret_cast<const f16x8*>(src + 2 * PART)};
+}
+
+__device__ __forceinline__ f16x8 mx_neg(f16x8 v) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(f16x8, __builtin_bit_cast(u32x4, v) ^ 0x80008000u);
+}
+
+// Product P of the 12 of a 32x32 block: the three of a real product (smallest
+// first), for each of re += ar br, im += ai br, re -= ai bi, im += ar bi; the
+// real and imaginary sums in turn.
+template <int P>
+__device__ __forceinline__ void mx_mfma(const MxOperand& ar, const MxOperand& ai, const MxOperand& br,
+                                        const MxOperand& bi, const MxOperand& bn, floatx16& re, floatx16& im) {
+  constexpr bool to_im = P & 1, second = P >= 6;
+  constexpr int part = (P / 2) % 3;
+  const MxOperand& a = to_im != second ? ai : ar;
+  const MxOperand& b = !second ? br : to_im ? bi : bn;
+  floatx16& acc = to_im ? im : re;
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(part == 0 ? a.l : a.h, part == 1 ? b.l : b.h, acc, 0, 0, 0);
+}
+
+// f(0), f(1), ... f(N - 1) with compile-time arguments
+template <int N, class F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl<N>(f, std::make_integer_sequence<int, N>{});
+}
+
+template <class M>
+__global__ __launch_bounds__(M::kThreads, 2) void beamlet_sum_sep_kernel(const SepTables tab, int64_t n, int64_t H,
+                                                                    int64_t W, int32_t ntx, int32_t nsplit,
+                                                                    const int32_t* __restrict__ flags,
+                                                                    float2* __restrict__ ws) {
+  constexpr int kT = M::kThreads, kW = M::kWaves, TW = M::TW, TH = M::TH;
+  __shared__ int32_t list[kMxBlock];
+  __shared__ int32_t wave_cnt[kW], wave_exp[kW];
+  __shared__ __align__(16) uint32_t fac[2][M::kBuffer];
   if (!matrix_path(flags)) return;  // beamlet_sum_kernel covers this launch
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   // the slices of one tile are consecutive workgroups: the heavy tiles near
   // the pattern's centre are spread through the dispatch order instead of
   // all ending it
   const int split = blockIdx.x % nsplit, tile = blockIdx.x / nsplit;
-  const int32_t tx0 = (tile % ntx) * kTileW, ty0 = (tile / ntx) * kTileH;
+  const int32_t tx0 = (tile % ntx) * TW, ty0 = (tile / ntx) * TH;
   const int64_t b_begin = n * split / nsplit, b_end = n * (split + 1) / nsplit;
-  const float ftx0 = (float)tx0, fty0 = (float)ty0, ftx1 = (float)(tx0 + kTileW - 1), fty1 = (float)(ty0 + kTileH - 1);
-  const int mb = (wave >> 1) * 32, nb = (wave & 1) * 32;
-  // this thread's segment: beamlet gk of a chunk, axis (waves 0-1: x, 2-3: y), pixels p0 .. p0 + 15
-  const int gk = t & (kSepK - 1), gaxis = t >> 7, s0 = ((t >> 5) & 3) * kSepSeg;
-  const double p0 = (double)((gaxis == 0 ? tx0 : ty0) + s0);
-  floatx16 p1, p2, p3;
+  const float ftx0 = (float)tx0, fty0 = (float)ty0, ftx1 = (float)(tx0 + TW - 1), fty1 = (float)(ty0 + TH - 1);
+  constexpr int kCols = TW / (32 * M::BN);
+  const int mb = (wave / kCols) * 32 * M::BM, nb = (wave % kCols) * 32 * M::BN;
+  // operand reads: A[m][k] = Ey_k(ty0 + mb + m), B[k][n] = Ex_k(tx0 + nb + n); lane l holds row (column) l % 32,
+  // k = 8 (l / 32) .. + 7 (v_mfma_f32_32x32x16 operand layout)
+  const int a_at = mx_row(TW + mb + (lane & 31)) + 4 * (lane >> 5), b_at = mx_row(nb + (lane & 31)) + 4 * (lane >> 5);
+  // this thread's segment: beamlet gk of a chunk, 16 pixels from p0 of one axis
+  // (one axis a wave: TW is a multiple of a wave's pixels)
+  const int gk = t % M::KC, seg = t / M::KC;
+  const bool y_axis = __builtin_amdgcn_readfirstlane(seg * kMxSeg) >= TW, odd = lane & 1;
+  const double p0 = (double)(y_axis ? ty0 + seg * kMxSeg - TW : tx0 + seg * kMxSeg);
+  const double dtx0 = (double)tx0, dtx1 = (double)(tx0 + TW - 1);
+  const int dst_at = (gk / kMxK) * M::kStep + odd * M::kPart + mx_row(seg * kMxSeg) + (gk % kMxK) / 2;
+  floatx16 re[M::BM][M::BN], im[M::BM][M::BN];
 #pragma unroll
-  for (int j = 0; j < 16; ++j) p1[j] = p2[j] = p3[j] = 0.0f;
-  for (int64_t blk = b_begin; blk < b_end; blk += kSepBlock) {
-    // the beamlets of [blk, blk + kSepBlock) whose cutoff ellipse meets the
+  for (int i = 0; i < M::BM; ++i)
+#pragma unroll
+    for (int k = 0; k < M::BN; ++k)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) re[i][k][j] = im[i][k][j] = 0.0f;
+  int exp_now = kNoExp;  // the sums are held times 2^(2 kMxScale - exp_now)
+  for (int64_t blk = b_begin; blk < b_end; blk += kMxBlock) {
+    // the beamlets of [blk, blk + kMxBlock) whose cutoff ellipse meets the
     // tile, in order.  A separable beamlet's ellipse is axis-aligned
     // (alpha = 0): u^2 + gamma v^2 <= beta, so the tile's pixel centre nearest
     // (cx, cy) decides, exactly -- tiles in the corners of the ellipse's
     // bounding box are skipped.
-    int cnt = 0;
-    for (int64_t b0 = blk; b0 < b_end && b0 < blk + kSepBlock; b0 += kThreads) {
+    int cnt = 0, exp_blk = kNoExp;
+    for (int64_t b0 = blk; b0 < b_end && b0 < blk + kMxBlock; b0 += kT) {
       const int64_t b = b0 + t;
       bool hit = false;
+      int top = kNoExp;
       if (b < b_end) {
-        const tg_beamlet_coef& c = coef[b];
-        const float du = fmaxf(fmaxf(ftx0 - c.cx, c.cx - ftx1), 0.0f);
-        const float dv = fmaxf(fmaxf(fty0 - c.cy, c.cy - fty1), 0.0f);
-        hit = fmaf(c.gamma * dv, dv, du * du) <= c.beta;
+        const float4 c = tab.cull[b];  // cx, cy, gamma, beta
+        const float2 p = tab.peak[b];
+        const float du = fmaxf(fmaxf(ftx0 - c.x, c.x - ftx1), 0.0f);
+        const float dv = fmaxf(fmaxf(fty0 - c.y, c.y - fty1), 0.0f);
+        hit = fmaf(c.z * dv, dv, du * du) <= c.w;
+        // no term of the beamlet in this tile exceeds 2^top (the centre's f32 rounding taken off the distances)
+        const float dus = fmaxf(fmaf(-0x1p-22f, fabsf(c.x), du), 0.0f), dvs = fmaxf(fmaf(-0x1p-22f, fabsf(c.y), dv), 0.0f);
+        if (hit) top = (int)fminf(fmaxf(ceilf(fmaf(p.y, fmaf(c.z * dvs, dvs, dus * dus), p.x)), -1e6f), 1e6f) + 1;
       }
       const uint64_t mask = __ballot(hit);
-      if (lane == 0) wave_cnt[wave] = __popcll(mask);
+      top = wave_max_i32(top);
+      if (lane == 0) wave_cnt[wave] = __popcll(mask), wave_exp[wave] = top;
       __syncthreads();
       int off = cnt, total = 0;
 #pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
+      for (int w = 0; w < kW; ++w) {
         off += (w < wave) ? wave_cnt[w] : 0;
         total += wave_cnt[w];
+        exp_blk = max(exp_blk, wave_exp[w]);
       }
       if (hit) list[off + __popcll(mask & ((1ull << lane) - 1ull))] = (int32_t)(b - blk);
       cnt += total;
       __syncthreads();  // wave_cnt is rewritten next; the list is complete after the last pass
     }
     if (cnt == 0) continue;
-    const int nch = (cnt + kSepK - 1) / kSepK;
-    // chunk q's beamlet for this thread (past cnt: the last one again, evaluated as zero)
-    auto beamlet = [&](int q) -> int64_t { return blk + list[min(q * kSepK + gk, cnt - 1)]; };
-    double2 v0, v1, v2;  // the parameters of the chunk evaluated next
-    load_axis(par, beamlet(0), gaxis, v0, v1, v2);
-    {
-      SegGen sg = seg_setup(v0, v1, v2, p0, gk < cnt);
-      float2* dst = &fac[0][gaxis][gk][s0];
+    if (exp_blk > exp_now) {  // larger terms than so far: the sums move to their scale (an exact power of two)
+      if (exp_now != kNoExp) {
 #pragma unroll
-      for (int j = 0; j < kSepSeg; ++j) dst[j] = seg_next(sg, j);
+        for (int i = 0; i < M::BM; ++i)
+#pragma unroll
+          for (int k = 0; k < M::BN; ++k)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+              re[i][k][j] = ldexpf(re[i][k][j], exp_now - exp_blk);
+              im[i][k][j] = ldexpf(im[i][k][j], exp_now - exp_blk);
+            }
+      }
+      exp_now = exp_blk;
     }
-    load_axis(par, beamlet(1), gaxis, v0, v1, v2);
+    const int nch = (cnt + M::KC - 1) / M::KC;
+    // chunk q's beamlet for this thread (past cnt: the last one again,
+    // evaluated as zero), and the power of two its factor is multiplied by: an
+    // x factor's largest value in the tile goes to [2^14, 2^15) and the y
+    // factor takes the rest
+    float ex = 0.0f;
+    auto load = [&](int q) {
+      const int64_t i = blk + list[min(q * M::KC + gk, cnt - 1)];
+      const SepAxis a = load_sep(tab, i, y_axis);
+      const double* x = tab.x + 4 * i;
+      const float qx = y_axis ? __int_as_float(__double2loint(x[0])) : a.q2l;
+      const double cen = y_axis ? x[3] : a.cen;
+      const float du = (float)fmax(fmax(dtx0 - cen, cen - dtx1), 0.0);
+      const float top = fmaxf(floorf(qx * du * du), -1e6f);
+      ex = (float)kMxScale + (y_axis ? top - (float)exp_now : -top);
+      return a;
+    };
+    SepAxis v = load(0);
+    {
+      SegGen sg = seg_setup(v, p0, ex, gk < cnt, odd);
+      v = load(1);
+      uint32_t* dst = &fac[0][dst_at];
+#pragma unroll
+      for (int j = 0; j < kMxSeg; ++j)
+        mx_pack(seg_next(sg, j), odd, dst[j * (kMxK / 2)], dst[j * (kMxK / 2) + 2 * M::kPart]);
+    }
     __syncthreads();
     for (int c = 0; c < nch; ++c) {
-      const int cur = c & 1;
-      // A[m][k] = Ey_k(ty0 + mb + m) from lane m + 32 k, B[k][n] = Ex_k(tx0 + nb + n)
-      // from lane n + 32 k (v_mfma_f32_32x32x2f32 operand layout); every
-      // chunk runs all kSepK (zero past cnt)
-      // (operands one k pair ahead, so LDS latency hides behind the products)
-      const float2* ea = &fac[cur][1][lane >> 5][mb + (lane & 31)];
-      const float2* eb = &fac[cur][0][lane >> 5][nb + (lane & 31)];
-      float2 a = ea[0], b = eb[0];
-      if (c + 1 < nch) {
-        // chunk c + 1 into the other buffer, one segment value per k pair,
-        // and chunk c + 2's parameters in flight
-        SegGen sg = seg_setup(v0, v1, v2, p0, (c + 1) * kSepK + gk < cnt);
-        load_axis(par, beamlet(c + 2), gaxis, v0, v1, v2);
-        // keep these loads here: sunk below the products (as the scheduler
-        // does by itself), the next chunk waited a whole memory round trip
-        __builtin_amdgcn_sched_barrier(0);
-        // (the values are stored after the products: a store into the
-        // other buffer between them would order every later operand read
-        // behind it)
-        float2 val[kSepSeg];
+      const uint32_t* cur = fac[c & 1];
+      constexpr int S = M::KC / kMxK;
+      MxOperand ar[S][M::BM], ai[S][M::BM], br[S][M::BN], bi[S][M::BN], bn;
 #pragma unroll
-        for (int kk = 0; kk < kSepK; kk += 2) {
-          float2 an = a, bn = b;
-          if (kk + 2 < kSepK) {
-            an = ea[(kk + 2) * kSepRow];
-            bn = eb[(kk + 2) * kSepRow];
-          }
-          sep_mfma(a, b, p1, p2, p3);
-          val[kk >> 1] = seg_next(sg, kk >> 1);
-          a = an;
-          b = bn;
-          // issue order: products and the value's dependent vector
-          // instructions alternate (each covers the other's latency)
+      for (int s = 0; s < S; ++s) {
 #pragma unroll
-          for (int i = 0; i < 3; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // four VALU
-          }
+        for (int i = 0; i < M::BM; ++i) {
+          ar[s][i] = mx_load<M::kPart>(cur + s * M::kStep + a_at + i * kBlockRow);
+          ai[s][i] = mx_load<M::kPart>(cur + s * M::kStep + M::kPart + a_at + i * kBlockRow);
         }
-        float2* dst = &fac[cur ^ 1][gaxis][gk][s0];
 #pragma unroll
-        for (int j = 0; j < kSepSeg; ++j) dst[j] = val[j];
-      } else {
-#pragma unroll
-        for (int kk = 0; kk < kSepK; kk += 2) {
-          float2 an = a, bn = b;
-          if (kk + 2 < kSepK) {
-            an = ea[(kk + 2) * kSepRow];
-            bn = eb[(kk + 2) * kSepRow];
-          }
-          sep_mfma(a, b, p1, p2, p3);
-          a = an;
-          b = bn;
+        for (int k = 0; k < M::BN; ++k) {
+          br[s][k] = mx_load<M::kPart>(cur + s * M::kStep + b_at + k * kBlockRow);
+          bi[s][k] = mx_load<M::kPart>(cur + s * M::kStep + M::kPart + b_at + k * kBlockRow);
         }
       }
-      __syncthreads();  // chunk c + 1 is complete; the next iteration rewrites buffer `cur`
+      // chunk c + 1's factors (past the last chunk: zeros nobody reads), and
+      // chunk c + 2's parameters in flight
+      SegGen sg = seg_setup(v, p0, ex, (c + 1) * M::KC + gk < cnt, odd);
+      v = load(c + 2);
+      __builtin_amdgcn_s_setprio(1);
+      uint32_t* dst = &fac[(c & 1) ^ 1][dst_at];
+      // a pixel of the segment beside its share of the products.  (The barriers
+      // keep the steps apart: left alone, the scheduler issues all products
+      // first and the evaluation after them.)
+      static_for<kMxSeg>([&](auto step) {
+        constexpr int j = step, kMfma = 12 * M::BM * M::BN * S;
+        __builtin_amdgcn_sched_barrier(0);
+        static_for<(j + 1) * kMfma / kMxSeg - j * kMfma / kMxSeg>([&](auto sub) {
+          constexpr int q = j * kMfma / kMxSeg + sub, P = q % 12;
+          constexpr int i = q / 12 % M::BM, k = q / (12 * M::BM) % M::BN, s = q / (12 * M::BM * M::BN);
+          if constexpr (P == 0 && i == 0) bn = {mx_neg(bi[s][k].h), mx_neg(bi[s][k].l)};
+          mx_mfma<P>(ar[s][i], ai[s][i], br[s][k], bi[s][k], bn, re[i][k], im[i][k]);
+        });
+        mx_pack(seg_next(sg, j), odd, dst[j * (kMxK / 2)], dst[j * (kMxK / 2) + 2 * M::kPart]);
+      });
+      __builtin_amdgcn_s_setprio(0);
+      __syncthreads();  // chunk c + 1 is complete and chunk c read
     }
   }
   // accumulator j of lane l holds row 8 (j / 4) + 4 (l / 32) + j % 4, column l % 32
 #pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int64_t py = ty0 + mb + 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
-    const int64_t px = tx0 + nb + (lane & 31);
-    if (py < H && px < W) ws[((int64_t)split * H + py) * W + px] = make_float2(p1[j] - p2[j], p3[j] - (p1[j] + p2[j]));
-  }
+  for (int i = 0; i < M::BM; ++i)
+#pragma unroll
+    for (int k = 0; k < M::BN; ++k)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const int64_t py = ty0 + mb + 32 * i + 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
+        const int64_t px = tx0 + nb + 32 * k + (lane & 31);
+        if (py < H && px < W)
+          ws[((int64_t)split * H + py) * W + px] =
+              make_float2(ldexpf(re[i][k][j], exp_now - 2 * kMxScale), ldexpf(im[i][k][j], exp_now - 2 * kMxScale));
+      }
 }
 
 __global__ __launch_bounds__(256) void split_sum_kernel(const float2* __restrict__ ws, int64_t npix, int32_t nsplit,
@@ -525,6 +711,14 @@ int splits_for(int64_t n, int64_t H, int64_t W) {
   return (int)s;
 }
 
+template <class M>
+void launch_sep_sum(const SepTables& tab, int64_t n, int64_t H, int64_t W, int nsplit, const int32_t* flags, float2* ws,
+                    hipStream_t s) {
+  const int64_t ntx = tg::cdiv(W, (int64_t)M::TW), ntiles = ntx * tg::cdiv(H, (int64_t)M::TH);
+  hipLaunchKernelGGL(beamlet_sum_sep_kernel<M>, dim3((unsigned)(ntiles * nsplit)), dim3(M::kThreads), 0, s, tab, n, H,
+                     W, (int32_t)ntx, (int32_t)nsplit, flags, ws);
+}
+
 // The recurrence tile sum (beamlet_sum_kernel) for a tile shape
 // (tg_tile_shape): one workgroup per (tile, beamlet slice).
 int launch_recurrence_sum(int32_t shape, const tg_beamlet_coef* coef, int64_t n, int64_t H, int64_t W, int nsplit,
@@ -575,13 +769,13 @@ extern "C" int tg_beamlet_coefficients(const double* params, int64_t n, const do
 }
 
 // Workspace of tg_beamlet_sum: [nsplit, H, W] complex64 slice tiles (padded to
-// 256 bytes), the kFlagBlocks path flags, then n SepParams records.
+// 256 bytes), the kFlagBlocks path flags, then n separable beamlets' factors.
 int64_t slices_bytes(int nsplit, int64_t H, int64_t W) {
   return ((int64_t)nsplit * H * W * (int64_t)sizeof(float2) + 255) / 256 * 256;
 }
 
 int64_t sum_workspace_bytes(int nsplit, int64_t n, int64_t H, int64_t W) {
-  return slices_bytes(nsplit, H, W) + kFlagBlocks * (int64_t)sizeof(int32_t) + n * (int64_t)sizeof(SepParams);
+  return slices_bytes(nsplit, H, W) + kFlagBlocks * (int64_t)sizeof(int32_t) + n * kSepBytes;
 }
 
 extern "C" int64_t tg_beamlet_sum_workspace(int64_t n, int64_t height, int64_t width) {
@@ -609,15 +803,13 @@ extern "C" int tg_beamlet_sum(const tg_beamlet_coef* coef, int64_t n, int64_t he
   int32_t path = TG_BEAMLET_PATH_AUTO;
   tg::tune_lookup(TG_TUNE_BEAMLET_PATH, key, path);
   int32_t* flags = (int32_t*)((char*)workspace + slices);
-  SepParams* par = (SepParams*)(flags + kFlagBlocks);
+  const SepTables tab = sep_tables(flags + kFlagBlocks, n);
   // which tile sum runs is decided on the device (no host round trip, so the
   // call stays graph-capturable); the other kernel's workgroups exit at once
   hipLaunchKernelGGL(sep_flag_kernel, dim3(kFlagBlocks), dim3(256), 0, (hipStream_t)stream, coef, n,
-                     (int32_t)(path == TG_BEAMLET_PATH_VALU), flags, par);
+                     (int32_t)(path == TG_BEAMLET_PATH_VALU), flags, tab);
   TG_LAUNCH_CHECK("sep_flag_kernel launch");
-  hipLaunchKernelGGL(beamlet_sum_sep_kernel, dim3((unsigned)(ntiles * nsplit)), dim3(kThreads), 0,
-                     (hipStream_t)stream, coef, (const SepParams*)par, n, height, width, (int32_t)ntx,
-                     (int32_t)ntiles, (int32_t)nsplit, (const int32_t*)flags, (float2*)workspace);
+  launch_sep_sum<SepTile>(tab, n, height, width, nsplit, flags, (float2*)workspace, (hipStream_t)stream);
   TG_LAUNCH_CHECK("beamlet_sum_sep_kernel launch");
   int32_t shape = TG_TILE_64x64_RUN16;
   tg::tune_lookup(TG_TUNE_TILE_SHAPE, key, shape);
