@@ -343,6 +343,7 @@ int tg_stem_fit_noalloc(const tg_stem_geometry* g, const double* params, const f
  * x, y, dx, dy, pathlength, amp_re, amp_im, waist_x, waist_y, radius_x,
  * radius_y (inf allowed), wavelength, theta, 0, 0, 0. */
 #define TG_BEAMLET_NPARAM 16
+#define TG_BEAMLET_NCOLUMN 13 /* the columns that have a meaning */
 
 enum tg_beamlet_mode {
   TG_BEAMLET_PROPAGATED = 0,  /* make_gaussian_image: field after a 5x5 ABCD   */
@@ -362,6 +363,24 @@ typedef struct tg_beamlet_coef {
   float box_w, box_h;  /* half-extents of that ellipse (pixels; huge: unbounded) */
 } tg_beamlet_coef;     /* 136 bytes */
 
+/* One parameter column of n beamlets: element i at data + i stride (elements;
+ * stride 0: one value in device memory for all), or `value` for all. */
+enum { TG_COLUMN_VALUE = 0, TG_COLUMN_F32 = 1, TG_COLUMN_F64 = 2 };
+typedef struct tg_beamlet_column {
+  const void* data;
+  int64_t stride;
+  double value;
+  int32_t type;
+  int32_t pad;
+} tg_beamlet_column;  /* 32 bytes */
+
+/* Parameter rows from columns: params[i, c] = columns[c] of beamlet i for the
+ * TG_BEAMLET_NCOLUMN columns that have a meaning, 0 behind them.  `matrix` (25
+ * f64 on the host, or NULL) is written to matrix_out (device): a shared
+ * ray-transfer matrix. */
+int tg_beamlet_pack(const tg_beamlet_column* columns, int64_t n, double* params, const double* matrix,
+                    double* matrix_out, void* stream);
+
 /* Coefficients of n beamlets.
  *   params  [n, TG_BEAMLET_NPARAM] f64 (device)
  *   abcd    [n or 1, 5, 5] f64 ray-transfer matrices (propagated mode; NULL
@@ -379,10 +398,10 @@ int tg_beamlet_coefficients(const double* params, int64_t n, const double* abcd,
  * Two tile sums (tg_beamlet_path), chosen on the device per launch:
  *   - every beamlet separable (Phi without a px*py term, envelope decaying
  *     along both axes, as for untilted round or axis-aligned beams): each
- *     64x64 tile is a complex matrix product Ey^T Ex over the beamlets whose
- *     cutoff box overlaps it, Ex/Ey from f64 phases, on the matrix cores
- *     (f32 MFMA); culling is per tile, so terms below the cut inside an
- *     overlapping tile are summed too;
+ *     128x128 tile is a complex matrix product Ey^T Ex over the beamlets whose
+ *     cutoff ellipse meets it, Ex/Ey from f64 phases, on the matrix cores
+ *     (factors as two f16 halves, f32 sums); culling is per tile, so terms
+ *     below the cut inside such a tile are summed too;
  *   - otherwise the per-lane f32 recurrence over 16-pixel runs, culled per
  *     run to the cutoff ellipse. */
 int64_t tg_beamlet_sum_workspace(int64_t n, int64_t height, int64_t width);

@@ -32,6 +32,8 @@
 //   dL/dtheta = Re[amp sum_k G_k dc_k/dtheta]
 // with dc_k/dtheta from forward-mode dual numbers through the same
 // coefficient algebra (one pass per parameter and ray-transfer entry).
+#include <string.h>
+
 #include <utility>
 
 #include "beamlet_common.hpp"
@@ -39,6 +41,32 @@
 namespace {
 
 using namespace tgb;
+
+// The parameter rows of n beamlets from their 13 columns (an array each, or a
+// value for all), and a matrix that the host knows: one launch in place of the
+// torch operations that converted, stacked and copied them.  Bound: the launch,
+// the rows' store for many beamlets (131,072: 17 MB).  A lane writes one entry,
+// so that a wavefront stores 512 bytes in a row.
+struct PackArgs {
+  tg_beamlet_column col[TG_BEAMLET_NCOLUMN];
+  double matrix[25];
+};
+
+__global__ __launch_bounds__(256) void beamlet_pack_kernel(const PackArgs a, int64_t n, double* __restrict__ out,
+                                                           double* __restrict__ matrix_out) {
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (matrix_out != nullptr && i < 25) matrix_out[i] = a.matrix[i];
+  const int c = threadIdx.x % TG_BEAMLET_NPARAM;  // the stride below is a multiple of it
+  const tg_beamlet_column col = a.col[c < TG_BEAMLET_NCOLUMN ? c : 0];
+  const int32_t type = c < TG_BEAMLET_NCOLUMN ? col.type : TG_COLUMN_VALUE;
+  const double value = c < TG_BEAMLET_NCOLUMN ? col.value : 0.0;
+  for (; i < n * TG_BEAMLET_NPARAM; i += (int64_t)gridDim.x * 256) {
+    const int64_t at = i / TG_BEAMLET_NPARAM * col.stride;
+    out[i] = type == TG_COLUMN_F64   ? static_cast<const double*>(col.data)[at]
+             : type == TG_COLUMN_F32 ? (double)static_cast<const float*>(col.data)[at]
+                                     : value;
+  }
+}
 
 __global__ __launch_bounds__(256) void beamlet_coef_kernel(const double* __restrict__ params, int64_t n,
                                                            const double* __restrict__ abcd, int64_t abcd_stride,
@@ -749,6 +777,29 @@ int launch_recurrence_sum(int32_t shape, const tg_beamlet_coef* coef, int64_t n,
 }
 
 }  // namespace
+
+extern "C" int tg_beamlet_pack(const tg_beamlet_column* columns, int64_t n, double* params, const double* matrix,
+                               double* matrix_out, void* stream) {
+  tg::clear_error();
+  TG_REQUIRE(n >= 0, "tg_beamlet_pack: negative count");
+  TG_REQUIRE((matrix == nullptr) == (matrix_out == nullptr), "tg_beamlet_pack: matrix and matrix_out go together");
+  if (n == 0 && matrix == nullptr) return TG_OK;
+  TG_REQUIRE(n == 0 || (columns != nullptr && params != nullptr), "tg_beamlet_pack: NULL buffer");
+  PackArgs a{};
+  for (int c = 0; c < TG_BEAMLET_NCOLUMN && n > 0; ++c) {
+    a.col[c] = columns[c];
+    TG_REQUIRE(columns[c].type >= TG_COLUMN_VALUE && columns[c].type <= TG_COLUMN_F64,
+               "tg_beamlet_pack: column %d has an unknown type %d", c, columns[c].type);
+    TG_REQUIRE(columns[c].type == TG_COLUMN_VALUE || columns[c].data != nullptr, "tg_beamlet_pack: column %d is NULL",
+               c);
+  }
+  if (matrix != nullptr) memcpy(a.matrix, matrix, sizeof(a.matrix));
+  const int64_t blocks = tg::cdiv(n * TG_BEAMLET_NPARAM, 256);
+  hipLaunchKernelGGL(beamlet_pack_kernel, dim3((unsigned)(blocks < 1 ? 1 : blocks > 16384 ? 16384 : blocks)),
+                     dim3(256), 0, (hipStream_t)stream, a, n, params, matrix_out);
+  TG_LAUNCH_CHECK("beamlet_pack_kernel launch");
+  return TG_OK;
+}
 
 extern "C" int tg_beamlet_coefficients(const double* params, int64_t n, const double* abcd, int64_t abcd_stride,
                                        int32_t mode, const double* pix2m, double nsigma, tg_beamlet_coef* out,
