@@ -34,6 +34,8 @@
 // coefficient algebra (one pass per parameter and ray-transfer entry).
 #include <string.h>
 
+#include <algorithm>
+#include <cmath>
 #include <utility>
 
 #include "beamlet_common.hpp"
@@ -250,7 +252,7 @@ __global__ __launch_bounds__(kThreads) void beamlet_sum_kernel(const tg_beamlet_
 // pairs per segment instead of a sine and cosine per value).
 //
 // 131,072 beamlets, 1024^2, 4 sigma, the whole sum: 4.64 ms with f32 products,
-// now 2.4 ms (tile sum 2.25, slices 0.105).  Bound: vector issue (63% of the
+// now 2.15 ms (tile sum 2.06, slices 0.08).  Bound: vector issue (63% of the
 // cycles, 520 instructions a chunk) and the matrix cores (46%) together, at
 // the 1.9 GHz that this mix runs at.
 // ---------------------------------------------------------------------------
@@ -585,12 +587,25 @@ __global__ __launch_bounds__(M::kThreads, 2) void beamlet_sum_sep_kernel(const S
       }
 }
 
+// The slices' sum, in order.  Bound: reading them; four loads in flight hide
+// some of the latency where a small image has too few wavefronts for that (300
+// beamlets on 100^2 pixels, the whole sum in 64 slices: 34 -> 24 us; eight: 22,
+// but large images lose 3%).
 __global__ __launch_bounds__(256) void split_sum_kernel(const float2* __restrict__ ws, int64_t npix, int32_t nsplit,
                                                         float2* __restrict__ field) {
+  constexpr int kAhead = 4;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= npix) return;
   double re = 0.0, im = 0.0;
-  for (int s = 0; s < nsplit; ++s) {
+  int s = 0;
+  for (; s + kAhead <= nsplit; s += kAhead) {
+    float2 v[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) v[k] = ws[(int64_t)(s + k) * npix + i];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) re += v[k].x, im += v[k].y;
+  }
+  for (; s < nsplit; ++s) {
     const float2 v = ws[(int64_t)s * npix + i];
     re += v.x;
     im += v.y;
@@ -727,13 +742,22 @@ int splits_for(int64_t n, int64_t H, int64_t W) {
     return (int)s;
   }
   const int64_t ntiles = tg::cdiv(H, kTileH) * tg::cdiv(W, kTileW);
-  // Many small work items (tile x beamlet slice) let the hardware scheduler
-  // balance tiles near the centre of the pattern, which overlap many more
-  // beamlets than the edge tiles.
-  const int64_t want = 64LL * tg::cu_count();
-  int64_t s = tg::cdiv(want, ntiles);
-  const int64_t by_n = tg::cdiv(n, 256);  // at least ~256 beamlets per slice
-  if (s > by_n) s = by_n;
+  // Few beamlets: about six workgroups of 64x64 pixels a CU, down to slices of
+  // sqrt(n) beamlets, below which the slices' own cost (a start, a partial
+  // image) takes over.  Whole sums, 256 beamlets a slice as a rule / this one:
+  // 500 rotated beamlets on 300^2 203 / 40 us, 2,048 on 500 x 612 120 / 77,
+  // 300 on 100^2 132 / 28, 64 on 64^2 63 / 18; 4,096 on 600 x 612 65 / 65, 64 on
+  // 600 x 612 34 / 36 (4 slices: 24).
+  // Many separable ones: whole rounds of the matrix-core kernel's tiles (two
+  // workgroups a CU at a time; tiles of uneven weight want some rounds), slices
+  // of at least 600.  20,000 on 512^2: 32 slices, a round, 152 us, 39 slices
+  // 212; 131,072 on 1024^2: 16 / 32 / 64 / 128 slices 2.50 / 2.15 / 2.15 /
+  // 2.30 ms; 50,000 on 1000 x 300 533 / 468 us.
+  const int64_t few = std::min<int64_t>(6LL * tg::cu_count() / ntiles, (int64_t)std::sqrt((double)n));
+  const int64_t sep_tiles = tg::cdiv(H, (int64_t)SepTile::TH) * tg::cdiv(W, (int64_t)SepTile::TW);
+  const int64_t slots = 2LL * tg::cu_count();
+  const int64_t rounds = std::min<int64_t>(4, (int64_t)((double)n * (double)sep_tiles / (600.0 * (double)slots)));
+  int64_t s = std::max(few, rounds * slots / sep_tiles);
   if (s > 128) s = 128;
   if (s < 1) s = 1;
   return (int)s;

@@ -1,0 +1,22 @@
+"""The beamlet slices that tg_beamlet_sum_workspace reserves: 1 to 128, never
+more than the beamlets, over sizes from nothing to the largest."""
+import numpy as np
+import pytest
+
+from temgymcore_amd import _lib, autotune
+from temgymcore_amd import gaussian  # noqa: F401  (registers the signatures)
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_slices_are_bounded(seed):
+    lib = _lib.load()
+    autotune.clear()
+    rng = np.random.default_rng(seed)
+    sizes = np.exp(rng.uniform(0, np.log(4096), (200, 2))).astype(int) + 1
+    for (h, w), n in zip(sizes.tolist(), np.exp(rng.uniform(0, np.log(2e6), 200)).astype(int).tolist()):
+        for k in (0, 1, n):
+            slices = lib.tg_beamlet_sum_workspace(k, h, w) - 256 * 4 - 96 * k
+            assert slices % 256 == 0
+            low = slices - 255
+            nsplit = [s for s in range(1, 129) if low <= s * h * w * 8 <= slices]
+            assert nsplit and nsplit[0] <= max(k, 1)
