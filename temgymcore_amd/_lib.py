@@ -8,6 +8,7 @@ stale library raises ``RuntimeError``.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import threading
 
@@ -168,8 +169,15 @@ def check(status: int, what: str) -> None:
     raise RuntimeError(f"{what}: {msg}")
 
 
+@functools.lru_cache(maxsize=None)
+def _device(index: int) -> torch.device:
+    return torch.device("cuda", index)
+
+
 def require_device() -> torch.device:
     """The HIP device vectorised work runs on (torch's current device)."""
+    if torch.cuda.is_initialized():
+        return _device(torch._C._cuda_getDevice())
     if not torch.cuda.is_available():
         raise RuntimeError(
             "temgymcore_amd: vectorised rays run on the MI355X HIP kernels and need a GPU; "
@@ -179,5 +187,9 @@ def require_device() -> torch.device:
 
 
 def stream_ptr(device: torch.device | None = None) -> int:
-    """Raw hipStream_t of torch's current stream on `device`."""
-    return torch.cuda.current_stream(device).cuda_stream
+    """Raw hipStream_t of torch's current stream on `device` (without the
+    Stream object that torch.cuda.current_stream makes: 0.1 us for 1.8)."""
+    if not torch.cuda.is_initialized():
+        return torch.cuda.current_stream(device).cuda_stream
+    index = None if device is None else device.index
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice() if index is None else index)

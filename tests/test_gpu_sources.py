@@ -110,3 +110,20 @@ def test_device_rays_feed_the_ray_program(device):
     ref = O.run_to_end(O.make_ray(*host, 0.0, 0.0), [("plane", 0.0), ("lens", 0.5, 0.25), ("detector", 1.0)])
     for k in ("x", "y", "dx", "dy", "pathlength"):
         np.testing.assert_array_equal(getattr(out, k).cpu().numpy(), ref[k], err_msg=k)
+
+
+def test_ring_tables_in_flight_stay_apart(device):
+    """Several sources' tables are under way behind a busy stream: each bundle
+    is the one that the source gives alone."""
+    sources = [(S.PointSource(z=0.0, semi_conv=1e-3 * (k + 1)), n) for k, n in enumerate((3000, 50, 3000, 7, 20000))]
+    alone = []
+    for src, n in sources:
+        alone.append(src.make_rays(n, device=device))
+        torch.cuda.synchronize()
+    a = torch.ones(4096, 4096, device=device)
+    for _ in range(20):
+        a = (a @ a).clamp_(0, 1)
+    behind = [src.make_rays(n, device=device) for src, n in sources]
+    torch.cuda.synchronize()
+    for x, y in zip(alone, behind):
+        assert torch.equal(x.dx, y.dx) and torch.equal(x.dy, y.dy)
