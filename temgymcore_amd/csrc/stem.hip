@@ -676,18 +676,19 @@ constexpr int kPerLane = 8;
 constexpr int64_t kTile = (int64_t)kThreads * kPerLane;
 
 // Tile `it` (camera c = it / ntile, tile it % ntile) of scan position s:
-// kPerLane float4 per lane, lane-strided so each load instruction of a
+// N float4 per lane, lane-strided so each load instruction of a
 // wavefront covers 1 KiB of contiguous targets.  Streamed once: non-temporal.
 // Indices past the row's end are clamped to its last float4 (the tile sums
 // skip those pairs), so every load is issued unpredicated: predicated loads
 // made the compiler wait for all outstanding loads before the first use.
+template <int N>
 __device__ __forceinline__ void load_tile(const f4* __restrict__ T4, int64_t S, int64_t s, int64_t npair,
-                                          int64_t ntile, int64_t it, f4 (&dst)[kPerLane]) {
+                                          int64_t ntile, int64_t it, f4 (&dst)[N]) {
   const int64_t c = it / ntile, tile = it - c * ntile;
   const int64_t row = (c * S + s) * npair;
   const int64_t q0 = tile * kTile + threadIdx.x;
 #pragma unroll
-  for (int k = 0; k < kPerLane; ++k) {
+  for (int k = 0; k < N; ++k) {
     const int64_t q = q0 + (int64_t)k * kThreads;
     dst[k] = __builtin_nontemporal_load(T4 + row + (q < npair ? q : npair - 1));
   }
@@ -701,65 +702,87 @@ __device__ __forceinline__ void load_tile(const f4* __restrict__ T4, int64_t S, 
 // is linear in the moments with coefficients affine in the camera length
 // L_c, so entries 0..17 need only the camera sums of the x and y residual
 // totals, plain and L-weighted; entry 18 + c takes camera c alone and the
-// last entry sums |r|^2.
+// last entry sums |r|^2.  In two parts, so that the coefficients of thread t
+// can be made while the targets are on their way.
+struct FitCoef {
+  double x, xl, y, yl;
+};
+
+__device__ __forceinline__ FitCoef fit_coef(const tg_stem_geometry& G, const double* __restrict__ P, const ScanPos& p,
+                                            int64_t s, int t) {
+  const int np = 18 + G.n_cam + 1;
+  const double* A = P;
+  FitCoef f = {0.0, 0.0, 0.0, 0.0};
+  if (t >= np - 1) return f;
+  if (t >= 18) {
+    f.x = row_dot(A, 2, p) + G.offsets[2];  // dbx / dL
+    f.y = row_dot(A, 3, p) + G.offsets[3];  // dby / dL
+  } else if (t < 16) {
+    // d/dA[r][k] of sum_c |r_c|^2: rows 0, 1 act on the offsets (x, y),
+    // rows 2, 3 on the slopes (scaled by L_c); column k picks v[k]
+    const int k = t & 3;
+    f.x = 2.0 * (k == 0 ? p.spx : k == 1 ? p.spy : k == 2 ? p.stx : p.sty);
+  } else {
+    // d(Bx, By) / d(spx, spy) = a + b L_c, with st = pivot * sp
+    const double d = G.defocus, kap = G.pivot;
+    const double ax_x = kap * d + (A[0] + A[2] * kap), bx_x = A[8] + A[10] * kap;
+    const double ax_y = A[1] + A[3] * kap, bx_y = A[9] + A[11] * kap;
+    const double ay_x = A[4] + A[6] * kap, by_x = A[12] + A[14] * kap;
+    const double ay_y = kap * d + (A[5] + A[7] * kap), by_y = A[13] + A[15] * kap;
+    double dsx, dsy;
+    if (t == 16) {
+      // step: sp = step * (rotated integer pixel offsets), so d sp / d step
+      // is the offsets themselves (finite at step = 0, where sp / step is 0/0)
+      const int64_t i = s / G.scan_w, j = s % G.scan_w;
+      const double u1 = (double)i - 0.5 * (G.scan_h - 1);
+      const double v1 = (double)j - 0.5 * (G.scan_w - 1);
+      double sn, cs;
+      sincos(P[17] * (kPi / 180.0), &sn, &cs);
+      dsx = -sn * u1 + cs * v1;
+      dsy = -(cs * u1 + sn * v1);
+    } else {        // rotation in degrees: d sp_x = sp_y dphi, d sp_y = -sp_x dphi
+      dsx = p.spy * (kPi / 180.0);
+      dsy = -p.spx * (kPi / 180.0);
+    }
+    f.x = ax_x * dsx + ax_y * dsy;
+    f.xl = bx_x * dsx + bx_y * dsy;
+    f.y = ay_x * dsx + ay_y * dsy;
+    f.yl = by_x * dsx + by_y * dsy;
+  }
+  return f;
+}
+
+// Entry t of a scan position from its moments M [n_cam][kMom].
+__device__ __forceinline__ double fit_value(const tg_stem_geometry& G, const double* __restrict__ P, const FitCoef& f,
+                                            const double* M, int t) {
+  const double* L = P + 18;
+  double g = 0.0;
+  if (t == 18 + G.n_cam) {
+    for (int c = 0; c < G.n_cam; ++c) g += M[c * kMom + 6];
+  } else if (t >= 18) {
+    const double* m = M + (t - 18) * kMom;
+    g = 2.0 * (m[1] + f.x * m[0] + m[5] + f.y * m[3]);
+  } else {
+    double sx = 0.0, sxl = 0.0, sy = 0.0, syl = 0.0;
+    for (int c = 0; c < G.n_cam; ++c) {
+      sx += M[c * kMom];
+      sxl += L[c] * M[c * kMom];
+      sy += M[c * kMom + 3];
+      syl += L[c] * M[c * kMom + 3];
+    }
+    const int r = t >> 2;
+    g = t < 16 ? f.x * (r == 0 ? sx : r == 1 ? sy : r == 2 ? sxl : syl)
+               : 2.0 * (f.x * sx + f.xl * sxl + f.y * sy + f.yl * syl);
+  }
+  return g;
+}
+
 __device__ __forceinline__ void fit_epilogue(const tg_stem_geometry& G, const double* __restrict__ P,
                                              const ScanPos& p, const double (&M)[TG_STEM_MAX_CAM][kMom], int64_t s,
                                              int64_t S, double* __restrict__ partials) {
   const int np = 18 + G.n_cam + 1;
   const int t = threadIdx.x;
-  if (t >= np) return;
-  const double* A = P;
-  const double* L = P + 18;
-  double g = 0.0;
-  if (t == np - 1) {
-    for (int c = 0; c < G.n_cam; ++c) g += M[c][6];
-  } else if (t >= 18) {
-    const int c = t - 18;
-    const double dbx_dl = row_dot(A, 2, p) + G.offsets[2];
-    const double dby_dl = row_dot(A, 3, p) + G.offsets[3];
-    g = 2.0 * (M[c][1] + dbx_dl * M[c][0] + M[c][5] + dby_dl * M[c][3]);
-  } else {
-    double sx = 0.0, sxl = 0.0, sy = 0.0, syl = 0.0;
-    for (int c = 0; c < G.n_cam; ++c) {
-      sx += M[c][0];
-      sxl += L[c] * M[c][0];
-      sy += M[c][3];
-      syl += L[c] * M[c][3];
-    }
-    if (t < 16) {
-      // d/dA[r][k] of sum_c |r_c|^2: rows 0, 1 act on the offsets (x, y),
-      // rows 2, 3 on the slopes (scaled by L_c); column k picks v[k]
-      const int r = t >> 2, k = t & 3;
-      const double vk = k == 0 ? p.spx : k == 1 ? p.spy : k == 2 ? p.stx : p.sty;
-      const double m = r == 0 ? sx : r == 1 ? sy : r == 2 ? sxl : syl;
-      g = 2.0 * vk * m;
-    } else {
-      // d(Bx, By) / d(spx, spy) = a + b L_c, with st = pivot * sp
-      const double d = G.defocus, kap = G.pivot;
-      const double ax_x = kap * d + (A[0] + A[2] * kap), bx_x = A[8] + A[10] * kap;
-      const double ax_y = A[1] + A[3] * kap, bx_y = A[9] + A[11] * kap;
-      const double ay_x = A[4] + A[6] * kap, by_x = A[12] + A[14] * kap;
-      const double ay_y = kap * d + (A[5] + A[7] * kap), by_y = A[13] + A[15] * kap;
-      double dsx, dsy;
-      if (t == 16) {
-        // step: sp = step * (rotated integer pixel offsets), so d sp / d step
-        // is the offsets themselves (finite at step = 0, where sp / step is 0/0)
-        const int64_t i = s / G.scan_w, j = s % G.scan_w;
-        const double u1 = (double)i - 0.5 * (G.scan_h - 1);
-        const double v1 = (double)j - 0.5 * (G.scan_w - 1);
-        double sn, cs;
-        sincos(P[17] * (kPi / 180.0), &sn, &cs);
-        dsx = -sn * u1 + cs * v1;
-        dsy = -(cs * u1 + sn * v1);
-      } else {        // rotation in degrees: d sp_x = sp_y dphi, d sp_y = -sp_x dphi
-        dsx = p.spy * (kPi / 180.0);
-        dsy = -p.spx * (kPi / 180.0);
-      }
-      g = 2.0 * ((ax_x * dsx + ax_y * dsy) * sx + (bx_x * dsx + bx_y * dsy) * sxl + (ay_x * dsx + ay_y * dsy) * sy +
-                 (by_x * dsx + by_y * dsy) * syl);
-    }
-  }
-  partials[s * np + t] = g;
+  if (t < np) partials[s * np + t] = fit_value(G, P, fit_coef(G, P, p, s, t), M[0], t);
 }
 
 // Camera-length constants of the residual r = th a + b - t as double-float
@@ -786,10 +809,12 @@ __device__ __forceinline__ CamConst cam_const(const tg_stem_geometry& G, const d
   return k;
 }
 
-// Adds one tile's residual moments to m[7] (per lane, FP32).
+// Adds the residual moments of one tile's first N pairs a lane to m[7] (per
+// lane, FP32).
+template <int N>
 __device__ __forceinline__ void accumulate_tile(const tg_stem_geometry& G, const float* __restrict__ th,
-                                                const CamConst& K, const f4 (&cur)[kPerLane], int64_t tile,
-                                                int64_t npair, float (&m)[kMom]) {
+                                                const CamConst& K, const f4 (&cur)[N], int64_t tile, int64_t npair,
+                                                float (&m)[kMom]) {
   const int half = G.n_side >> 1, drow = kThreads / half, dcol = kThreads % half;
   // ray pair q = (row iy, columns 2*hc, 2*hc+1); stepped without division
   const int64_t q0 = tile * kTile + threadIdx.x;
@@ -799,13 +824,13 @@ __device__ __forceinline__ void accumulate_tile(const tg_stem_geometry& G, const
     // two columns are fixed, rows advance by drow per pair
     const float tx0 = th[2 * hc], tx1 = th[2 * hc + 1];
 #pragma unroll
-    for (int k = 0; k < kPerLane; ++k) {
-      const f4 t = cur[k];
+    for (int k = 0; k < N; ++k) {
+      const f4 g = cur[k];
       const float ty = th[iy + k * drow];
-      const float rx0 = (fmaf(tx0, K.a_hi, -t.x) + K.bx_hi) + fmaf(tx0, K.a_lo, K.bx_lo);
-      const float ry0 = (fmaf(ty, K.a_hi, -t.y) + K.by_hi) + fmaf(ty, K.a_lo, K.by_lo);
-      const float rx1 = (fmaf(tx1, K.a_hi, -t.z) + K.bx_hi) + fmaf(tx1, K.a_lo, K.bx_lo);
-      const float ry1 = (fmaf(ty, K.a_hi, -t.w) + K.by_hi) + fmaf(ty, K.a_lo, K.by_lo);
+      const float rx0 = (fmaf(tx0, K.a_hi, -g.x) + K.bx_hi) + fmaf(tx0, K.a_lo, K.bx_lo);
+      const float ry0 = (fmaf(ty, K.a_hi, -g.y) + K.by_hi) + fmaf(ty, K.a_lo, K.by_lo);
+      const float rx1 = (fmaf(tx1, K.a_hi, -g.z) + K.bx_hi) + fmaf(tx1, K.a_lo, K.bx_lo);
+      const float ry1 = (fmaf(ty, K.a_hi, -g.w) + K.by_hi) + fmaf(ty, K.a_lo, K.by_lo);
       m[0] += rx0 + rx1;
       m[1] = fmaf(rx0, tx0, fmaf(rx1, tx1, m[1]));
       m[2] = fmaf(rx0 + rx1, ty, m[2]);
@@ -817,14 +842,14 @@ __device__ __forceinline__ void accumulate_tile(const tg_stem_geometry& G, const
     return;
   }
 #pragma unroll
-  for (int k = 0; k < kPerLane; ++k) {
+  for (int k = 0; k < N; ++k) {
     if (q0 + (int64_t)k * kThreads < npair) {
-      const f4 t = cur[k];
+      const f4 g = cur[k];
       const float tx0 = th[2 * hc], tx1 = th[2 * hc + 1], ty = th[iy];
-      const float rx0 = (fmaf(tx0, K.a_hi, -t.x) + K.bx_hi) + fmaf(tx0, K.a_lo, K.bx_lo);
-      const float ry0 = (fmaf(ty, K.a_hi, -t.y) + K.by_hi) + fmaf(ty, K.a_lo, K.by_lo);
-      const float rx1 = (fmaf(tx1, K.a_hi, -t.z) + K.bx_hi) + fmaf(tx1, K.a_lo, K.bx_lo);
-      const float ry1 = (fmaf(ty, K.a_hi, -t.w) + K.by_hi) + fmaf(ty, K.a_lo, K.by_lo);
+      const float rx0 = (fmaf(tx0, K.a_hi, -g.x) + K.bx_hi) + fmaf(tx0, K.a_lo, K.bx_lo);
+      const float ry0 = (fmaf(ty, K.a_hi, -g.y) + K.by_hi) + fmaf(ty, K.a_lo, K.by_lo);
+      const float rx1 = (fmaf(tx1, K.a_hi, -g.z) + K.bx_hi) + fmaf(tx1, K.a_lo, K.bx_lo);
+      const float ry1 = (fmaf(ty, K.a_hi, -g.w) + K.by_hi) + fmaf(ty, K.a_lo, K.by_lo);
       m[0] += rx0 + rx1;
       m[1] = fmaf(rx0, tx0, fmaf(rx1, tx1, m[1]));
       m[2] = fmaf(rx0 + rx1, ty, m[2]);
@@ -908,31 +933,101 @@ __global__ __launch_bounds__(kThreads) void stem_fit_kernel(const tg_stem_geomet
   fit_epilogue(G, sp, p, M, s, S, partials);
 }
 
+// Variant "scan" where one camera's rays are at most four pairs a lane (N): the
+// instructions of the set-up and the sums then bound it, not the targets, so
+// one wavefront sets the position up for all (a lane a camera, the
+// coefficients of the terms beside it), no more loads are issued than the rays
+// need, and the same wavefront makes the terms.  Whole fits, stem_fit_kernel /
+// this one: 64x64 positions, 16^2 rays, 1 camera 30.5 / 22.4 us; 30^2, 3
+// cameras 57.9 / 42.1; 32^2, 8 cameras 119.5 / 89.8; 45x50, 44^2, 8 cameras
+// 82.8 / 61.9.  With eight pairs a lane its registers cost more than the set-up:
+// 46^2, 3 cameras 62.3 / 71.9.
+template <int N>
+__global__ __launch_bounds__(kThreads) void stem_fit_small_kernel(const tg_stem_geometry G,
+                                                                  const double* __restrict__ P,
+                                                                  const float* __restrict__ T,
+                                                                  double* __restrict__ partials) {
+  __shared__ float th[kMaxSide];
+  __shared__ double wm[TG_STEM_MAX_CAM][kWaves][kMom];
+  __shared__ double M[TG_STEM_MAX_CAM][kMom];
+  __shared__ CamConst sk[TG_STEM_MAX_CAM];
+  const int64_t S = (int64_t)G.scan_h * G.scan_w, s = blockIdx.x;
+  const int64_t npair = ((int64_t)G.n_side * G.n_side) >> 1;
+  const f4* __restrict__ T4 = (const f4*)T;
+  f4 cur[N], nxt[N];
+  load_tile(T4, S, s, npair, 1, 0, cur);
+  FitCoef f = {};
+  if (threadIdx.x < 64) {
+    const ScanPos p = scan_position(G, P, s);
+    if (threadIdx.x < G.n_cam) sk[threadIdx.x] = cam_const(G, P, p, threadIdx.x);
+    f = fit_coef(G, P, p, s, threadIdx.x);
+  } else {
+    for (int k = (int)threadIdx.x - 64; k < G.n_side; k += kThreads - 64) th[k] = slope_of(G, k);
+  }
+  __syncthreads();
+  for (int c = 0; c < G.n_cam; ++c) {
+    if (c + 1 < G.n_cam) load_tile(T4, S, s, npair, 1, c + 1, nxt);
+    float m[kMom];
+#pragma unroll
+    for (int k = 0; k < kMom; ++k) m[k] = 0.f;
+    accumulate_tile(G, th, sk[c], cur, 0, npair, m);
+    wave_moments(m, wm[c]);
+#pragma unroll
+    for (int k = 0; k < N; ++k) cur[k] = nxt[k];
+  }
+  __syncthreads();
+  if (threadIdx.x >= 64) return;  // one wavefront from here
+  for (int i = threadIdx.x; i < G.n_cam * kMom; i += 64) {
+    const int c = i / kMom, k = i % kMom;
+    double acc = 0.0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) acc += wm[c][w][k];
+    M[c][k] = acc;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  const int np = 18 + G.n_cam + 1;
+  if (threadIdx.x < np) partials[s * np + threadIdx.x] = fit_value(G, P, f, M[0], threadIdx.x);
+}
+
 // Variant "camera": one workgroup per (scan position, camera length) --
 // n_cam times more, shorter work items, for scans too small to fill the
 // device one workgroup per position.  Each pays the per-workgroup set-up
 // (slopes, scan position, camera constants) without a second tile to
-// overlap it with, so on large scans it is slower than "scan".  Writes the camera's FP64 moments; stem_fit_epilogue
-// finishes each scan position with the same arithmetic as the scan variant.
+// overlap it with, so on large scans it is slower than "scan".  Writes the
+// camera's FP64 moments; stem_fit_sum_kernel (or stem_fit_epilogue) makes the
+// terms of them with the same arithmetic as the scan variant.
+// Bound: latency.  So the targets' loads come first, N of them a lane (as many
+// as the rays need where they are one tile), and one wavefront makes the
+// constants while the others fill the slopes.  With the terms and sums in one
+// launch, whole fits before / now: 13x21 positions, 62^2 rays, 3 cameras 13.7 /
+// 11.7 us; 7x13, 30^2, 3 12.4 / 9.4; 31x33, 30^2, 8 43.5 / 28.9; 5x5, 16^2, 1 11.5
+// / 8.4.
+template <int N>
 __global__ __launch_bounds__(kThreads) void stem_fit_cam_kernel(const tg_stem_geometry G,
                                                                 const double* __restrict__ P,
                                                                 const float* __restrict__ T,
                                                                 double* __restrict__ cam_mom) {
   __shared__ float th[kMaxSide];
   __shared__ double wm[kWaves][kMom];
+  __shared__ CamConst sk;
   const int64_t S = (int64_t)G.scan_h * G.scan_w;
   const int64_t J = (int64_t)G.n_side * G.n_side;
-  fill_slopes(G, th);
-  __syncthreads();
   const int64_t npair = J >> 1;
-  const int64_t ntile = (npair + kTile - 1) / kTile;
+  const int64_t ntile = N < kPerLane ? 1 : (npair + kTile - 1) / kTile;
   const f4* __restrict__ T4 = (const f4*)T;
   const int64_t s = blockIdx.x;
   const int c = blockIdx.y;
-  f4 cur[kPerLane], nxt[kPerLane];
+  f4 cur[N], nxt[N];
   load_tile(T4, S, s, npair, ntile, (int64_t)c * ntile, cur);
-  const ScanPos p = scan_position(G, P, s);
-  const CamConst K = cam_const(G, P, p, c);
+  if (threadIdx.x < 64) {
+    const CamConst k = cam_const(G, P, scan_position(G, P, s), c);
+    if (threadIdx.x == 0) sk = k;
+  } else {
+    for (int k = (int)threadIdx.x - 64; k < G.n_side; k += kThreads - 64) th[k] = slope_of(G, k);
+  }
+  __syncthreads();
+  const CamConst K = sk;
   float m[kMom];
 #pragma unroll
   for (int k = 0; k < kMom; ++k) m[k] = 0.f;
@@ -940,7 +1035,7 @@ __global__ __launch_bounds__(kThreads) void stem_fit_cam_kernel(const tg_stem_ge
     if (tile + 1 < ntile) load_tile(T4, S, s, npair, ntile, (int64_t)c * ntile + tile + 1, nxt);
     accumulate_tile(G, th, K, cur, tile, npair, m);
 #pragma unroll
-    for (int k = 0; k < kPerLane; ++k) cur[k] = nxt[k];
+    for (int k = 0; k < N; ++k) cur[k] = nxt[k];
   }
   wave_moments(m, wm);
   __syncthreads();
@@ -975,9 +1070,21 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
   return v;
 }
 
+// The sum of a block's values, wavefronts in order, into *out.
+__device__ __forceinline__ void block_sum_store(double acc, double* __restrict__ out) {
+  __shared__ double red[kSumThreads / 64];
+  acc = wave_sum_f64(acc);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    double v = threadIdx.x < kSumThreads / 64 ? red[threadIdx.x] : 0.0;
+    v = wave_sum_f64(v);
+    if (threadIdx.x == 0) *out = v;
+  }
+}
+
 __global__ __launch_bounds__(kSumThreads) void row_sum_kernel(const double* __restrict__ partials, int64_t rows,
                                                               int64_t cols, double* __restrict__ out) {
-  __shared__ double red[kSumThreads / 64];
   const double* __restrict__ src = partials + blockIdx.x;  // column blockIdx.x of [rows, cols]
   double acc = 0.0;
   int64_t r = threadIdx.x;
@@ -992,14 +1099,30 @@ __global__ __launch_bounds__(kSumThreads) void row_sum_kernel(const double* __re
     acc += d;
   }
   for (; r < rows; r += kSumThreads) acc += src[r * cols];
-  acc = wave_sum_f64(acc);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
-  __syncthreads();
-  if (threadIdx.x < 64) {
-    double v = threadIdx.x < kSumThreads / 64 ? red[threadIdx.x] : 0.0;
-    v = wave_sum_f64(v);
-    if (threadIdx.x == 0) out[blockIdx.x] = v;
+  block_sum_store(acc, out + blockIdx.x);
+}
+
+// Variant "camera", the terms and their sums in one launch: block t makes entry
+// t of every scan position from the cameras' moments, as stem_fit_epilogue
+// does, keeps them, and sums them in row_sum_kernel's order.  For up to 2,048
+// cameras' moments: each block reads all of them, a position a lane, which for
+// more takes longer than the launch that it saves (whole fits in two launches /
+// in three: 600 positions, 3 cameras 17.7 / 19.1 us; 992, 2 13.8 / 16.0; 440, 8
+// 27.8 / 27.1; 992, 8 52.5 / 47.5).
+__global__ __launch_bounds__(kSumThreads) void stem_fit_sum_kernel(const tg_stem_geometry G,
+                                                                   const double* __restrict__ P,
+                                                                   const double* __restrict__ cam_mom,
+                                                                   double* __restrict__ partials,
+                                                                   double* __restrict__ out) {
+  const int64_t S = (int64_t)G.scan_h * G.scan_w;
+  const int t = blockIdx.x, np = gridDim.x;
+  double acc = 0.0;
+  for (int64_t s = threadIdx.x; s < S; s += kSumThreads) {
+    const double v = fit_value(G, P, fit_coef(G, P, scan_position(G, P, s), s, t), cam_mom + s * G.n_cam * kMom, t);
+    partials[s * np + t] = v;
+    acc += v;
   }
+  block_sum_store(acc, out + t);
 }
 
 int validate(const tg_stem_geometry* g, const double* params) {
@@ -1091,35 +1214,60 @@ extern "C" int64_t tg_stem_fit_workspace(const tg_stem_geometry* g) {
 
 namespace {
 
-// The per-scan-position terms [S, np] at the head of the workspace (the
-// launches of tg_stem_fit before its final reduction).
-int fit_terms(const tg_stem_geometry* g, const double* params, const float* targets, double* workspace,
-              hipStream_t stream) {
+// The first launch of a fit: the per-scan-position terms [S, np] at the head of
+// the workspace (variant "scan"), or the cameras' moments behind them.
+int fit_first(const tg_stem_geometry* g, const double* params, const float* targets, double* workspace,
+              hipStream_t stream, int32_t& variant) {
   TG_REQUIRE(targets != nullptr && workspace != nullptr, "tg_stem_fit: NULL buffer");
   TG_REQUIRE(((uintptr_t)targets & 15) == 0, "tg_stem_fit: targets must be 16-byte aligned");
   const int64_t S = (int64_t)g->scan_h * g->scan_w;
   const int np = 18 + g->n_cam + 1;
-  double* partials = workspace;                   // [S, np]
-  double* cam_mom = workspace + (int64_t)np * S;  // [S, n_cam, 7]
   // launch variant: the autotuner's choice, else one workgroup per scan
   // position when that gives every CU several workgroups, and one per (scan
   // position, camera length) for small scans
   const int64_t key[4] = {S, (int64_t)g->n_side * g->n_side, g->n_cam, 0};
-  int32_t variant = S >= 4LL * tg::cu_count() ? TG_STEM_FIT_SCAN : TG_STEM_FIT_CAMERA;
+  variant = S >= 4LL * tg::cu_count() ? TG_STEM_FIT_SCAN : TG_STEM_FIT_CAMERA;
   int32_t tuned = 0;
   if (tg::tune_lookup(TG_TUNE_STEM_FIT, key, tuned)) variant = tuned;
+  const int64_t npair = ((int64_t)g->n_side * g->n_side) >> 1;
   if (variant == TG_STEM_FIT_SCAN) {
-    hipLaunchKernelGGL(stem_fit_kernel, dim3((unsigned)S), dim3(kThreads), 0, (hipStream_t)stream, *g, params,
-                       targets, partials);
+    auto* kernel = npair <= 2 * kThreads   ? stem_fit_small_kernel<2>
+                   : npair <= 4 * kThreads ? stem_fit_small_kernel<4>
+                                           : stem_fit_kernel;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)S), dim3(kThreads), 0, stream, *g, params, targets, workspace);
     TG_LAUNCH_CHECK("stem_fit_kernel launch");
   } else {
-    hipLaunchKernelGGL(stem_fit_cam_kernel, dim3((unsigned)S, (unsigned)g->n_cam), dim3(kThreads), 0,
-                       (hipStream_t)stream, *g, params, targets, cam_mom);
+    auto* kernel = npair <= 2 * kThreads   ? stem_fit_cam_kernel<2>
+                   : npair <= 4 * kThreads ? stem_fit_cam_kernel<4>
+                                           : stem_fit_cam_kernel<kPerLane>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)S, (unsigned)g->n_cam), dim3(kThreads), 0, stream, *g, params, targets,
+                       workspace + (int64_t)np * S);
     TG_LAUNCH_CHECK("stem_fit_cam_kernel launch");
-    hipLaunchKernelGGL(stem_fit_epilogue, dim3((unsigned)S), dim3(64), 0, (hipStream_t)stream, *g, params, cam_mom,
-                       partials);
+  }
+  return TG_OK;
+}
+
+// tg_stem_fit with checked arguments
+int fit_run(const tg_stem_geometry* g, const double* params, const float* targets, double* workspace, double* out,
+            hipStream_t stream) {
+  int32_t variant = 0;
+  const int st = fit_first(g, params, targets, workspace, stream, variant);
+  if (st != TG_OK) return st;
+  const int64_t S = (int64_t)g->scan_h * g->scan_w;
+  const int np = 18 + g->n_cam + 1;
+  double* cam_mom = workspace + (int64_t)np * S;  // [S, n_cam, 7]
+  if (variant != TG_STEM_FIT_SCAN && S * g->n_cam <= 2 * kSumThreads && S <= kSumThreads) {
+    hipLaunchKernelGGL(stem_fit_sum_kernel, dim3((unsigned)np), dim3(kSumThreads), 0, stream, *g, params, cam_mom,
+                       workspace, out);
+    TG_LAUNCH_CHECK("stem_fit_sum_kernel launch");
+    return TG_OK;
+  }
+  if (variant != TG_STEM_FIT_SCAN) {
+    hipLaunchKernelGGL(stem_fit_epilogue, dim3((unsigned)S), dim3(64), 0, stream, *g, params, cam_mom, workspace);
     TG_LAUNCH_CHECK("stem_fit_epilogue launch");
   }
+  hipLaunchKernelGGL(row_sum_kernel, dim3((unsigned)np), dim3(kSumThreads), 0, stream, workspace, S, (int64_t)np, out);
+  TG_LAUNCH_CHECK("row_sum_kernel launch");
   return TG_OK;
 }
 
@@ -1130,7 +1278,14 @@ extern "C" int tg_stem_fit_terms(const tg_stem_geometry* g, const double* params
   tg::clear_error();
   int st = validate(g, params);
   if (st != TG_OK) return st;
-  return fit_terms(g, params, targets, workspace, (hipStream_t)stream);
+  int32_t variant = 0;
+  st = fit_first(g, params, targets, workspace, (hipStream_t)stream, variant);
+  if (st != TG_OK || variant == TG_STEM_FIT_SCAN) return st;
+  const int64_t S = (int64_t)g->scan_h * g->scan_w;
+  hipLaunchKernelGGL(stem_fit_epilogue, dim3((unsigned)S), dim3(64), 0, (hipStream_t)stream, *g, params,
+                     workspace + (18 + g->n_cam + 1) * S, workspace);
+  TG_LAUNCH_CHECK("stem_fit_epilogue launch");
+  return TG_OK;
 }
 
 extern "C" int tg_stem_fit(const tg_stem_geometry* g, const double* params, const float* targets, double* workspace,
@@ -1139,14 +1294,7 @@ extern "C" int tg_stem_fit(const tg_stem_geometry* g, const double* params, cons
   int st = validate(g, params);
   if (st != TG_OK) return st;
   TG_REQUIRE(out != nullptr, "tg_stem_fit: NULL buffer");
-  st = fit_terms(g, params, targets, workspace, (hipStream_t)stream);
-  if (st != TG_OK) return st;
-  const int64_t S = (int64_t)g->scan_h * g->scan_w;
-  const int np = 18 + g->n_cam + 1;
-  hipLaunchKernelGGL(row_sum_kernel, dim3((unsigned)np), dim3(kSumThreads), 0, (hipStream_t)stream, workspace, S,
-                     (int64_t)np, out);
-  TG_LAUNCH_CHECK("row_sum_kernel launch");
-  return TG_OK;
+  return fit_run(g, params, targets, workspace, out, (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1211,12 +1359,5 @@ extern "C" int tg_stem_fit_noalloc(const tg_stem_geometry* g, const double* para
   if (st != TG_OK) return st;
   // every word of the workspace a launch reads is written earlier in the same
   // call (per-position rows, per-camera moments): nothing needs clearing
-  st = fit_terms(g, params, targets, ws, (hipStream_t)stream);
-  if (st != TG_OK) return st;
-  const int64_t S = (int64_t)g->scan_h * g->scan_w;
-  const int np = 18 + g->n_cam + 1;
-  hipLaunchKernelGGL(row_sum_kernel, dim3((unsigned)np), dim3(kSumThreads), 0, (hipStream_t)stream, ws, S,
-                     (int64_t)np, out);
-  TG_LAUNCH_CHECK("row_sum_kernel launch");
-  return TG_OK;
+  return fit_run(g, params, targets, ws, out, (hipStream_t)stream);
 }
