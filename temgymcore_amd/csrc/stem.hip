@@ -19,6 +19,7 @@
 // Per-scan-position gradient rows go to a workspace that a second kernel sums
 // in a fixed order (deterministic FP64 result).
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 
 #include "tg_common.hpp"
@@ -151,12 +152,53 @@ __device__ __forceinline__ float sample_value(const tg_stem_geometry& G, const f
   return bilinear_tiled(G, img, tile, oy, ox, fy, fx);
 }
 
+// What all rays of a scan position share: the sample map, the origin of the
+// tile x tile image (accumulator) tile around the footprint centre, and the
+// constants of some camera lengths.
+struct PositionSetup {
+  SampleMap smap;
+  float a[TG_STEM_MAX_CAM], bx[TG_STEM_MAX_CAM], by[TG_STEM_MAX_CAM];
+  int oy, ox;
+};
+
+// By one wavefront for its workgroup, a lane a camera length (cam0 ..
+// cam0 + n_cam - 1): about 600 instructions, f64 for the most part, that cost
+// the other wavefronts as much again each when all made them.  Whole calls, all /
+// one: forward of 5x5 positions, 16^2 rays 12.7 / 10.0 us, 64x64 positions, 16^2
+// rays, 3 cameras 17.3 / 14.7; back-projection of 64x64 positions, 64^2 rays
+// 72.4 / 69.5.
+template <int TILE>
+__device__ __forceinline__ void position_setup(const tg_stem_geometry& G, const double* __restrict__ P, int64_t s,
+                                               int cam0, int n_cam, PositionSetup& out) {
+  const int lane = threadIdx.x & 63;
+  const double L = P[18 + cam0 + min(lane, n_cam - 1)];
+  const ScanPos p = scan_position(G, P, s);
+  const SampleMap m = sample_map(G, p);
+  double bx, by;
+  offsets_at(G, P, p, L, bx, by);
+  if (lane < n_cam) {
+    out.a[lane] = (float)(G.defocus + L);
+    out.bx[lane] = (float)bx;
+    out.by[lane] = (float)by;
+  }
+  if (lane == 0) {
+    out.smap = m;
+    // (origins far outside the image only send every lookup to global memory)
+    out.oy = (int)fmin(fmax(floor(m.fy0) - TILE / 2, -4.0 * TILE), (double)G.img_h + 4.0 * TILE);
+    out.ox = (int)fmin(fmax(floor(m.fx0) - TILE / 2, -4.0 * TILE), (double)G.img_w + 4.0 * TILE);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // forward
 // ---------------------------------------------------------------------------
 // rays per lane: a workgroup covers 4096 rays (one scan position of the
 // 64x64 workload), so its set-up (slopes, scan position, camera offsets)
-// is paid once per 4096 rays rather than per 1024
+// is paid once per 4096 rays rather than per 1024.  Bound: HBM writes, 8 B a
+// ray and camera length and 4 B a value: 16.7M rays 34 us into memory written
+// just before (37.7 with a ray a lane and 8- and 4-byte stores), 41 us a call
+// in a row (29 at a fill's rate: the workgroups' outputs lie 32 KB apart.
+// Workgroups of 512 and 1,024 threads, closer together, took 38 and 49 us.)
 constexpr int kFwdRays = 16;
 
 __global__ __launch_bounds__(kThreads) void stem_forward_kernel(const tg_stem_geometry G, const double* __restrict__ P,
@@ -164,22 +206,20 @@ __global__ __launch_bounds__(kThreads) void stem_forward_kernel(const tg_stem_ge
                                                                 float* __restrict__ coords,
                                                                 float* __restrict__ values,
                                                                 float* __restrict__ image4d) {
-  __shared__ float th[kMaxSide];
-  __shared__ float sh_a[TG_STEM_MAX_CAM], sh_bx[TG_STEM_MAX_CAM], sh_by[TG_STEM_MAX_CAM];
+  __shared__ __align__(8) float th[kMaxSide];
+  __shared__ PositionSetup sh;
   __shared__ float tile[kImgTile * kImgTile];
   const int64_t s = blockIdx.y;
   const int64_t S = (int64_t)G.scan_h * G.scan_w;
   const int64_t J = (int64_t)G.n_side * G.n_side;
-  for (int k = threadIdx.x; k < G.n_side; k += kThreads) th[k] = slope_of(G, k);
-  const ScanPos p = scan_position(G, P, s);
-  const SampleMap smap = sample_map(G, p);
-  // the image tile around the footprint centre (origins far outside the
-  // image only send every lookup to global memory)
-  const int oy = (int)fmin(fmax(floor(smap.fy0) - kImgTile / 2, -4.0 * kImgTile), (double)G.img_h + 4.0 * kImgTile);
-  const int ox = (int)fmin(fmax(floor(smap.fx0) - kImgTile / 2, -4.0 * kImgTile), (double)G.img_w + 4.0 * kImgTile);
-  // camera length of this thread's camera constants, loaded before the tile
-  // so that both arrive in one round trip
-  const double Lc = P[18 + min((int)threadIdx.x, G.n_cam - 1)];
+  if (threadIdx.x < 64) {
+    position_setup<kImgTile>(G, P, s, 0, G.n_cam, sh);
+  } else {
+    for (int k = (int)threadIdx.x - 64; k < G.n_side; k += kThreads - 64) th[k] = slope_of(G, k);
+  }
+  __syncthreads();
+  const SampleMap smap = sh.smap;
+  const int oy = sh.oy, ox = sh.ox;
   if (img != nullptr) {
     // all of a thread's tile loads are issued before the first is used
     // (clamped indices, unpredicated; pixels outside the image become 0):
@@ -200,13 +240,6 @@ __global__ __launch_bounds__(kThreads) void stem_forward_kernel(const tg_stem_ge
       tile[k] = (yy >= 0 && yy < G.img_h && xx >= 0 && xx < G.img_w) ? tv[i] : 0.0f;
     }
   }
-  if (threadIdx.x < G.n_cam) {
-    double bx, by;
-    offsets_at(G, P, p, Lc, bx, by);
-    sh_a[threadIdx.x] = (float)(G.defocus + Lc);
-    sh_bx[threadIdx.x] = (float)bx;
-    sh_by[threadIdx.x] = (float)by;
-  }
   __syncthreads();
   // the tile lies inside the image: lookups whose neighbours are all in the
   // tile need no image-bounds tests
@@ -216,40 +249,64 @@ __global__ __launch_bounds__(kThreads) void stem_forward_kernel(const tg_stem_ge
   float* __restrict__ vrow = values != nullptr ? values + s * J : nullptr;
   float2* __restrict__ crow = coords != nullptr ? (float2*)coords + s * J : nullptr;
   const int64_t cstride = S * J;  // between camera lengths, in float2
-  // ray j = (row iy, column ix), stepped by kThreads without dividing
-  const int n = G.n_side, drow = kThreads / n, dcol = kThreads % n;
-  const int j0 = jb + (int)threadIdx.x;
+  // Rays j, j + 1 = (row iy, columns ix, ix + 1; n_side is even), stepped by
+  // 2 kThreads without dividing.  Two a lane, so that they are stored together
+  // where the outputs are aligned for it.
+  const int n = G.n_side, drow = 2 * kThreads / n, dcol = 2 * kThreads % n;
+  const int j0 = jb + 2 * (int)threadIdx.x;
   int iy = j0 / n, ix = j0 - (j0 / n) * n;
   const bool need_v = values != nullptr || image4d != nullptr;
-#pragma unroll 4
-  for (int u = 0; u < kFwdRays; ++u, ix += dcol, iy += drow) {
+  const bool wide_c = ((uintptr_t)coords & 15) == 0, wide_v = ((uintptr_t)values & 7) == 0;
+#pragma unroll 2
+  for (int u = 0; u < kFwdRays / 2; ++u, ix += dcol, iy += drow) {
     if (ix >= n) {
       ix -= n;
       ++iy;
     }
-    const int j = j0 + u * kThreads;
+    const int j = j0 + u * 2 * kThreads;
     if (j >= (int)J) continue;
-    const float tx = th[ix], ty = th[iy];
-    float v = 0.0f;
+    const float2 tx = *(const float2*)(th + ix);
+    const float ty = th[iy];
+    float2 v = make_float2(0.0f, 0.0f);
     if (need_v) {
       double fy, fx;
-      sample_pixel(smap, tx, ty, fy, fx);
-      v = sample_value(G, img, tile, oy, ox, tile_inside, fy, fx);
-      if (vrow != nullptr) vrow[j] = v;
+      sample_pixel(smap, tx.x, ty, fy, fx);
+      v.x = sample_value(G, img, tile, oy, ox, tile_inside, fy, fx);
+      sample_pixel(smap, tx.y, ty, fy, fx);
+      v.y = sample_value(G, img, tile, oy, ox, tile_inside, fy, fx);
+      if (vrow != nullptr) {
+        if (wide_v) {
+          *(float2*)(vrow + j) = v;
+        } else {
+          vrow[j] = v.x;
+          vrow[j + 1] = v.y;
+        }
+      }
     }
     float2* __restrict__ co = crow;
     for (int c = 0; c < G.n_cam; ++c, co += cstride) {
-      const float xd = fmaf(tx, sh_a[c], sh_bx[c]);
-      const float yd = fmaf(ty, sh_a[c], sh_by[c]);
-      if (co != nullptr) co[j] = make_float2(xd, yd);
+      const float2 xd = make_float2(fmaf(tx.x, sh.a[c], sh.bx[c]), fmaf(tx.y, sh.a[c], sh.bx[c]));
+      const float yd = fmaf(ty, sh.a[c], sh.by[c]);
+      if (co != nullptr) {
+        if (wide_c) {
+          *(f4*)(co + j) = f4{xd.x, yd, xd.y, yd};
+        } else {
+          co[j] = make_float2(xd.x, yd);
+          co[j + 1] = make_float2(xd.y, yd);
+        }
+      }
       if (c == 0 && image4d != nullptr) {
-        const double fy = __dadd_rn(__dadd_rn(__dmul_rn(G.det_m[0], (double)yd), __dmul_rn(G.det_m[1], (double)xd)),
-                                    G.det_m[2]);
-        const double fx = __dadd_rn(__dadd_rn(__dmul_rn(G.det_m[3], (double)yd), __dmul_rn(G.det_m[4], (double)xd)),
-                                    G.det_m[5]);
-        const int32_t py = tg::xla_f64_to_i32(rint(fy)), px = tg::xla_f64_to_i32(rint(fx));
-        if (py >= 0 && py < G.det_h && px >= 0 && px < G.det_w)
-          unsafeAtomicAdd(image4d + (s * G.det_h + py) * G.det_w + px, v);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const float x = k == 0 ? xd.x : xd.y;
+          const double fy = __dadd_rn(__dadd_rn(__dmul_rn(G.det_m[0], (double)yd), __dmul_rn(G.det_m[1], (double)x)),
+                                      G.det_m[2]);
+          const double fx = __dadd_rn(__dadd_rn(__dmul_rn(G.det_m[3], (double)yd), __dmul_rn(G.det_m[4], (double)x)),
+                                      G.det_m[5]);
+          const int32_t py = tg::xla_f64_to_i32(rint(fy)), px = tg::xla_f64_to_i32(rint(fx));
+          if (py >= 0 && py < G.det_h && px >= 0 && px < G.det_w)
+            unsafeAtomicAdd(image4d + (s * G.det_h + py) * G.det_w + px, k == 0 ? v.x : v.y);
+        }
       }
     }
   }
@@ -278,38 +335,21 @@ __global__ __launch_bounds__(kThreads) void stem_forward_kernel(const tg_stem_ge
 // 207-219 us; non-temporal stores 196 us.
 constexpr int kBandFloats = 6144;
 
-struct BandSetup {
-  SampleMap smap;
-  float a, bx, by;
-  int oy, ox;
-};
-
 __global__ __launch_bounds__(kThreads) void stem_dataset_kernel(const tg_stem_geometry G, const double* __restrict__ P,
                                                                 const float* __restrict__ img, int band_rows,
                                                                 int bands_each, float* __restrict__ image4d) {
   __shared__ float th[kMaxSide];
   __shared__ float tile[kImgTile * kImgTile];
   __shared__ __align__(16) float band[kBandFloats + 4];
-  __shared__ BandSetup sh;
+  __shared__ PositionSetup sh;
   __shared__ int sh_lo[2], sh_hi[2];
   const int64_t s = blockIdx.y;
   const int n = G.n_side, W = G.det_w;
   const int row_begin = (int)blockIdx.x * bands_each * band_rows;
   const int row_end = min(row_begin + bands_each * band_rows, G.det_h);
   if (threadIdx.x < 64) {
-    const ScanPos p = scan_position(G, P, s);
-    const double L = P[18];
-    double bx, by;
-    offsets_at(G, P, p, L, bx, by);
-    const SampleMap m = sample_map(G, p);
+    position_setup<kImgTile>(G, P, s, 0, 1, sh);
     if (threadIdx.x == 0) {
-      sh.smap = m;
-      sh.a = (float)(G.defocus + L);
-      sh.bx = (float)bx;
-      sh.by = (float)by;
-      // the image tile around the footprint centre, as in stem_forward_kernel
-      sh.oy = (int)fmin(fmax(floor(m.fy0) - kImgTile / 2, -4.0 * kImgTile), (double)G.img_h + 4.0 * kImgTile);
-      sh.ox = (int)fmin(fmax(floor(m.fx0) - kImgTile / 2, -4.0 * kImgTile), (double)G.img_w + 4.0 * kImgTile);
       sh_lo[0] = n;
       sh_hi[0] = -1;
     }
@@ -317,7 +357,7 @@ __global__ __launch_bounds__(kThreads) void stem_dataset_kernel(const tg_stem_ge
   for (int k = threadIdx.x; k < n; k += kThreads) th[k] = slope_of(G, k);
   for (int k = threadIdx.x; k < kBandFloats / 4 + 1; k += kThreads) ((float4*)band)[k] = make_float4(0.f, 0.f, 0.f, 0.f);
   __syncthreads();
-  const float a = sh.a, bx = sh.bx, by = sh.by;
+  const float a = sh.a[0], bx = sh.bx[0], by = sh.by[0];
   const int oy = sh.oy, ox = sh.ox;
   for (int k = threadIdx.x; k < kImgTile * kImgTile; k += kThreads) {
     const int yy = oy + k / kImgTile, xx = ox + k % kImgTile;
@@ -436,8 +476,72 @@ __device__ __forceinline__ int bp_slot(const tg_stem_geometry& G, int oy, int ox
   return ty_ >= 0 && ty_ < kBpTile && tx_ >= 0 && tx_ < kBpTile ? ty_ * kBpTile + tx_ : kBpGlobal;
 }
 
+// One axis of a block's rays where sample and detector pixels are not rotated
+// against the slopes: the row (column) of each ray of that axis depends on its
+// own slope alone.
+struct BpAxis {
+  uint32_t at[kBpBlock];         // detector row (column), 0 where it is off the detector or past n
+  float w[kBpBlock][3];          // window weights, 0 where the ray is out
+  uint32_t hit, on_img, in_win;  // bit k: ray k lands on the detector, lies on the sample image, in the window
+  int anchor;
+};
+
+// slope: the slopes from index i0; (m, m0): detector coordinate m d + m0 of the
+// position d = slope a + b; (k, f0): sample coordinate k slope + f0.  Roundings
+// as in the general form, whose cross terms are exact zeros.
+__device__ __forceinline__ BpAxis bp_axis(const float* slope, int i0, int n, float a, float b, double m, double m0,
+                                          int det, double k, double f0, int img, bool& finite) {
+  BpAxis o;
+  o.hit = o.on_img = o.in_win = 0;
+  double f[kBpBlock];
+#pragma unroll
+  for (int i = 0; i < kBpBlock; ++i) {
+    const float t = slope[min(i0 + i, n - 1)];
+    const float d = fmaf(t, a, b);
+    finite = finite && d * 0.0f == 0.0f;
+    const int32_t p = tg::xla_f64_to_i32(rint(__dadd_rn(__dmul_rn(m, (double)d), m0)));
+    const bool ok = (i0 + i < n) & ((uint32_t)p < (uint32_t)det);
+    o.at[i] = ok ? (uint32_t)p : 0u;
+    o.hit |= (uint32_t)ok << i;
+    f[i] = fma(k, (double)t, f0);
+  }
+  const double lo = floor(fmin(f[0], f[kBpBlock - 1]));
+  const bool anchored = lo > -4.0 && lo < (double)img + 4.0;
+  o.anchor = anchored ? (int)lo : 0;
+#pragma unroll
+  for (int i = 0; i < kBpBlock; ++i) {
+    const double q = floor(f[i]);
+    const bool on = (q >= -1.0) & (q < (double)img);
+    const float w = (float)(f[i] - q);
+    const int at = (int)(on ? q : 0.0) - o.anchor;
+    const bool win = on & anchored & ((unsigned)at <= 1u);
+    o.on_img |= (uint32_t)on << i;
+    o.in_win |= (uint32_t)win << i;
+    const bool use = win & ((o.hit >> i) & 1u);
+    o.w[i][0] = use & (at == 0) ? 1.0f - w : 0.0f;
+    o.w[i][1] = use ? (at == 0 ? w : 1.0f - w) : 0.0f;
+    o.w[i][2] = use & (at != 0) ? w : 0.0f;
+  }
+  return o;
+}
+
+// bit r kBpBlock + c: bit r of rows and bit c of columns
+__device__ __forceinline__ uint32_t bp_outer(uint32_t rows, uint32_t cols) {
+  uint32_t m = 0;
+#pragma unroll
+  for (int r = 0; r < kBpBlock; ++r) m |= (rows >> r) & 1u ? cols << (r * kBpBlock) : 0u;
+  return m;
+}
+
 // WEIGHT: also accumulate weight[q] (the sum of w_q), else weight is unused.
-template <bool WEIGHT>
+// SEPARABLE: the cross terms of the sample and detector maps are zero, so that
+// rows and columns are binned, looked up and weighted once each: a block's
+// deposits are then sum_r wy_r (sum_c wx_c d_rc), 6 instructions a ray in place
+// of about 110, and its weights (sum_r wy_r) (sum_c wx_c).  Bound: the gathered
+// detector pixels (260 MB of cache lines for 16.7M rays); the general form,
+// vector issue.  64x64 positions: 64^2 rays 67.6 / 49.2 us, 20^2 rays (whole
+// call) 69.9 / 42.9.
+template <bool WEIGHT, bool SEPARABLE>
 __global__ __launch_bounds__(kThreads) void stem_backproject_kernel(const tg_stem_geometry G,
                                                                     const double* __restrict__ P,
                                                                     const float* __restrict__ data, int cam,
@@ -446,155 +550,215 @@ __global__ __launch_bounds__(kThreads) void stem_backproject_kernel(const tg_ste
   __shared__ float th[kMaxSide];
   __shared__ double t_img[kBpTile * kBpTile];
   __shared__ double t_w[WEIGHT ? kBpTile * kBpTile : 1];
-  __shared__ float sh_a, sh_bx, sh_by;
+  __shared__ PositionSetup sh;
   const int64_t s = blockIdx.y;
   const int n = G.n_side;
-  for (int k = threadIdx.x; k < n; k += kThreads) th[k] = slope_of(G, k);
-  for (int k = threadIdx.x; k < kBpTile * kBpTile; k += kThreads) {
-    t_img[k] = 0.0;
-    if (WEIGHT) t_w[k] = 0.0;
+  if (threadIdx.x < 64) {
+    position_setup<kBpTile>(G, P, s, cam, 1, sh);
+  } else {
+    for (int k = (int)threadIdx.x - 64; k < n; k += kThreads - 64) th[k] = slope_of(G, k);
+    for (int k = (int)threadIdx.x - 64; k < kBpTile * kBpTile; k += kThreads - 64) {
+      t_img[k] = 0.0;
+      if (WEIGHT) t_w[k] = 0.0;
+    }
   }
-  const ScanPos p = scan_position(G, P, s);
-  if (threadIdx.x == 0) {
-    const double L = P[18 + cam];
-    double bx, by;
-    offsets_at(G, P, p, L, bx, by);
-    sh_a = (float)(G.defocus + L);
-    sh_bx = (float)bx;
-    sh_by = (float)by;
-  }
-  // tile origin: the footprint centre (zero slope) minus half a tile
-  const SampleMap smap = sample_map(G, p);
-  const double oyd = floor(smap.fy0) - kBpTile / 2, oxd = floor(smap.fx0) - kBpTile / 2;
-  // origins far outside the image only route everything to global memory
-  const int oy = (int)fmin(fmax(oyd, -4.0 * kBpTile), (double)G.img_h + 4.0 * kBpTile);
-  const int ox = (int)fmin(fmax(oxd, -4.0 * kBpTile), (double)G.img_w + 4.0 * kBpTile);
   __syncthreads();
+  const SampleMap smap = sh.smap;
+  const int oy = sh.oy, ox = sh.ox;
+  const float sh_a = sh.a[0], sh_bx = sh.bx[0], sh_by = sh.by[0];
   // this thread's block of rays: rows iy0.., columns ix0.. (clipped to n)
   const int ntx = (n + kBpRayTile - 1) / kBpRayTile;
   const int iy0 = (int)(blockIdx.x / ntx) * kBpRayTile + (int)(threadIdx.x / 16) * kBpBlock;
   const int ix0 = (int)(blockIdx.x % ntx) * kBpRayTile + (int)(threadIdx.x % 16) * kBpBlock;
   if (iy0 < n && ix0 < n) {
-    // The sample position fma(ky_y, ty, fma(ky_x, tx, fy0)) (likewise fx) and
-    // the detector coordinate ((m0 yd) + (m1 xd)) + m2 (likewise fx) take
-    // their inner terms from the ray's column (tx, xd) or row (ty, yd) alone:
-    // computed once per row and column of the block, with the same roundings
-    // as the per-ray expressions of stem_forward_kernel.  Rows and columns
-    // past n repeat the last one (their rays are masked out below).
-    double cy[kBpBlock], cx[kBpBlock], tyd[kBpBlock];
-    double ry0[kBpBlock], ry3[kBpBlock], cx1[kBpBlock], cx4[kBpBlock];
-#pragma unroll
-    for (int k = 0; k < kBpBlock; ++k) {
-      const float tx = th[min(ix0 + k, n - 1)], ty = th[min(iy0 + k, n - 1)];
-      cy[k] = fma(smap.ky_x, (double)tx, smap.fy0);
-      cx[k] = fma(smap.kx_x, (double)tx, smap.fx0);
-      tyd[k] = (double)ty;
-      const float xd = fmaf(tx, sh_a, sh_bx), yd = fmaf(ty, sh_a, sh_by);
-      ry0[k] = __dmul_rn(G.det_m[0], (double)yd);
-      ry3[k] = __dmul_rn(G.det_m[3], (double)yd);
-      cx1[k] = __dmul_rn(G.det_m[1], (double)xd);
-      cx4[k] = __dmul_rn(G.det_m[4], (double)xd);
-    }
-    // window anchor: floor of the smallest sample coordinates over the
-    // block's corners (the position is affine in the slopes)
-    constexpr int L = kBpBlock - 1;
-    const double wy0 = floor(fmin(fmin(fma(smap.ky_y, tyd[0], cy[0]), fma(smap.ky_y, tyd[0], cy[L])),
-                                  fmin(fma(smap.ky_y, tyd[L], cy[0]), fma(smap.ky_y, tyd[L], cy[L]))));
-    const double wx0 = floor(fmin(fmin(fma(smap.kx_y, tyd[0], cx[0]), fma(smap.kx_y, tyd[0], cx[L])),
-                                  fmin(fma(smap.kx_y, tyd[L], cx[0]), fma(smap.kx_y, tyd[L], cx[L]))));
-    // anchors far outside the image: every ray deposits directly (and skips)
-    const bool anchored = wy0 > -4.0 && wy0 < (double)G.img_h + 4.0 && wx0 > -4.0 && wx0 < (double)G.img_w + 4.0;
-    const int Y = anchored ? (int)wy0 : 0, X = anchored ? (int)wx0 : 0;
+    int Y, X;  // window anchor
+    uint32_t direct = 0;  // rays deposited one by one
     double acc[9], accw[WEIGHT ? 9 : 1];
 #pragma unroll
     for (int k = 0; k < 9; ++k) acc[k] = 0.0;
 #pragma unroll
     for (int k = 0; k < (WEIGHT ? 9 : 1); ++k) accw[k] = 0.0;
-    // the block's 16 detector values, all loads issued before the first is
-    // used (the position's first pixel stands in for a ray off the detector
-    // or past n; `hit` says which rays are real): a load per ray behind its
-    // bounds test waited for each in turn.  One scan position's detector
-    // image is addressed by a 32-bit byte offset from a uniform base (the
-    // host bounds det_h * det_w by 2^30).
     const char* __restrict__ dimg = (const char*)(data + s * G.det_h * G.det_w);
-    float dv[kBpBlock * kBpBlock];
-    uint32_t hit = 0;
+    if constexpr (SEPARABLE) {
+      bool finite = true;
+      const BpAxis cols = bp_axis(th, ix0, n, sh_a, sh_bx, G.det_m[4], G.det_m[5], G.det_w, smap.kx_x, smap.fx0,
+                                  G.img_w, finite);
+      const BpAxis rows = bp_axis(th, iy0, n, sh_a, sh_by, G.det_m[0], G.det_m[2], G.det_h, smap.ky_y, smap.fy0,
+                                  G.img_h, finite);
+      Y = rows.anchor;
+      X = cols.anchor;
+      float dv[kBpBlock * kBpBlock];
 #pragma unroll
-    for (int r = 0; r < kBpBlock; ++r) {
+      for (int r = 0; r < kBpBlock; ++r)
 #pragma unroll
-      for (int c = 0; c < kBpBlock; ++c) {
-        const double dfy = __dadd_rn(__dadd_rn(ry0[r], cx1[c]), G.det_m[2]);
-        const double dfx = __dadd_rn(__dadd_rn(ry3[r], cx4[c]), G.det_m[5]);
-        const int32_t py = tg::xla_f64_to_i32(rint(dfy)), px = tg::xla_f64_to_i32(rint(dfx));
-        // (& rather than &&: one straight-line test, no exec-mask branches)
-        const bool ok = (iy0 + r < n) & (ix0 + c < n) & ((uint32_t)py < (uint32_t)G.det_h) &
-                        ((uint32_t)px < (uint32_t)G.det_w);
-        dv[r * kBpBlock + c] = *(const float*)(dimg + (ok ? (uint32_t)(py * G.det_w + px) << 2 : 0u));
-        hit |= (uint32_t)ok << (r * kBpBlock + c);
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);  // all 16 loads in flight before the deposits
-    // Per ray, straight-line: the window deposit runs for every ray with its
-    // weights and value selected to zero unless the ray is real, on the
-    // image and inside the window.  Rays on the image outside the window
-    // (wide footprints; rare) are marked in `direct` and deposited by the
-    // loop below.  (Conditional blocks in this unrolled loop would let the
-    // compiler sink the gathered loads into them and keep the rays' values
-    // live across them.)
-    uint32_t direct = 0;
+        for (int c = 0; c < kBpBlock; ++c)
+          dv[r * kBpBlock + c] = *(const float*)(dimg + ((rows.at[r] * (uint32_t)G.det_w + cols.at[c]) << 2));
+      __builtin_amdgcn_sched_barrier(0);  // all 16 loads in flight before the deposits
+      if (finite) {
+        const uint32_t use = bp_outer(rows.hit & rows.in_win, cols.hit & cols.in_win);
+        direct = bp_outer(rows.hit & rows.on_img, cols.hit & cols.on_img) & ~use;
+        double rx[kBpBlock][3], sx[3] = {0.0, 0.0, 0.0}, sy[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-    for (int r = 0; r < kBpBlock; ++r) {
+        for (int c = 0; c < kBpBlock; ++c)
 #pragma unroll
-      for (int c = 0; c < kBpBlock; ++c) {
-        const bool real = (hit >> (r * kBpBlock + c)) & 1u;
-        // bilinear weights at the sample-plane position, as in bilinear_tiled()
-        const double fy = fma(smap.ky_y, tyd[r], cy[c]), fx = fma(smap.kx_y, tyd[r], cx[c]);
-        const double y0d = floor(fy), x0d = floor(fx);
-        const bool on_img = (y0d >= -1.0) & (y0d < (double)G.img_h) & (x0d >= -1.0) & (x0d < (double)G.img_w);
-        // (positions off the image, NaN included, convert a stand-in 0)
-        const int y0 = (int)(on_img ? y0d : 0.0), x0 = (int)(on_img ? x0d : 0.0);
-        const float wy = (float)(fy - y0d), wx = (float)(fx - x0d);
-        const int dy = y0 - Y, dx = x0 - X;
-        const bool win = real & on_img & anchored & ((unsigned)dy <= 1u) & ((unsigned)dx <= 1u);
-        direct |= (uint32_t)(real & on_img & !win) << (r * kBpBlock + c);
-        // separable weights placed in the 3 x 3 window: row i of the window
-        // carries (1 - wy) at dy and wy at dy + 1, likewise columns.  rx * d
-        // is exact in FP64 (two 24-bit significands), so each deposit
-        // ry * rx * d is rounded once, by the FMA into the sum.
-        float ry[3] = {win & (dy == 0) ? 1.0f - wy : 0.0f, win ? (dy == 0 ? wy : 1.0f - wy) : 0.0f,
-                       win & (dy != 0) ? wy : 0.0f};
-        float rx[3] = {win & (dx == 0) ? 1.0f - wx : 0.0f, win ? (dx == 0 ? wx : 1.0f - wx) : 0.0f,
-                       win & (dx != 0) ? wx : 0.0f};
-        float df = win ? dv[r * kBpBlock + c] : 0.0f;
-        // (the selects stay in f32: without these empty statements the
-        // compiler converts first and selects both halves of each double)
+          for (int k = 0; k < 3; ++k) sx[k] += rx[c][k] = (double)cols.w[c][k];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) asm volatile("" : "+v"(ry[k]), "+v"(rx[k]));
-        asm volatile("" : "+v"(df));
-        const double d = (double)df;
-        double rxd[3], t[3];
+        for (int r = 0; r < kBpBlock; ++r) {
+          double t[3] = {0.0, 0.0, 0.0};
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          rxd[k] = (double)rx[k];
-          t[k] = rxd[k] * d;
-        }
+          for (int c = 0; c < kBpBlock; ++c) {
+            const double d = (double)((use >> (r * kBpBlock + c)) & 1u ? dv[r * kBpBlock + c] : 0.0f);
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          const double ryd = (double)ry[i];
+            for (int k = 0; k < 3; ++k) t[k] = fma(rx[c][k], d, t[k]);
+          }
 #pragma unroll
-          for (int k = 0; k < 3; ++k) {
-            acc[3 * i + k] = fma(ryd, t[k], acc[3 * i + k]);
-            if (WEIGHT) accw[3 * i + k] = fma(ryd, rxd[k], accw[3 * i + k]);
+          for (int i = 0; i < 3; ++i) {
+            const double ry = (double)rows.w[r][i];
+            sy[i] += ry;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) acc[3 * i + k] = fma(ry, t[k], acc[3 * i + k]);
           }
         }
-        // one ray at a time: instruction selection would otherwise defer
-        // every ray's sums past the last ray's set-up and hold all their
-        // weights live at once.  (The empty statements emit nothing; they
-        // make this ray's sums complete before the next ray's begin.)
+        if (WEIGHT) {
 #pragma unroll
-        for (int k = 0; k < 9; ++k) {
-          asm volatile("" : "+v"(acc[k]));
-          if (WEIGHT) asm volatile("" : "+v"(accw[k]));
+          for (int k = 0; k < 9; ++k) accw[k] = sy[k / 3] * sx[k % 3];
+        }
+      } else {
+        // an infinite or NaN position: the zero cross terms turn its partner's
+        // coordinate into NaN, so every ray by itself
+        for (int k = 0; k < kBpBlock * kBpBlock; ++k) {
+          const int iy = iy0 + k / kBpBlock, ix = ix0 + k % kBpBlock;
+          if (iy >= n || ix >= n) continue;
+          const float xd = fmaf(th[ix], sh_a, sh_bx), yd = fmaf(th[iy], sh_a, sh_by);
+          const double dfy = __dadd_rn(__dadd_rn(__dmul_rn(G.det_m[0], (double)yd), __dmul_rn(G.det_m[1], (double)xd)),
+                                       G.det_m[2]);
+          const double dfx = __dadd_rn(__dadd_rn(__dmul_rn(G.det_m[3], (double)yd), __dmul_rn(G.det_m[4], (double)xd)),
+                                       G.det_m[5]);
+          const int32_t py = tg::xla_f64_to_i32(rint(dfy)), px = tg::xla_f64_to_i32(rint(dfx));
+          double fy, fx;
+          sample_pixel(smap, th[ix], th[iy], fy, fx);
+          const double y0d = floor(fy), x0d = floor(fx);
+          const bool on = ((uint32_t)py < (uint32_t)G.det_h) & ((uint32_t)px < (uint32_t)G.det_w) & (y0d >= -1.0) &
+                          (y0d < (double)G.img_h) & (x0d >= -1.0) & (x0d < (double)G.img_w);
+          direct |= (uint32_t)on << k;
+        }
+      }
+    } else {
+      // The sample position fma(ky_y, ty, fma(ky_x, tx, fy0)) (likewise fx) and
+      // the detector coordinate ((m0 yd) + (m1 xd)) + m2 (likewise fx) take
+      // their inner terms from the ray's column (tx, xd) or row (ty, yd) alone:
+      // computed once per row and column of the block, with the same roundings
+      // as the per-ray expressions of stem_forward_kernel.  Rows and columns
+      // past n repeat the last one (their rays are masked out below).
+      double cy[kBpBlock], cx[kBpBlock], tyd[kBpBlock];
+      double ry0[kBpBlock], ry3[kBpBlock], cx1[kBpBlock], cx4[kBpBlock];
+#pragma unroll
+      for (int k = 0; k < kBpBlock; ++k) {
+        const float tx = th[min(ix0 + k, n - 1)], ty = th[min(iy0 + k, n - 1)];
+        cy[k] = fma(smap.ky_x, (double)tx, smap.fy0);
+        cx[k] = fma(smap.kx_x, (double)tx, smap.fx0);
+        tyd[k] = (double)ty;
+        const float xd = fmaf(tx, sh_a, sh_bx), yd = fmaf(ty, sh_a, sh_by);
+        ry0[k] = __dmul_rn(G.det_m[0], (double)yd);
+        ry3[k] = __dmul_rn(G.det_m[3], (double)yd);
+        cx1[k] = __dmul_rn(G.det_m[1], (double)xd);
+        cx4[k] = __dmul_rn(G.det_m[4], (double)xd);
+      }
+      // window anchor: floor of the smallest sample coordinates over the
+      // block's corners (the position is affine in the slopes)
+      constexpr int L = kBpBlock - 1;
+      const double wy0 = floor(fmin(fmin(fma(smap.ky_y, tyd[0], cy[0]), fma(smap.ky_y, tyd[0], cy[L])),
+                                    fmin(fma(smap.ky_y, tyd[L], cy[0]), fma(smap.ky_y, tyd[L], cy[L]))));
+      const double wx0 = floor(fmin(fmin(fma(smap.kx_y, tyd[0], cx[0]), fma(smap.kx_y, tyd[0], cx[L])),
+                                    fmin(fma(smap.kx_y, tyd[L], cx[0]), fma(smap.kx_y, tyd[L], cx[L]))));
+      // anchors far outside the image: every ray deposits directly (and skips)
+      const bool anchored = wy0 > -4.0 && wy0 < (double)G.img_h + 4.0 && wx0 > -4.0 && wx0 < (double)G.img_w + 4.0;
+      Y = anchored ? (int)wy0 : 0;
+      X = anchored ? (int)wx0 : 0;
+      // the block's 16 detector values, all loads issued before the first is
+      // used (the position's first pixel stands in for a ray off the detector
+      // or past n; `hit` says which rays are real): a load per ray behind its
+      // bounds test waited for each in turn.  One scan position's detector
+      // image is addressed by a 32-bit byte offset from a uniform base (the
+      // host bounds det_h * det_w by 2^30).
+      float dv[kBpBlock * kBpBlock];
+      uint32_t hit = 0;
+#pragma unroll
+      for (int r = 0; r < kBpBlock; ++r) {
+#pragma unroll
+        for (int c = 0; c < kBpBlock; ++c) {
+          const double dfy = __dadd_rn(__dadd_rn(ry0[r], cx1[c]), G.det_m[2]);
+          const double dfx = __dadd_rn(__dadd_rn(ry3[r], cx4[c]), G.det_m[5]);
+          const int32_t py = tg::xla_f64_to_i32(rint(dfy)), px = tg::xla_f64_to_i32(rint(dfx));
+          // (& rather than &&: one straight-line test, no exec-mask branches)
+          const bool ok = (iy0 + r < n) & (ix0 + c < n) & ((uint32_t)py < (uint32_t)G.det_h) &
+                          ((uint32_t)px < (uint32_t)G.det_w);
+          dv[r * kBpBlock + c] = *(const float*)(dimg + (ok ? (uint32_t)(py * G.det_w + px) << 2 : 0u));
+          hit |= (uint32_t)ok << (r * kBpBlock + c);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);  // all 16 loads in flight before the deposits
+      // Per ray, straight-line: the window deposit runs for every ray with its
+      // weights and value selected to zero unless the ray is real, on the
+      // image and inside the window.  Rays on the image outside the window
+      // (wide footprints; rare) are marked in `direct` and deposited by the
+      // loop below.  (Conditional blocks in this unrolled loop would let the
+      // compiler sink the gathered loads into them and keep the rays' values
+      // live across them.)
+#pragma unroll
+      for (int r = 0; r < kBpBlock; ++r) {
+#pragma unroll
+        for (int c = 0; c < kBpBlock; ++c) {
+          const bool real = (hit >> (r * kBpBlock + c)) & 1u;
+          // bilinear weights at the sample-plane position, as in bilinear_tiled()
+          const double fy = fma(smap.ky_y, tyd[r], cy[c]), fx = fma(smap.kx_y, tyd[r], cx[c]);
+          const double y0d = floor(fy), x0d = floor(fx);
+          const bool on_img = (y0d >= -1.0) & (y0d < (double)G.img_h) & (x0d >= -1.0) & (x0d < (double)G.img_w);
+          // (positions off the image, NaN included, convert a stand-in 0)
+          const int y0 = (int)(on_img ? y0d : 0.0), x0 = (int)(on_img ? x0d : 0.0);
+          const float wy = (float)(fy - y0d), wx = (float)(fx - x0d);
+          const int dy = y0 - Y, dx = x0 - X;
+          const bool win = real & on_img & anchored & ((unsigned)dy <= 1u) & ((unsigned)dx <= 1u);
+          direct |= (uint32_t)(real & on_img & !win) << (r * kBpBlock + c);
+          // separable weights placed in the 3 x 3 window: row i of the window
+          // carries (1 - wy) at dy and wy at dy + 1, likewise columns.  rx * d
+          // is exact in FP64 (two 24-bit significands), so each deposit
+          // ry * rx * d is rounded once, by the FMA into the sum.
+          float ry[3] = {win & (dy == 0) ? 1.0f - wy : 0.0f, win ? (dy == 0 ? wy : 1.0f - wy) : 0.0f,
+                         win & (dy != 0) ? wy : 0.0f};
+          float rx[3] = {win & (dx == 0) ? 1.0f - wx : 0.0f, win ? (dx == 0 ? wx : 1.0f - wx) : 0.0f,
+                         win & (dx != 0) ? wx : 0.0f};
+          float df = win ? dv[r * kBpBlock + c] : 0.0f;
+          // (the selects stay in f32: without these empty statements the
+          // compiler converts first and selects both halves of each double)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) asm volatile("" : "+v"(ry[k]), "+v"(rx[k]));
+          asm volatile("" : "+v"(df));
+          const double d = (double)df;
+          double rxd[3], t[3];
+#pragma unroll
+          for (int k = 0; k < 3; ++k) {
+            rxd[k] = (double)rx[k];
+            t[k] = rxd[k] * d;
+          }
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            const double ryd = (double)ry[i];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+              acc[3 * i + k] = fma(ryd, t[k], acc[3 * i + k]);
+              if (WEIGHT) accw[3 * i + k] = fma(ryd, rxd[k], accw[3 * i + k]);
+            }
+          }
+          // one ray at a time: instruction selection would otherwise defer
+          // every ray's sums past the last ray's set-up and hold all their
+          // weights live at once.  (The empty statements emit nothing; they
+          // make this ray's sums complete before the next ray's begin.)
+#pragma unroll
+          for (int k = 0; k < 9; ++k) {
+            asm volatile("" : "+v"(acc[k]));
+            if (WEIGHT) asm volatile("" : "+v"(accw[k]));
+          }
         }
       }
     }
@@ -1196,12 +1360,12 @@ extern "C" int tg_stem_backproject(const tg_stem_geometry* g, const double* para
              "tg_stem_backproject: detector of %lld pixels exceeds 2^30", (long long)g->det_h * g->det_w);
   const int64_t ntile = tg::cdiv((int64_t)g->n_side, (int64_t)kBpRayTile);
   dim3 grid((unsigned)(ntile * ntile), (unsigned)((int64_t)g->scan_h * g->scan_w));
-  if (weight != nullptr)
-    hipLaunchKernelGGL(stem_backproject_kernel<true>, grid, dim3(kThreads), 0, (hipStream_t)stream, *g, params, data4d,
-                       cam, image, weight);
-  else
-    hipLaunchKernelGGL(stem_backproject_kernel<false>, grid, dim3(kThreads), 0, (hipStream_t)stream, *g, params,
-                       data4d, cam, image, weight);
+  // grids whose axes lie along the slopes (no rotation between them)
+  const bool separable = g->img_m[1] == 0.0 && g->img_m[3] == 0.0 && g->det_m[1] == 0.0 && g->det_m[3] == 0.0 &&
+                         std::isfinite(g->defocus);
+  auto* kernel = weight != nullptr ? (separable ? stem_backproject_kernel<true, true> : stem_backproject_kernel<true, false>)
+                                   : (separable ? stem_backproject_kernel<false, true> : stem_backproject_kernel<false, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, (hipStream_t)stream, *g, params, data4d, cam, image, weight);
   TG_LAUNCH_CHECK("stem_backproject_kernel launch");
   return TG_OK;
 }
