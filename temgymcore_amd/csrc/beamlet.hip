@@ -651,13 +651,19 @@ __global__ __launch_bounds__(256) void beamlet_moment_kernel(const tg_beamlet_co
   const int64_t b = (int64_t)blockIdx.x * kBeamletsPerMomentBlock + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (b >= n) return;  // whole wavefronts leave; no block barrier below
   double M[kMoments];
-  beamlet_moments(unit[b], H, W, w, lane, M);
+  beamlet_moments<64>(unit[b], H, W, w, lane, M);
 #pragma unroll
   for (int k = 0; k < kMoments; ++k) M[k] = wave_sum_f64(M[k]);
   if (lane == 0) {
 #pragma unroll
     for (int k = 0; k < kMoments; ++k) moments[b * kMoments + k] = M[k];
   }
+}
+
+__global__ __launch_bounds__(64 * kSharedWaves) void beamlet_moment_shared_kernel(
+    const tg_beamlet_coef* __restrict__ unit, int32_t H, int32_t W, const float2* __restrict__ w,
+    double* __restrict__ moments) {
+  block_moments(unit[blockIdx.x], H, W, w, moments + (int64_t)blockIdx.x * kMoments);
 }
 
 // The chain rule of one beamlet (blockIdx.x, lane) along one direction
@@ -940,8 +946,12 @@ extern "C" int tg_beamlet_backward(const double* params, int64_t n, const double
   hipLaunchKernelGGL(conj_pad_kernel, dim3((unsigned)tg::cdiv(npix + kRun, 256)), dim3(256), 0, s,
                      (const float2*)grad_field, npix, w);
   TG_LAUNCH_CHECK("conj_pad_kernel launch");
-  hipLaunchKernelGGL(beamlet_moment_kernel, dim3((unsigned)tg::cdiv(n, kBeamletsPerMomentBlock)), dim3(256), 0, s,
-                     unit, n, (int32_t)height, (int32_t)width, w, moments);
+  if (share_moments(n))
+    hipLaunchKernelGGL(beamlet_moment_shared_kernel, dim3((unsigned)n), dim3(64 * kSharedWaves), 0, s, unit,
+                       (int32_t)height, (int32_t)width, w, moments);
+  else
+    hipLaunchKernelGGL(beamlet_moment_kernel, dim3((unsigned)tg::cdiv(n, kBeamletsPerMomentBlock)), dim3(256), 0, s,
+                       unit, n, (int32_t)height, (int32_t)width, w, moments);
   TG_LAUNCH_CHECK("beamlet_moment_kernel launch");
   // the 20 ray-transfer directions only where their gradient is wanted
   const unsigned n_dir = grad_abcd != nullptr ? 31 : 11;

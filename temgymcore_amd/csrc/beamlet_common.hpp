@@ -519,13 +519,15 @@ __device__ __forceinline__ void centre_pixel(const tg_beamlet_coef& c, int32_t H
 }
 
 constexpr int kMoments = 12;  // 6 complex moments
+constexpr int kSharedWaves = 4;  // wavefronts of a workgroup that shares one beamlet's
 
-// One wavefront's partial moments of beamlet c (wave-uniform record) over
+// One lane's share of the moments of beamlet c (wave-uniform record) over
 // the pixels of its cutoff ellipse in an H x W image of adjoint weights:
 //   M = sum over pixels of W E {1, u, v, u^2, uv, v^2}   (re, im interleaved)
 // with E = exp(Phi_c), (u, v) = pixel offsets from centre_pixel(c).  Lane
-// `lane` of 64 takes every 64th 16-pixel run; f32 within a run, f64 across
-// runs.  `wbase` needs kRun readable elements past the image (tail padding).
+// `lane` of LANES takes every LANES-th 16-pixel run; f32 within a run, f64
+// across runs.  `wbase` needs kRun readable elements past the image (tail padding).
+template <int LANES>
 __device__ inline void beamlet_moments(const tg_beamlet_coef& c, int32_t H, int32_t W,
                                        const float2* __restrict__ wbase, int lane, double (&M)[kMoments]) {
   // pixel box of the cutoff ellipse, clipped to the image (NaN -> whole image)
@@ -539,10 +541,10 @@ __device__ inline void beamlet_moments(const tg_beamlet_coef& c, int32_t H, int3
     const int32_t c0 = (int32_t)fc0, r0 = (int32_t)fr0;
     const int32_t nrows = (int32_t)fr1 - r0 + 1;
     const int32_t rpr = ((int32_t)fc1 - c0 + kRun) / kRun;  // 16-pixel runs per row
-    // lane -> (row offset, run) of task `lane`, then advance by 64 tasks per
-    // step without dividing: 64 = q rpr + rem
+    // lane -> (row offset, run) of task `lane`, then advance by LANES tasks per
+    // step without dividing: LANES = q rpr + rem
     int32_t rr = lane / rpr, run = lane - (lane / rpr) * rpr;
-    const int32_t q = 64 / rpr, rem = 64 - q * rpr;
+    const int32_t q = LANES / rpr, rem = LANES - q * rpr;
     const float2 K = make_float2(c.k_re, c.k_im);
     while (rr < nrows) {
       const int32_t row = r0 + rr;
@@ -617,5 +619,36 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
+
+// The moments of one beamlet by a workgroup of kSharedWaves wavefronts into
+// out[kMoments] (every thread of it calls this): the wavefronts' sums, in order.
+__device__ __forceinline__ void block_moments(const tg_beamlet_coef& c, int32_t H, int32_t W,
+                                              const float2* __restrict__ wbase, double* __restrict__ out) {
+  __shared__ double part[kSharedWaves][kMoments];
+  double M[kMoments];
+  beamlet_moments<64 * kSharedWaves>(c, H, W, wbase, threadIdx.x, M);
+#pragma unroll
+  for (int k = 0; k < kMoments; ++k) M[k] = wave_sum_f64(M[k]);
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int k = 0; k < kMoments; ++k) part[threadIdx.x >> 6][k] = M[k];
+  }
+  __syncthreads();
+  if (threadIdx.x < kMoments) {
+    double sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < kSharedWaves; ++w) sum += part[w][threadIdx.x];
+    out[threadIdx.x] = sum;
+  }
+}
+
+// Whether four wavefronts share a beamlet's moments: where one each would not
+// give every SIMD eight, and the time is that of a beamlet's runs one after the
+// other.  Backward of 64 beamlets on 500 x 612 pixels 69 / 37 us, 300 on 200^2
+// 61 / 38, 2,048 on 500 x 612 83 / 80, 4,096 on 600 x 612 with a 4-sigma cut
+// (few runs each) 59 / 66; a fit of two images, 100 Gaussians, 182 / 94.
+// Sixteen wavefronts are 1 to 7 us better for the smallest of these and slower
+// from 300 beamlets on.
+inline bool share_moments(int64_t n) { return n < 32LL * tg::cu_count(); }
 
 }  // namespace tgb

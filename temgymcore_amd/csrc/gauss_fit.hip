@@ -16,8 +16,9 @@
 //   fit_loss_kernel     per 4096-pixel chunk: u = sum of the slices (f64),
 //                       r = |u|^2 - T, loss partial sum of r^2 and the adjoint
 //                       weight W = (4/N) r conj(u).
-//   fit_loss_final      per instance: fixed-order sum of its partials / N.
-//   fit_moment_kernel   one wavefront per Gaussian, over the pixels of its
+//   fit_loss_final      a wavefront per instance: fixed-order sum of its
+//                       partials / N.
+//   fit_moment_kernel   one wavefront (four for few Gaussians) per Gaussian, over the pixels of its
 //                       cutoff ellipse: the six complex moments
 //                       sum W E {1, u, v, u^2, uv, v^2}, E = exp(Phi_unit),
 //                       (u, v) = pixel offsets from the Gaussian's centre
@@ -129,14 +130,16 @@ __global__ __launch_bounds__(256) void fit_loss_kernel(const FitInst* __restrict
   if (t == 0) loss_part[blockIdx.x] = (wsum[0] + wsum[1]) + (wsum[2] + wsum[3]);
 }
 
-__global__ __launch_bounds__(256) void fit_loss_final(const FitInst* __restrict__ insts, int32_t n_inst,
-                                                      const double* __restrict__ loss_part,
-                                                      double* __restrict__ loss) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n_inst) return;
+// A wavefront an instance (a lane an instance waited for each partial in turn:
+// 18 us for up to 64 of them).
+__global__ __launch_bounds__(64) void fit_loss_final(const FitInst* __restrict__ insts,
+                                                     const double* __restrict__ loss_part,
+                                                     double* __restrict__ loss) {
+  const FitInst& I = insts[blockIdx.x];
   double s = 0.0;
-  for (int b = insts[i].lb0; b < insts[i].lb1; ++b) s += loss_part[b];
-  loss[i] = s / ((double)insts[i].H * (double)insts[i].W);
+  for (int b = I.lb0 + (int)threadIdx.x; b < I.lb1; b += 64) s += loss_part[b];
+  s = wave_sum_f64(s);
+  if (threadIdx.x == 0) loss[blockIdx.x] = s / ((double)I.H * (double)I.W);
 }
 
 __global__ __launch_bounds__(256) void fit_moment_kernel(const tg_beamlet_coef* __restrict__ unit,
@@ -152,13 +155,22 @@ __global__ __launch_bounds__(256) void fit_moment_kernel(const tg_beamlet_coef* 
   const int32_t g = __builtin_amdgcn_readfirstlane(order[slot]);
   const FitInst& I = insts[__builtin_amdgcn_readfirstlane(gauss_inst[g])];
   double M[kMoments];
-  beamlet_moments(unit[g], I.H, I.W, weight + I.pix0, lane, M);
+  beamlet_moments<64>(unit[g], I.H, I.W, weight + I.pix0, lane, M);
 #pragma unroll
   for (int k = 0; k < kMoments; ++k) M[k] = wave_sum_f64(M[k]);
   if (lane == 0) {
 #pragma unroll
     for (int k = 0; k < kMoments; ++k) moments[(int64_t)g * kMoments + k] = M[k];
   }
+}
+
+__global__ __launch_bounds__(64 * kSharedWaves) void fit_moment_shared_kernel(
+    const tg_beamlet_coef* __restrict__ unit, const FitInst* __restrict__ insts,
+    const int32_t* __restrict__ gauss_inst, const int32_t* __restrict__ order, const float2* __restrict__ weight,
+    double* __restrict__ moments) {
+  const int32_t g = order[blockIdx.x];
+  const FitInst& I = insts[gauss_inst[g]];
+  block_moments(unit[g], I.H, I.W, weight + I.pix0, moments + (int64_t)g * kMoments);
 }
 
 __device__ __forceinline__ double re_mul(cd a, cd z) { return a.re * z.re - a.im * z.im; }
@@ -481,14 +493,17 @@ extern "C" int tg_gauss_fit_run(const tg_fit_plan* plan, void* workspace, const 
   TG_LAUNCH_CHECK("fit_loss_kernel launch");
   if (target == nullptr) return TG_OK;
   if (loss) {
-    hipLaunchKernelGGL(fit_loss_final, dim3((unsigned)tg::cdiv(plan->n_inst, 256)), dim3(256), 0, s, insts,
-                       plan->n_inst, loss_part, loss);
+    hipLaunchKernelGGL(fit_loss_final, dim3((unsigned)plan->n_inst), dim3(64), 0, s, insts, loss_part, loss);
     TG_LAUNCH_CHECK("fit_loss_final launch");
   }
   if (grad == nullptr || G == 0) return TG_OK;
   if (plan->n_moment_blocks > 0) {
-    hipLaunchKernelGGL(fit_moment_kernel, dim3((unsigned)plan->n_moment_blocks), dim3(256), 0, s, unit, insts, ginst,
-                       order, plan->n_assigned, weight, moments);
+    if (share_moments(plan->n_assigned))
+      hipLaunchKernelGGL(fit_moment_shared_kernel, dim3((unsigned)plan->n_assigned), dim3(64 * kSharedWaves), 0, s,
+                         unit, insts, ginst, order, weight, moments);
+    else
+      hipLaunchKernelGGL(fit_moment_kernel, dim3((unsigned)plan->n_moment_blocks), dim3(256), 0, s, unit, insts, ginst,
+                         order, plan->n_assigned, weight, moments);
     TG_LAUNCH_CHECK("fit_moment_kernel launch");
   }
   hipLaunchKernelGGL(fit_grad_kernel, dim3((unsigned)tg::cdiv(G, 256)), dim3(256), 0, s, params, G, ginst, insts,
