@@ -322,21 +322,24 @@ class _PackParams(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         out = []
+        cols, n = g.unbind(1), len(g)
         for k, (col, kind, shape, dtype, count) in enumerate(ctx.slots):
             if not ctx.needs_input_grad[2 + k]:
                 out.append(None)
-            elif kind == "pair":
+                continue
+            if kind == "pair":
                 v = g[:, col:col + 2]
-                v = v.sum(0, keepdim=True) if count == 2 and len(g) != 1 else v.contiguous()
-                out.append(v.to(dtype).reshape(shape))
+                v = v.sum(0, keepdim=True) if count == 2 and n != 1 else v.contiguous()
             else:
-                v = g[:, col]
+                v = cols[col]
                 if dtype.is_complex:
                     part = torch.float32 if dtype == torch.complex64 else torch.float64
-                    v = torch.complex(v.to(part), g[:, col + 1].to(part))
-                if count == 1 and len(g) != 1:
+                    v = torch.complex(v.to(part), cols[col + 1].to(part))
+                if count == 1 and n != 1:
                     v = v.sum(0)
-                out.append(v.to(dtype).reshape(shape))
+            if v.dtype != dtype:
+                v = v.to(dtype)
+            out.append(v if v.shape == shape else v.reshape(shape))
         return (None, None, *out)
 
 
@@ -533,13 +536,13 @@ def _check_beamlet_inputs(params: torch.Tensor, mode: int, abcd: torch.Tensor | 
 
 
 def beamlet_coefficients(params: torch.Tensor, grid, mode: int, abcd: torch.Tensor | None = None,
-                         abcd_stride: int = 0, cutoff: float | None = None) -> torch.Tensor:
+                         abcd_stride: int = 0, cutoff: float | None = None, *, pix2m=None) -> torch.Tensor:
     """Run the f64 coefficient kernel; returns a uint8 tensor of n packed records."""
     _check_beamlet_inputs(params, mode, abcd, abcd_stride)
     lib = _lib.load()
     n = int(params.shape[0])
     out = torch.empty(n * ctypes.sizeof(BeamletCoef), dtype=torch.uint8, device=params.device)
-    m = _pix2m(grid)
+    m = _pix2m(grid) if pix2m is None else pix2m
     st = lib.tg_beamlet_coefficients(params.data_ptr(), n, abcd.data_ptr() if abcd is not None else None,
                                      abcd_stride, mode, m.ctypes.data, float(cutoff or 0.0), out.data_ptr(),
                                      _lib.stream_ptr(params.device))
@@ -572,11 +575,11 @@ class BeamletSum:
 
 
 def beamlet_field(params: torch.Tensor, grid, mode: int, abcd: torch.Tensor | None = None, abcd_stride: int = 0,
-                  cutoff: float | None = None) -> torch.Tensor:
+                  cutoff: float | None = None, *, pix2m=None) -> torch.Tensor:
     """complex64 field [H, W] of the beamlets params [n, 16] on `grid`."""
     params = params.detach().contiguous()
     abcd = None if abcd is None else abcd.detach().contiguous()
-    coef = beamlet_coefficients(params, grid, mode, abcd, abcd_stride, cutoff)
+    coef = beamlet_coefficients(params, grid, mode, abcd, abcd_stride, cutoff, pix2m=pix2m)
     summer = BeamletSum(params.shape[0], grid.shape, params.device)
     summer.run(coef)
     return summer.image  # (its own buffer: no copy)
@@ -584,7 +587,7 @@ def beamlet_field(params: torch.Tensor, grid, mode: int, abcd: torch.Tensor | No
 
 def beamlet_backward(params: torch.Tensor, grid, mode: int, grad_field: torch.Tensor,
                      abcd: torch.Tensor | None = None, abcd_stride: int = 0, cutoff: float | None = None,
-                     want_abcd: bool = False):
+                     want_abcd: bool = False, *, pix2m=None):
     """Adjoint of ``beamlet_field``: (dL/dparams [n, 16] f64, dL/dT [n, 25] f64
     or None) for the field cotangent grad_field = dL/dRe + i dL/dIm."""
     lib = _lib.load()
@@ -603,7 +606,7 @@ def beamlet_backward(params: torch.Tensor, grid, mode: int, grad_field: torch.Te
     ws_bytes = int(lib.tg_beamlet_backward_workspace(n, H, W))
     raw = torch.empty(ws_bytes + 256, dtype=torch.uint8, device=params.device)
     off = (-raw.data_ptr()) % 256
-    m = _pix2m(grid)
+    m = _pix2m(grid) if pix2m is None else pix2m
     st = lib.tg_beamlet_backward(params.data_ptr(), n, abcd.data_ptr() if abcd is not None else None, abcd_stride,
                                  mode, m.ctypes.data, float(cutoff or 0.0), H, W,
                                  torch.view_as_real(g).data_ptr(), grad.data_ptr(),
@@ -618,14 +621,15 @@ class _BeamletField(torch.autograd.Function):
     def forward(ctx, params, abcd, grid, mode, abcd_stride, cutoff):
         ctx.save_for_backward(params, abcd)
         ctx.grid, ctx.mode, ctx.abcd_stride, ctx.cutoff = grid, mode, abcd_stride, cutoff
-        return beamlet_field(params, grid, mode, abcd, abcd_stride, cutoff)
+        ctx.pix2m = _pix2m(grid)
+        return beamlet_field(params, grid, mode, abcd, abcd_stride, cutoff, pix2m=ctx.pix2m)
 
     @staticmethod
     def backward(ctx, grad_field):
         params, abcd = ctx.saved_tensors
         want_abcd = abcd is not None and ctx.needs_input_grad[1]
         gp, ga = beamlet_backward(params, ctx.grid, ctx.mode, grad_field, abcd, ctx.abcd_stride, ctx.cutoff,
-                                  want_abcd=want_abcd)
+                                  want_abcd=want_abcd, pix2m=ctx.pix2m)
         g_abcd = None
         if want_abcd:
             ga = ga.view(-1, 5, 5)
