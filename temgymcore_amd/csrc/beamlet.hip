@@ -651,7 +651,7 @@ __global__ __launch_bounds__(256) void beamlet_moment_kernel(const tg_beamlet_co
   const int64_t b = (int64_t)blockIdx.x * kBeamletsPerMomentBlock + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (b >= n) return;  // whole wavefronts leave; no block barrier below
   double M[kMoments];
-  beamlet_moments<64>(unit[b], H, W, w, lane, M);
+  beamlet_moments<1>(unit[b], H, W, w, lane, M);
 #pragma unroll
   for (int k = 0; k < kMoments; ++k) M[k] = wave_sum_f64(M[k]);
   if (lane == 0) {

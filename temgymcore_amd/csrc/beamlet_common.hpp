@@ -521,15 +521,79 @@ __device__ __forceinline__ void centre_pixel(const tg_beamlet_coef& c, int32_t H
 constexpr int kMoments = 12;  // 6 complex moments
 constexpr int kSharedWaves = 4;  // wavefronts of a workgroup that shares one beamlet's
 
-// One lane's share of the moments of beamlet c (wave-uniform record) over
-// the pixels of its cutoff ellipse in an H x W image of adjoint weights:
+// The terms of Phi that a row fixes (run_start's, at row py).
+struct RowTerms {
+  double lre, lim, cre, cim;
+};
+
+// The moments of pixels xs .. xs + cnt of a row (cnt < kRun; WHOLE: all kRun)
+// with weights w, added to M: v = row - pcy, ub = xs - pcx.  f32 within the run,
+// f64 across runs.
+template <bool WHOLE>
+__device__ __forceinline__ void run_moments(const tg_beamlet_coef& c, const RowTerms& r, int32_t xs, int32_t cnt,
+                                            const float2 (&w)[kRun], double ub, double v, double (&M)[kMoments]) {
+  const double px = (double)xs, px2 = 2.0 * px + 1.0;
+  float2 F = cexp_f(fma(fma(c.phi[0], px, r.lre), px, r.cre), fma(fma(c.phi[1], px, r.lim), px, r.cim));
+  float2 R = cexp_f(fma(c.phi[0], px2, r.lre), fma(c.phi[1], px2, r.lim));
+  const float2 K = make_float2(c.k_re, c.k_im);
+  float2 s0 = make_float2(0.f, 0.f), s1 = s0, s2 = s0;
+  // branch-free: steps past cnt are computed and discarded (select, so
+  // an overflowing tail cannot leak into the sums)
+#pragma unroll
+  for (int k = 0; k < kRun; ++k) {
+    float2 P = cmulf(w[k], F);
+    if (!WHOLE && k > 0) {
+      const bool on = k <= cnt;
+      P.x = on ? P.x : 0.0f;
+      P.y = on ? P.y : 0.0f;
+    }
+    s0.x += P.x;
+    s0.y += P.y;
+    s1.x = fmaf((float)k, P.x, s1.x);
+    s1.y = fmaf((float)k, P.y, s1.y);
+    s2.x = fmaf((float)(k * k), P.x, s2.x);
+    s2.y = fmaf((float)(k * k), P.y, s2.y);
+    if (k + 1 < kRun) {
+      F = cmulf(F, R);
+      R = cmulf(R, K);
+    }
+  }
+  // run sums over k = x - xs -> moments in u = x - pcx = ub + k, v = row - pcy
+  const double a0r = s0.x, a0i = s0.y, a1r = s1.x, a1i = s1.y, a2r = s2.x, a2i = s2.y, vv = v * v;
+  const double u1r = fma(ub, a0r, a1r), u1i = fma(ub, a0i, a1i);  // sum u P
+  M[0] += a0r;
+  M[1] += a0i;
+  M[2] += u1r;
+  M[3] += u1i;
+  M[4] = fma(v, a0r, M[4]);
+  M[5] = fma(v, a0i, M[5]);
+  M[6] += fma(ub, u1r + a1r, a2r);  // sum u^2 P = ub (ub a0 + 2 a1) + a2
+  M[7] += fma(ub, u1i + a1i, a2i);
+  M[8] = fma(v, u1r, M[8]);
+  M[9] = fma(v, u1i, M[9]);
+  M[10] = fma(vv, a0r, M[10]);
+  M[11] = fma(vv, a0i, M[11]);
+}
+
+// Thread t's share (of 64 WAVES) of the moments of beamlet c (wave-uniform
+// record) over the pixels of its cutoff ellipse in an H x W image of adjoint
+// weights:
 //   M = sum over pixels of W E {1, u, v, u^2, uv, v^2}   (re, im interleaved)
-// with E = exp(Phi_c), (u, v) = pixel offsets from centre_pixel(c).  Lane
-// `lane` of LANES takes every LANES-th 16-pixel run; f32 within a run, f64
-// across runs.  `wbase` needs kRun readable elements past the image (tail padding).
-template <int LANES>
+// with E = exp(Phi_c), (u, v) = pixel offsets from centre_pixel(c).  `wbase`
+// needs kRun readable elements past the image (tail padding).
+//
+// Bound: vector issue and the power it draws (18 instructions a pixel of a
+// whole run, 21 of a cut one, about 70 a run).  So a lane keeps a row, whose
+// extent and terms of Phi it makes once, and walks its 16-pixel runs column by
+// column (fewer than 64 rows: the wavefront takes several columns at a time):
+// the runs inside the ellipse are then whole for all lanes at once.
+// 76,000 Gaussians on 256 images of 128^2 to 512^2 pixels: 2.69 ms with the runs
+// dealt to the lanes in turn, 2.34 so; 9,000 beamlets on 600^2 257 / 238 us with
+// the rest of their backward; 4,096 on 600 x 612 with a 4-sigma cut, whose few
+// rows fill the lanes less well, 59 / 68.
+template <int WAVES>
 __device__ inline void beamlet_moments(const tg_beamlet_coef& c, int32_t H, int32_t W,
-                                       const float2* __restrict__ wbase, int lane, double (&M)[kMoments]) {
+                                       const float2* __restrict__ wbase, int t, double (&M)[kMoments]) {
   // pixel box of the cutoff ellipse, clipped to the image (NaN -> whole image)
   const float fc0 = fmaxf(ceilf(c.cx - c.box_w), 0.0f), fc1 = fminf(floorf(c.cx + c.box_w), (float)(W - 1));
   const float fr0 = fmaxf(ceilf(c.cy - c.box_h), 0.0f), fr1 = fminf(floorf(c.cy + c.box_h), (float)(H - 1));
@@ -537,79 +601,53 @@ __device__ inline void beamlet_moments(const tg_beamlet_coef& c, int32_t H, int3
   centre_pixel(c, H, W, pcx, pcy);
 #pragma unroll
   for (int k = 0; k < kMoments; ++k) M[k] = 0.0;
-  if (fc0 <= fc1 && fr0 <= fr1) {
-    const int32_t c0 = (int32_t)fc0, r0 = (int32_t)fr0;
-    const int32_t nrows = (int32_t)fr1 - r0 + 1;
-    const int32_t rpr = ((int32_t)fc1 - c0 + kRun) / kRun;  // 16-pixel runs per row
-    // lane -> (row offset, run) of task `lane`, then advance by LANES tasks per
-    // step without dividing: LANES = q rpr + rem
-    int32_t rr = lane / rpr, run = lane - (lane / rpr) * rpr;
-    const int32_t q = LANES / rpr, rem = LANES - q * rpr;
-    const float2 K = make_float2(c.k_re, c.k_im);
-    while (rr < nrows) {
-      const int32_t row = r0 + rr;
-      const int32_t x0 = c0 + run * kRun;
-      int32_t xs, xe;
-      if (row_extent(c, row, x0, W, xs, xe)) {
-        // the pixels xs .. xe (at most kRun) of this run, as xs + k: their 16
-        // weights are loaded at once, before the f64 run-start math so that
-        // their latency overlaps it; reads past xe land in the row, the next
-        // row or the buffer's kRun-element tail padding (xs <= W - 1) and are
-        // masked out below
-        const float2* wrun = wbase + (int64_t)row * W + xs;
-        float2 w[kRun];
+  if (!(fc0 <= fc1 && fr0 <= fr1)) return;
+  const int32_t c0 = __builtin_amdgcn_readfirstlane((int32_t)fc0), r0 = __builtin_amdgcn_readfirstlane((int32_t)fr0);
+  const int32_t nrows = __builtin_amdgcn_readfirstlane((int32_t)fr1) - r0 + 1;
+  const int32_t rpr = (__builtin_amdgcn_readfirstlane((int32_t)fc1) - c0 + kRun) / kRun;  // 16-pixel runs per row
+  const int32_t cend = (int32_t)min((int64_t)c0 + (int64_t)rpr * kRun, (int64_t)W) - 1;    // last pixel of the runs
+  const int lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  int lg = 6;  // 2^lg rows and 2^(6 - lg) columns at a time
+  while (lg > 2 && (1 << (lg - 1)) >= nrows) --lg;
+  const int ncol = 64 >> lg;
+  const double* a = c.phi;
+  for (int32_t rb = 0; rb < nrows; rb += 1 << lg) {
+    const int32_t row = r0 + rb + (lane & ((1 << lg) - 1));
+    // the row's pixels inside the ellipse (row_extent, for all its runs)
+    int32_t lo = c0, hi = cend;
+    if (c.gamma > 0.0f) {
+      const float v = (float)row - c.cy;
+      const float t2 = fmaf(-c.gamma * v, v, c.beta);
+      const float sq = __builtin_amdgcn_sqrtf(t2);
+      const float mid = fmaf(-c.alpha, v, c.cx);
+      lo = max((int32_t)fminf(fmaxf(ceilf(mid - sq), (float)c0), (float)(cend + 1)), c0);
+      hi = min((int32_t)fmaxf(fminf(floorf(mid + sq), (float)cend), (float)(c0 - 1)), cend);
+      if (t2 < 0.0f) hi = -1;
+    }
+    if (row >= r0 + nrows) hi = -1;
+    const double py = (double)row, v = py - (double)pcy;
+    const RowTerms r = {fma(a[2], py, a[6]), fma(a[3], py, a[7]), fma(fma(a[4], py, a[8]), py, a[10]),
+                        fma(fma(a[5], py, a[9]), py, a[11])};
+    const float2* __restrict__ wrow = wbase + (int64_t)row * W;
+    for (int32_t col = wave * ncol; col < rpr; col += WAVES * ncol) {
+      const int32_t x0 = c0 + (col + (lane >> lg)) * kRun;
+      const int32_t xs = max(lo, x0), xe = min(hi, x0 + kRun - 1);
+      if (xs > xe) continue;
+      // the pixels xs .. xe (at most kRun) of this run, as xs + k: their 16
+      // weights are loaded at once, before the f64 run-start math so that
+      // their latency overlaps it; reads past xe land in the row, the next
+      // row or the buffer's kRun-element tail padding (xs <= W - 1) and are
+      // masked out below
+      float2 w[kRun];
 #pragma unroll
-        for (int k = 0; k < kRun; ++k) w[k] = wrun[k];
-        // keep all 16 loads ahead of the math: one memory round trip per run
-        __builtin_amdgcn_sched_barrier(0);
-        const int32_t cnt = xe - xs;  // last active k
-        float2 F, R;
-        run_start(c, xs, row, F, R);
-        float2 s0 = make_float2(0.f, 0.f), s1 = s0, s2 = s0;
-        // branch-free: steps past cnt are computed and discarded (select, so
-        // an overflowing tail cannot leak into the sums)
-#pragma unroll
-        for (int k = 0; k < kRun; ++k) {
-          float2 P = cmulf(w[k], F);
-          if (k > 0) {
-            const bool on = k <= cnt;
-            P.x = on ? P.x : 0.0f;
-            P.y = on ? P.y : 0.0f;
-          }
-          s0.x += P.x;
-          s0.y += P.y;
-          s1.x = fmaf((float)k, P.x, s1.x);
-          s1.y = fmaf((float)k, P.y, s1.y);
-          s2.x = fmaf((float)(k * k), P.x, s2.x);
-          s2.y = fmaf((float)(k * k), P.y, s2.y);
-          if (k + 1 < kRun) {
-            F = cmulf(F, R);
-            R = cmulf(R, K);
-          }
-        }
-        // run sums over k = x - xs -> moments in u = x - pcx = ub + k, v = row - pcy
-        const double ub = (double)xs - (double)pcx, v = (double)row - (double)pcy, vv = v * v;
-        const double a0r = s0.x, a0i = s0.y, a1r = s1.x, a1i = s1.y, a2r = s2.x, a2i = s2.y;
-        const double u1r = fma(ub, a0r, a1r), u1i = fma(ub, a0i, a1i);  // sum u P
-        M[0] += a0r;
-        M[1] += a0i;
-        M[2] += u1r;
-        M[3] += u1i;
-        M[4] = fma(v, a0r, M[4]);
-        M[5] = fma(v, a0i, M[5]);
-        M[6] += fma(ub, u1r + a1r, a2r);  // sum u^2 P = ub (ub a0 + 2 a1) + a2
-        M[7] += fma(ub, u1i + a1i, a2i);
-        M[8] = fma(v, u1r, M[8]);
-        M[9] = fma(v, u1i, M[9]);
-        M[10] = fma(vv, a0r, M[10]);
-        M[11] = fma(vv, a0i, M[11]);
-      }
-      run += rem;
-      rr += q;
-      if (run >= rpr) {
-        run -= rpr;
-        ++rr;
-      }
+      for (int k = 0; k < kRun; ++k) w[k] = wrow[xs + k];
+      // keep all 16 loads ahead of the math: one memory round trip per run
+      __builtin_amdgcn_sched_barrier(0);
+      const double ub = (double)xs - (double)pcx;
+      if (__ballot(xe - xs != kRun - 1) == 0)
+        run_moments<true>(c, r, xs, kRun - 1, w, ub, v, M);
+      else
+        run_moments<false>(c, r, xs, xe - xs, w, ub, v, M);
     }
   }
 }
@@ -626,7 +664,7 @@ __device__ __forceinline__ void block_moments(const tg_beamlet_coef& c, int32_t 
                                               const float2* __restrict__ wbase, double* __restrict__ out) {
   __shared__ double part[kSharedWaves][kMoments];
   double M[kMoments];
-  beamlet_moments<64 * kSharedWaves>(c, H, W, wbase, threadIdx.x, M);
+  beamlet_moments<kSharedWaves>(c, H, W, wbase, threadIdx.x, M);
 #pragma unroll
   for (int k = 0; k < kMoments; ++k) M[k] = wave_sum_f64(M[k]);
   if ((threadIdx.x & 63) == 0) {
@@ -643,12 +681,12 @@ __device__ __forceinline__ void block_moments(const tg_beamlet_coef& c, int32_t 
 }
 
 // Whether four wavefronts share a beamlet's moments: where one each would not
-// give every SIMD eight, and the time is that of a beamlet's runs one after the
-// other.  Backward of 64 beamlets on 500 x 612 pixels 69 / 37 us, 300 on 200^2
-// 61 / 38, 2,048 on 500 x 612 83 / 80, 4,096 on 600 x 612 with a 4-sigma cut
-// (few runs each) 59 / 66; a fit of two images, 100 Gaussians, 182 / 94.
-// Sixteen wavefronts are 1 to 7 us better for the smallest of these and slower
-// from 300 beamlets on.
-inline bool share_moments(int64_t n) { return n < 32LL * tg::cu_count(); }
+// give every SIMD four, and the time is that of a beamlet's runs one after the
+// other.  One wavefront / four, backward of 64 beamlets on 500 x 612 pixels 59 /
+// 36 us, 300 on 200^2 53 / 37, 2,048 on 500 x 612 76 / 75, 4,096 on 300^2 122 /
+// 113, 4,096 on 600 x 612 with a 4-sigma cut (few runs each) 68 / 75; a fit of
+// two images, 100 Gaussians, 151 / 89.  Sixteen wavefronts are 1 to 7 us better
+// for the smallest of these and slower from 300 beamlets on.
+inline bool share_moments(int64_t n) { return n < 16LL * tg::cu_count(); }
 
 }  // namespace tgb

@@ -155,7 +155,7 @@ __global__ __launch_bounds__(256) void fit_moment_kernel(const tg_beamlet_coef* 
   const int32_t g = __builtin_amdgcn_readfirstlane(order[slot]);
   const FitInst& I = insts[__builtin_amdgcn_readfirstlane(gauss_inst[g])];
   double M[kMoments];
-  beamlet_moments<64>(unit[g], I.H, I.W, weight + I.pix0, lane, M);
+  beamlet_moments<1>(unit[g], I.H, I.W, weight + I.pix0, lane, M);
 #pragma unroll
   for (int k = 0; k < kMoments; ++k) M[k] = wave_sum_f64(M[k]);
   if (lane == 0) {
