@@ -470,7 +470,7 @@ def _result_fit(units, ms_per_step, step_ms, kern_ms, graph_ms, gpu_out, achieve
         config={"workload": "stem_fit: 64x64 scan, 64x64 rays, 8 camera lengths, 1.07 GB f32 targets",
                 "units_per_step": units, "event_ms_per_step": step_ms, "graph_replay_ms_per_step": graph_ms,
                 "dominant_kernel_event_ms": kern_ms,
-                "kernels_per_step": "stem_fit_kernel + row_sum_kernel, or stem_fit_cam_kernel + stem_fit_epilogue + "
+                "kernels_per_step": "stem_fit_kernel + row_sum_kernel, or stem_fit_cam_kernel<N> + stem_fit_epilogue + "
                                     "row_sum_kernel (the tuned variant); roofline.achieved uses the event time of "
                                     "the per-scan-position pass alone (tg_stem_fit_terms)",
                 "cpu_port_rel_diff_on_sample": rel, "loss": float(gpu_out[-1])},

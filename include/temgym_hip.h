@@ -286,7 +286,8 @@ int tg_stem_dataset(const tg_stem_geometry* geom, const double* params, const fl
  * Two launch variants give identical results: TG_STEM_FIT_SCAN (one
  * workgroup per scan position; the default when S >= 4 x the CU count) and
  * TG_STEM_FIT_CAMERA (one per scan position and camera length; the default
- * for smaller scans); the tuning knob TG_TUNE_STEM_FIT overrides. */
+ * for smaller scans; up to 2,048 of them are reduced by one launch); the
+ * tuning knob TG_TUNE_STEM_FIT overrides. */
 /* Shadow-image back-projection: the adjoint of tg_stem_forward's 4D deposit
  * with respect to the sample image (the consumer of 4D-STEM data the
  * reference describes, README.md:13-16).  For every ray (s, j) whose detector

@@ -18,8 +18,9 @@
 //                       weight W = (4/N) r conj(u).
 //   fit_loss_final      a wavefront per instance: fixed-order sum of its
 //                       partials / N.
-//   fit_moment_kernel   one wavefront (four for few Gaussians) per Gaussian, over the pixels of its
-//                       cutoff ellipse: the six complex moments
+//   fit_moment_kernel   one wavefront (four for few Gaussians) per Gaussian,
+//                       over the pixels of its cutoff ellipse: the six complex
+//                       moments
 //                       sum W E {1, u, v, u^2, uv, v^2}, E = exp(Phi_unit),
 //                       (u, v) = pixel offsets from the Gaussian's centre
 //                       pixel.  f32 within a 16-pixel run, f64 across runs
