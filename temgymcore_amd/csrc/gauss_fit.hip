@@ -96,6 +96,13 @@ __global__ __launch_bounds__(kThreads) void fit_forward_kernel(const tg_beamlet_
                            partial + I.ws0 + (int64_t)it.slice * H * (int64_t)W);
 }
 
+// Bound: reading the partial fields.  Four pixels a thread at a time keep as many
+// loads in flight (the index clamped, so that none waits for a test): one pixel
+// at a time waited for each slice and then for the target.  Whole fits, one /
+// four pixels (instances, up to Gaussians each, up to pixels a side): 256 x 2,000
+// on 512^2 3,931 / 3,885 us, 20 x 2,000 on 512^2 634 / 612, 2 x 2,000 on 140^2 219 /
+// 212, 2 x 100 on 512^2 88 / 85, 200 x 100 on 200^2 241 / 238; eight pixels 3,886,
+// 608, 210, 85, 243.
 __global__ __launch_bounds__(256) void fit_loss_kernel(const FitInst* __restrict__ insts,
                                                        const LossBlock* __restrict__ blocks,
                                                        const float2* __restrict__ partial,
@@ -108,20 +115,39 @@ __global__ __launch_bounds__(256) void fit_loss_kernel(const FitInst* __restrict
   const double scale = 4.0 / (double)npix;
   const int t = threadIdx.x;
   double acc = 0.0;
-  for (int k = 0; k < kLossChunk / 256; ++k) {
-    const int64_t p = (int64_t)lb.chunk * kLossChunk + k * 256 + t;
-    if (p >= npix) break;
-    double ur = 0.0, ui = 0.0;
-    for (int s = 0; s < I.nslice; ++s) {
-      const float2 v = partial[I.ws0 + (int64_t)s * npix + p];
-      ur += v.x;
-      ui += v.y;
+  constexpr int kPix = 4;  // pixels a thread at a time
+  for (int k = 0; k < kLossChunk / 256; k += kPix) {
+    const int64_t p0 = (int64_t)lb.chunk * kLossChunk + k * 256 + t;
+    if (p0 >= npix) break;
+    int64_t p[kPix];
+    float want[kPix];
+    double ur[kPix], ui[kPix];
+#pragma unroll
+    for (int q = 0; q < kPix; ++q) {
+      p[q] = min(p0 + q * 256, npix - 1);
+      want[q] = target ? target[I.pix0 + p[q]] : 0.f;
+      ur[q] = ui[q] = 0.0;
     }
-    if (field) field[I.pix0 + p] = make_float2((float)ur, (float)ui);
-    if (target) {
-      const double r = (ur * ur + ui * ui) - (double)target[I.pix0 + p];
-      acc += r * r;
-      weight[I.pix0 + p] = make_float2((float)(scale * r * ur), (float)(-scale * r * ui));
+    const float2* __restrict__ src = partial + I.ws0;
+    for (int s = 0; s < I.nslice; ++s, src += npix) {
+      float2 v[kPix];
+#pragma unroll
+      for (int q = 0; q < kPix; ++q) v[q] = src[p[q]];
+#pragma unroll
+      for (int q = 0; q < kPix; ++q) {
+        ur[q] += v[q].x;
+        ui[q] += v[q].y;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kPix; ++q) {
+      if (p0 + q * 256 >= npix) break;
+      if (field) field[I.pix0 + p[q]] = make_float2((float)ur[q], (float)ui[q]);
+      if (target) {
+        const double r = (ur[q] * ur[q] + ui[q] * ui[q]) - (double)want[q];
+        acc += r * r;
+        weight[I.pix0 + p[q]] = make_float2((float)(scale * r * ur[q]), (float)(-scale * r * ui[q]));
+      }
     }
   }
   if (!target) return;
