@@ -470,20 +470,23 @@ __device__ __forceinline__ void tile_sum(const tg_beamlet_coef* __restrict__ coe
     }
     if (hit) sh.list[off + __popcll(mask & ((1ull << lane) - 1ull))] = (int32_t)(b - b0);
     __syncthreads();
-    // (the next record is loaded while this one is summed)
-    tg_beamlet_coef next = coef[b0 + __builtin_amdgcn_readfirstlane(sh.list[0])];
-    for (int q = 0; q < total; ++q) {
-      const tg_beamlet_coef c = next;
-      next = coef[b0 + __builtin_amdgcn_readfirstlane(sh.list[min(q + 1, total - 1)])];
-      int32_t xs, xe;
-      if (row >= H || !row_extent<RUN>(c, row, x0, W, xs, xe)) continue;
-      float2 F, R;
-      run_start(c, xs, row, F, R);
-      const float2 K = make_float2(c.k_re, c.k_im);
-      // bit 31 - j: pixel x0 + j is inside
-      uint32_t inside = (0xffffffffu >> (xs - x0)) & ~(0x7fffffffu >> (xe - x0));
+    // (the next record is loaded while this one is summed; with no beamlet in the
+    // list, list[0] is whatever LDS held)
+    if (total > 0) {
+      tg_beamlet_coef next = coef[b0 + __builtin_amdgcn_readfirstlane(sh.list[0])];
+      for (int q = 0; q < total; ++q) {
+        const tg_beamlet_coef c = next;
+        next = coef[b0 + __builtin_amdgcn_readfirstlane(sh.list[min(q + 1, total - 1)])];
+        int32_t xs, xe;
+        if (row >= H || !row_extent<RUN>(c, row, x0, W, xs, xe)) continue;
+        float2 F, R;
+        run_start(c, xs, row, F, R);
+        const float2 K = make_float2(c.k_re, c.k_im);
+        // bit 31 - j: pixel x0 + j is inside
+        uint32_t inside = (0xffffffffu >> (xs - x0)) & ~(0x7fffffffu >> (xe - x0));
 #pragma unroll
-      for (int j = 0; j < RUN; ++j) run_step(inside, acc[j], F, R, K);
+        for (int j = 0; j < RUN; ++j) run_step(inside, acc[j], F, R, K);
+      }
     }
     __syncthreads();  // the list is rewritten by the next chunk
   }
