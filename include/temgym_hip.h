@@ -400,9 +400,12 @@ int tg_beamlet_coefficients(const double* params, int64_t n, const double* abcd,
  *   - every beamlet separable (Phi without a px*py term, envelope decaying
  *     along both axes, as for untilted round or axis-aligned beams): each
  *     128x128 tile is a complex matrix product Ey^T Ex over the beamlets whose
- *     cutoff ellipse meets it, Ex/Ey from f64 phases, on the matrix cores
- *     (factors as two f16 halves, f32 sums); culling is per tile, so terms
- *     below the cut inside such a tile are summed too;
+ *     cutoff ellipse meets it, Ex/Ey from f64 phases, on the matrix cores.
+ *     Factors are two f16 halves with f32 sums where all terms of a slice and
+ *     tile that the cut keeps lie within 2^20 of the largest there (2^25 for
+ *     a term at its cut), and f32 for any other slice and tile.  Culling is per
+ *     tile, so a term below the cut inside such a tile is summed too, wholly
+ *     or in part;
  *   - otherwise the per-lane f32 recurrence over 16-pixel runs, culled per
  *     run to the cutoff ellipse. */
 int64_t tg_beamlet_sum_workspace(int64_t n, int64_t height, int64_t width);

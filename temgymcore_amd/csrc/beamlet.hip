@@ -210,13 +210,18 @@ __global__ __launch_bounds__(kThreads) void beamlet_sum_kernel(const tg_beamlet_
 // carry), and a real product is ah bh + ah bl + al bh in f32 accumulators (what
 // is left out is below 2^-22 |a b|).  f16 has few exponents, so the factors are
 // scaled: each x factor by the power of two that takes its largest value in
-// the tile to [2^14, 2^15), and the y factor, amplitude included, by the rest,
-// so that no term exceeds 2^28 times 2^exp_now, the largest term met so far in
-// the tile.  A list block with larger terms rescales the sums first (an exact
-// power of two).  Parts of a factor below 2^-39 of its largest value in the
-// tile are lost, far below the f32 rounding of that value.  Against complex128,
-// norm of the error over norm of the field, 131,072 beamlets on 1024^2: 3.9e-6
-// (f32 products: 4.2e-6; both are the phasor recurrence's error).
+// the tile (its pixels on the image) to [2^14, 2^15), and the y factor,
+// amplitude included, by the rest, so that no term exceeds 2^29 times
+// 2^exp, the largest of the slice's terms in the tile.  What a factor has below
+// 2^-25 is lost, 2^-39 of its largest value: so the halves serve a slice and
+// tile all of whose terms that are to be kept lie within 2^20 of 2^exp (then no
+// kept term is off by more than 2^-19 of itself), or are cut off at no less than
+// 2^-25 of it (2^-14 of the weakest kept, in the mean 2^-16, where the cut leaves
+// out terms of that size).  Any other -- tails without a cut, weak beamlets
+// beside strong ones -- is left to the f32 products of beamlet_sum_wide_kernel.
+// Against complex128, norm of the error over norm of the field, 131,072
+// beamlets on 1024^2: 3.9e-6 (f32 products: 4.2e-6; both are the phasor
+// recurrence's error).
 //
 // Rate.  12 v_mfma_f32_32x32x16_f16 take 16 beamlets of a 32x32 block, 25
 // cycles a beamlet, where f32 products (three v_mfma_f32_32x32x2_f32 a pair)
@@ -252,9 +257,9 @@ __global__ __launch_bounds__(kThreads) void beamlet_sum_kernel(const tg_beamlet_
 // pairs per segment instead of a sine and cosine per value).
 //
 // 131,072 beamlets, 1024^2, 4 sigma, the whole sum: 4.64 ms with f32 products,
-// now 2.15 ms (tile sum 2.06, slices 0.08).  Bound: vector issue (63% of the
-// cycles, 520 instructions a chunk) and the matrix cores (46%) together, at
-// the 1.9 GHz that this mix runs at.
+// now 2.17 ms (of which the search for the range is 0.02).  Bound: vector issue
+// (63% of the cycles, 520 instructions a chunk) and the matrix cores (46%)
+// together, at the 1.9 GHz that this mix runs at.
 // ---------------------------------------------------------------------------
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -264,7 +269,11 @@ typedef float floatx2 __attribute__((ext_vector_type(2)));
 constexpr int kMxK = 16;           // beamlets per MFMA
 constexpr int kMxSeg = 16;         // pixels per evaluated segment
 constexpr int kMxBlock = 1024;     // beamlets per list build
-constexpr int kMxScale = 14;       // factors are held times 2^14 and at most 2^15: their low halves stay normal
+constexpr int kMxScaleX = 14;      // x factors are held times 2^14, below 2^15
+constexpr int kMxScaleY = 15;      // y factors at most 2^15 (f16 ends at 2^16)
+constexpr int kMxScale = kMxScaleX + kMxScaleY;
+constexpr int kMxRange = 20;       // bits from the largest term to the weakest that the halves serve
+constexpr int kMxCutBits = 5;      // further bits for a term at its own cut
 
 // A TW x TH tile, KC beamlets a chunk, BM x BN 32x32 blocks a wave: LDS layout
 // and workgroup.
@@ -272,7 +281,9 @@ template <int TW_, int TH_, int KC_, int BM_, int BN_>
 struct MxTile {
   static constexpr int TW = TW_, TH = TH_, KC = KC_, BM = BM_, BN = BN_;
   static constexpr int kPix = TW + TH;  // x pixels, then y pixels
-  static constexpr int kWaves = TW * TH / (1024 * BM * BN), kThreads = 64 * kWaves;
+  // waves side by side and one below the other; a wave's blocks lie as far apart
+  static constexpr int kCols = TW / (32 * BN), kRows = TH / (32 * BM);
+  static constexpr int kWaves = kCols * kRows, kThreads = 64 * kWaves;
   // dwords (two beamlets each) of one component of one split part, and of the
   // four of them for one MFMA's beamlets
   static constexpr int kPart = kPix * (kMxK / 2) + kPix / 16 * 16 + 8;
@@ -286,6 +297,7 @@ struct MxTile {
 using SepTile = MxTile<128, 128, 16, 2, 2>;
 
 constexpr int kNoExp = -(1 << 24);  // no beamlet met yet
+constexpr int kLeft = 0x7fa51e55;   // (a signalling NaN, which no sum is)
 
 __device__ __forceinline__ int wave_max_i32(int v) {
 #pragma unroll
@@ -294,8 +306,7 @@ __device__ __forceinline__ int wave_max_i32(int v) {
 }
 
 // dword offset of a pixel's row within a part
-constexpr int kBlockRow = 32 * (kMxK / 2) + 32;  // 32 pixels further
-__device__ __forceinline__ int mx_row(int pix) { return pix * (kMxK / 2) + (pix >> 4) * 16; }
+__host__ __device__ constexpr int mx_row(int pix) { return pix * (kMxK / 2) + (pix >> 4) * 16; }
 
 // Evaluation state of one 16-pixel segment starting at pixel p0: the
 // log2-scaled envelope, evaluated directly, and the unit phasor
@@ -422,7 +433,7 @@ __global__ __launch_bounds__(M::kThreads, 2) void beamlet_sum_sep_kernel(const S
                                                                     float2* __restrict__ ws) {
   constexpr int kT = M::kThreads, kW = M::kWaves, TW = M::TW, TH = M::TH;
   __shared__ int32_t list[kMxBlock];
-  __shared__ int32_t wave_cnt[kW], wave_exp[kW];
+  __shared__ int32_t wave_cnt[kW], wave_low[kW];
   __shared__ __align__(16) uint32_t fac[2][M::kBuffer];
   if (!matrix_path(flags)) return;  // beamlet_sum_kernel covers this launch
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -432,9 +443,11 @@ __global__ __launch_bounds__(M::kThreads, 2) void beamlet_sum_sep_kernel(const S
   const int split = blockIdx.x % nsplit, tile = blockIdx.x / nsplit;
   const int32_t tx0 = (tile % ntx) * TW, ty0 = (tile / ntx) * TH;
   const int64_t b_begin = n * split / nsplit, b_end = n * (split + 1) / nsplit;
-  const float ftx0 = (float)tx0, fty0 = (float)ty0, ftx1 = (float)(tx0 + TW - 1), fty1 = (float)(ty0 + TH - 1);
-  constexpr int kCols = TW / (32 * M::BN);
-  const int mb = (wave / kCols) * 32 * M::BM, nb = (wave % kCols) * 32 * M::BN;
+  // the tile's pixels on the image: nothing past them is scaled for
+  const int32_t tx1 = (int32_t)min((int64_t)tx0 + TW, W) - 1, ty1 = (int32_t)min((int64_t)ty0 + TH, H) - 1;
+  const float ftx0 = (float)tx0, fty0 = (float)ty0, ftx1 = (float)tx1, fty1 = (float)ty1;
+  const int mb = (wave / M::kCols) * 32, nb = (wave % M::kCols) * 32;
+  constexpr int kBlockX = 32 * M::kCols, kBlockY = 32 * M::kRows;  // from a wave's block to its next
   // operand reads: A[m][k] = Ey_k(ty0 + mb + m), B[k][n] = Ex_k(tx0 + nb + n); lane l holds row (column) l % 32,
   // k = 8 (l / 32) .. + 7 (v_mfma_f32_32x32x16 operand layout)
   const int a_at = mx_row(TW + mb + (lane & 31)) + 4 * (lane >> 5), b_at = mx_row(nb + (lane & 31)) + 4 * (lane >> 5);
@@ -443,7 +456,7 @@ __global__ __launch_bounds__(M::kThreads, 2) void beamlet_sum_sep_kernel(const S
   const int gk = t % M::KC, seg = t / M::KC;
   const bool y_axis = __builtin_amdgcn_readfirstlane(seg * kMxSeg) >= TW, odd = lane & 1;
   const double p0 = (double)(y_axis ? ty0 + seg * kMxSeg - TW : tx0 + seg * kMxSeg);
-  const double dtx0 = (double)tx0, dtx1 = (double)(tx0 + TW - 1);
+  const double dtx0 = (double)tx0, dtx1 = (double)tx1;
   const int dst_at = (gk / kMxK) * M::kStep + odd * M::kPart + mx_row(seg * kMxSeg) + (gk % kMxK) / 2;
   floatx16 re[M::BM][M::BN], im[M::BM][M::BN];
 #pragma unroll
@@ -452,58 +465,75 @@ __global__ __launch_bounds__(M::kThreads, 2) void beamlet_sum_sep_kernel(const S
     for (int k = 0; k < M::BN; ++k)
 #pragma unroll
       for (int j = 0; j < 16; ++j) re[i][k][j] = im[i][k][j] = 0.0f;
-  int exp_now = kNoExp;  // the sums are held times 2^(2 kMxScale - exp_now)
+  // A separable beamlet's cutoff ellipse is axis-aligned (alpha = 0): u^2 +
+  // gamma v^2 <= beta, so the tile's pixel centre nearest (cx, cy) decides,
+  // exactly, whether it meets the tile -- tiles in the corners of the ellipse's
+  // bounding box are skipped.
+  auto meets = [&](float4 c, float& du, float& dv) {  // cx, cy, gamma, beta
+    du = fmaxf(fmaxf(ftx0 - c.x, c.x - ftx1), 0.0f);
+    dv = fmaxf(fmaxf(fty0 - c.y, c.y - fty1), 0.0f);
+    return fmaf(c.z * dv, dv, du * du) <= c.w;
+  };
+  // The exponents of the slice's largest term in the tile and of the least that is to be kept.
+  int exp_now = kNoExp, low = -kNoExp;
+#pragma unroll 2
+  for (int64_t b = b_begin + t; b < b_end; b += kT) {
+    const float4 c = tab.cull[b];
+    const float2 p = tab.peak[b];
+    float du, dv;
+    if (!meets(c, du, dv)) continue;
+    // no term exceeds 2^top (the centre's f32 rounding taken off the distances)
+    du = fmaxf(fmaf(-0x1p-22f, fabsf(c.x), du), 0.0f);
+    dv = fmaxf(fmaf(-0x1p-22f, fabsf(c.y), dv), 0.0f);
+    const float top = ceilf(fmaf(p.y, fmaf(c.z * dv, dv, du * du), p.x));
+    // nor is any that is to be kept below 2^far: the pixel farthest from the centre, or the cut
+    du = fmaxf(c.x - ftx0, ftx1 - c.x);
+    dv = fmaxf(c.y - fty0, fty1 - c.y);
+    const float far = fmaxf(fmaf(p.y, fmaf(c.z * dv, dv, du * du), p.x), fmaf(p.y, c.w, p.x) + (float)kMxCutBits);
+    exp_now = max(exp_now, (int)fminf(fmaxf(top, -1e6f), 1e6f));
+    low = min(low, (int)(far >= -1e6f ? fminf(floorf(far), 1e6f) : -1e6f));
+  }
+  exp_now = wave_max_i32(exp_now);
+  low = -wave_max_i32(-low);
+  if (lane == 0) wave_cnt[wave] = exp_now, wave_low[wave] = low;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kW; ++w) {
+    exp_now = max(exp_now, wave_cnt[w]);
+    low = min(low, wave_low[w]);
+  }
+  exp_now = __builtin_amdgcn_readfirstlane(exp_now);
+  const bool leave = exp_now != kNoExp && low < exp_now - kMxRange;  // more than the halves hold
+  if (leave) {
+    const int32_t x = tx0 + (t & 1) * kTileW, y = ty0 + (t >> 1) * kTileH;
+    static_assert(TW == 2 * kTileW && TH == 2 * kTileH, "four tiles of beamlet_sum_wide_kernel");
+    if (t < 4 && x < W && y < H)
+      ws[((int64_t)split * H + y) * W + x] = make_float2(__int_as_float(kLeft), __int_as_float(exp_now));
+    return;
+  }
+  __syncthreads();  // wave_cnt is rewritten
+  // the sums are held times 2^(kMxScale - exp_now)
   for (int64_t blk = b_begin; blk < b_end; blk += kMxBlock) {
-    // the beamlets of [blk, blk + kMxBlock) whose cutoff ellipse meets the
-    // tile, in order.  A separable beamlet's ellipse is axis-aligned
-    // (alpha = 0): u^2 + gamma v^2 <= beta, so the tile's pixel centre nearest
-    // (cx, cy) decides, exactly -- tiles in the corners of the ellipse's
-    // bounding box are skipped.
-    int cnt = 0, exp_blk = kNoExp;
+    // the beamlets of [blk, blk + kMxBlock) that meet the tile, in order
+    int cnt = 0;
     for (int64_t b0 = blk; b0 < b_end && b0 < blk + kMxBlock; b0 += kT) {
       const int64_t b = b0 + t;
-      bool hit = false;
-      int top = kNoExp;
-      if (b < b_end) {
-        const float4 c = tab.cull[b];  // cx, cy, gamma, beta
-        const float2 p = tab.peak[b];
-        const float du = fmaxf(fmaxf(ftx0 - c.x, c.x - ftx1), 0.0f);
-        const float dv = fmaxf(fmaxf(fty0 - c.y, c.y - fty1), 0.0f);
-        hit = fmaf(c.z * dv, dv, du * du) <= c.w;
-        // no term of the beamlet in this tile exceeds 2^top (the centre's f32 rounding taken off the distances)
-        const float dus = fmaxf(fmaf(-0x1p-22f, fabsf(c.x), du), 0.0f), dvs = fmaxf(fmaf(-0x1p-22f, fabsf(c.y), dv), 0.0f);
-        if (hit) top = (int)fminf(fmaxf(ceilf(fmaf(p.y, fmaf(c.z * dvs, dvs, dus * dus), p.x)), -1e6f), 1e6f) + 1;
-      }
+      float du, dv;
+      const bool hit = b < b_end && meets(tab.cull[b], du, dv);
       const uint64_t mask = __ballot(hit);
-      top = wave_max_i32(top);
-      if (lane == 0) wave_cnt[wave] = __popcll(mask), wave_exp[wave] = top;
+      if (lane == 0) wave_cnt[wave] = __popcll(mask);
       __syncthreads();
       int off = cnt, total = 0;
 #pragma unroll
       for (int w = 0; w < kW; ++w) {
         off += (w < wave) ? wave_cnt[w] : 0;
         total += wave_cnt[w];
-        exp_blk = max(exp_blk, wave_exp[w]);
       }
       if (hit) list[off + __popcll(mask & ((1ull << lane) - 1ull))] = (int32_t)(b - blk);
       cnt += total;
       __syncthreads();  // wave_cnt is rewritten next; the list is complete after the last pass
     }
     if (cnt == 0) continue;
-    if (exp_blk > exp_now) {  // larger terms than so far: the sums move to their scale (an exact power of two)
-      if (exp_now != kNoExp) {
-#pragma unroll
-        for (int i = 0; i < M::BM; ++i)
-#pragma unroll
-          for (int k = 0; k < M::BN; ++k)
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-              re[i][k][j] = ldexpf(re[i][k][j], exp_now - exp_blk);
-              im[i][k][j] = ldexpf(im[i][k][j], exp_now - exp_blk);
-            }
-      }
-      exp_now = exp_blk;
-    }
     const int nch = (cnt + M::KC - 1) / M::KC;
     // chunk q's beamlet for this thread (past cnt: the last one again,
     // evaluated as zero), and the power of two its factor is multiplied by: an
@@ -518,7 +548,7 @@ __global__ __launch_bounds__(M::kThreads, 2) void beamlet_sum_sep_kernel(const S
       const double cen = y_axis ? x[3] : a.cen;
       const float du = (float)fmax(fmax(dtx0 - cen, cen - dtx1), 0.0);
       const float top = fmaxf(floorf(qx * du * du), -1e6f);
-      ex = (float)kMxScale + (y_axis ? top - (float)exp_now : -top);
+      ex = y_axis ? (float)kMxScaleY + top - (float)exp_now : (float)kMxScaleX - top;
       return a;
     };
     SepAxis v = load(0);
@@ -539,13 +569,13 @@ __global__ __launch_bounds__(M::kThreads, 2) void beamlet_sum_sep_kernel(const S
       for (int s = 0; s < S; ++s) {
 #pragma unroll
         for (int i = 0; i < M::BM; ++i) {
-          ar[s][i] = mx_load<M::kPart>(cur + s * M::kStep + a_at + i * kBlockRow);
-          ai[s][i] = mx_load<M::kPart>(cur + s * M::kStep + M::kPart + a_at + i * kBlockRow);
+          ar[s][i] = mx_load<M::kPart>(cur + s * M::kStep + a_at + mx_row(i * kBlockY));
+          ai[s][i] = mx_load<M::kPart>(cur + s * M::kStep + M::kPart + a_at + mx_row(i * kBlockY));
         }
 #pragma unroll
         for (int k = 0; k < M::BN; ++k) {
-          br[s][k] = mx_load<M::kPart>(cur + s * M::kStep + b_at + k * kBlockRow);
-          bi[s][k] = mx_load<M::kPart>(cur + s * M::kStep + M::kPart + b_at + k * kBlockRow);
+          br[s][k] = mx_load<M::kPart>(cur + s * M::kStep + b_at + mx_row(k * kBlockX));
+          bi[s][k] = mx_load<M::kPart>(cur + s * M::kStep + M::kPart + b_at + mx_row(k * kBlockX));
         }
       }
       // chunk c + 1's factors (past the last chunk: zeros nobody reads), and
@@ -579,12 +609,179 @@ __global__ __launch_bounds__(M::kThreads, 2) void beamlet_sum_sep_kernel(const S
     for (int k = 0; k < M::BN; ++k)
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
-        const int64_t py = ty0 + mb + 32 * i + 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
-        const int64_t px = tx0 + nb + 32 * k + (lane & 31);
+        const int64_t py = ty0 + mb + i * kBlockY + 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
+        const int64_t px = tx0 + nb + k * kBlockX + (lane & 31);
         if (py < H && px < W)
           ws[((int64_t)split * H + py) * W + px] =
-              make_float2(ldexpf(re[i][k][j], exp_now - 2 * kMxScale), ldexpf(im[i][k][j], exp_now - 2 * kMxScale));
+              make_float2(ldexpf(re[i][k][j], exp_now - kMxScale), ldexpf(im[i][k][j], exp_now - kMxScale));
       }
+}
+
+// ---------------------------------------------------------------------------
+// The same sum with f32 factors and products, for the slices and tiles that
+// beamlet_sum_sep_kernel leaves (marked in the tile's first pixel: kLeft and the
+// largest term's exponent), a 64x64 tile a workgroup, wave w the 32x32 block at
+// rows 32 (w / 2), columns 32 (w % 2).  |Ex| <= 1 and is at least exp(-80) at a
+// pixel that is to be kept; Ey, amplitude included, is taken up by the power of
+// two that brings the largest term to 2^10 (no visible value of Ey then exceeds
+// 2^126, as its beamlet's term is at most exp(80) below it), never down: what a
+// normal f32 holds of the field is held.  One k pair of the complex product is
+// three real products (Gauss): p1 += a.re b.re, p2 += a.im b.im, p3 += (a.re +
+// a.im)(b.re + b.im); then Re = p1 - p2 and Im = p3 - (p1 + p2).  Vector
+// instructions and f32 MFMAs of a SIMD do not execute together (their times
+// add), so the evaluation's instruction count is what it costs: one segment a
+// thread and chunk, a value between the products of each k pair.  (In one kernel
+// with the f16 products its registers spilled theirs.)  131,072 beamlets of 100
+// pixels on 1024^2, no cut: 7.98 ms; where every tile is left out, 8 us for the
+// workgroups of such an image, 1 us for a small one's.
+// ---------------------------------------------------------------------------
+constexpr int kWideScale = 10;
+constexpr int kWideBlock = 2048;          // beamlets per list build
+constexpr int kWideK = 32;                // beamlets per LDS chunk (the product's K)
+constexpr int kWideRow = kTileW + 1;      // LDS row pitch (float2): a bank offset per beamlet row
+static_assert(kTileW == 64 && kTileH == 64 && kThreads == 256 && kWideK * 2 * (kTileW / kMxSeg) == kThreads &&
+                  kMxSeg == kWideK / 2,
+              "64x64 tiles, four waves, one segment per thread and one segment value per k pair");
+
+__device__ __forceinline__ void wide_mfma(float2 a, float2 b, floatx16& p1, floatx16& p2, floatx16& p3) {
+  p1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, p1, 0, 0, 0);
+  p2 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, p2, 0, 0, 0);
+  p3 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x + a.y, b.x + b.y, p3, 0, 0, 0);
+}
+
+__global__ __launch_bounds__(kThreads) void beamlet_sum_wide_kernel(const SepTables tab, int64_t n, int64_t H,
+                                                                    int64_t W, int32_t ntx, int32_t nsplit,
+                                                                    const int32_t* __restrict__ flags,
+                                                                    float2* __restrict__ ws) {
+  __shared__ int32_t list[kWideBlock];
+  __shared__ int32_t wave_cnt[kWaves];
+  __shared__ float2 fac[2][2][kWideK][kWideRow];  // [buffer][x: Ex_k(tx0 + n), y: Ey_k(ty0 + m)][k][pixel]
+  const int split = blockIdx.x % nsplit, tile = blockIdx.x / nsplit;
+  const int32_t tx0 = (tile % ntx) * kTileW, ty0 = (tile / ntx) * kTileH;
+  const float2 mark = ws[((int64_t)split * H + ty0) * W + tx0];
+  if (__float_as_int(mark.x) != kLeft) return;  // beamlet_sum_sep_kernel's
+  if (!matrix_path(flags)) return;              // beamlet_sum_kernel covers this launch (the mark is an older one's)
+  const int exp_now = __float_as_int(mark.y);
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int64_t b_begin = n * split / nsplit, b_end = n * (split + 1) / nsplit;
+  const int32_t tx1 = (int32_t)min((int64_t)tx0 + kTileW, W) - 1, ty1 = (int32_t)min((int64_t)ty0 + kTileH, H) - 1;
+  const float ftx0 = (float)tx0, fty0 = (float)ty0, ftx1 = (float)tx1, fty1 = (float)ty1;
+  const int mb = (wave >> 1) * 32, nb = (wave & 1) * 32;
+  // this thread's segment: beamlet gk of a chunk, axis (waves 0-1: x, 2-3: y), pixels p0 .. p0 + 15
+  const int gk = t & (kWideK - 1), s0 = ((t >> 5) & 3) * kMxSeg;
+  const bool y_axis = __builtin_amdgcn_readfirstlane(t >> 7) != 0;
+  const double p0 = (double)((y_axis ? ty0 : tx0) + s0);
+  const double* axis = y_axis ? tab.y : tab.x;
+  const int axis_step = y_axis ? 5 : 4;
+  const int scale = max(kWideScale - exp_now, 0);
+  const float ex = y_axis ? (float)scale : 0.0f;
+  floatx16 p1, p2, p3;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) p1[j] = p2[j] = p3[j] = 0.0f;
+  for (int64_t blk = b_begin; blk < b_end; blk += kWideBlock) {
+    const int64_t end = min(b_end, blk + kWideBlock);
+    int cnt = 0;
+    for (int64_t b0 = blk; b0 < end; b0 += kThreads) {
+      const int64_t b = b0 + t;
+      bool hit = false;
+      if (b < end) {
+        const float4 c = tab.cull[b];  // cx, cy, gamma, beta
+        const float du = fmaxf(fmaxf(ftx0 - c.x, c.x - ftx1), 0.0f);
+        const float dv = fmaxf(fmaxf(fty0 - c.y, c.y - fty1), 0.0f);
+        hit = fmaf(c.z * dv, dv, du * du) <= c.w;
+      }
+      const uint64_t mask = __ballot(hit);
+      if (lane == 0) wave_cnt[wave] = __popcll(mask);
+      __syncthreads();
+      int off = cnt, total = 0;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        off += (w < wave) ? wave_cnt[w] : 0;
+        total += wave_cnt[w];
+      }
+      if (hit) list[off + __popcll(mask & ((1ull << lane) - 1ull))] = (int32_t)(b - blk);
+      cnt += total;
+      __syncthreads();  // wave_cnt is rewritten next; the list is complete after the last pass
+    }
+    if (cnt == 0) continue;
+    // chunk q's beamlet for this thread (past cnt: the last one again, evaluated
+    // as zero): load_sep without a branch, which the loads in flight would wait at
+    auto load = [&](int q) -> SepAxis {
+      const double* a = axis + axis_step * (blk + list[min(q * kWideK + gk, cnt - 1)]);
+      const double c0 = a[3];
+      return {__int_as_float(__double2loint(a[0])), __int_as_float(__double2hiint(a[0])), a[1], a[2], y_axis ? c0 : 0.0,
+              a[axis_step - 1]};
+    };
+    SepAxis v = load(0);
+    {
+      SegGen sg = seg_setup(v, p0, ex, gk < cnt, false);
+      v = load(1);
+      float2* dst = &fac[0][y_axis][gk][s0];
+#pragma unroll
+      for (int j = 0; j < kMxSeg; ++j) dst[j] = seg_next(sg, j);
+    }
+    __syncthreads();
+    const int nch = (cnt + kWideK - 1) / kWideK;
+    for (int c = 0; c < nch; ++c) {
+      // A[m][k] = Ey_k(ty0 + mb + m) from lane m + 32 k, B[k][n] = Ex_k(tx0 + nb + n) from lane n + 32 k
+      // (v_mfma_f32_32x32x2f32 operand layout); operands one k pair ahead, so LDS latency hides behind the products
+      const float2* ea = &fac[c & 1][1][lane >> 5][mb + (lane & 31)];
+      const float2* eb = &fac[c & 1][0][lane >> 5][nb + (lane & 31)];
+      float2 a = ea[0], b = eb[0];
+      if (c + 1 < nch) {
+        // chunk c + 1's factors beside the products, and chunk c + 2's parameters in flight
+        SegGen sg = seg_setup(v, p0, ex, (c + 1) * kWideK + gk < cnt, false);
+        v = load(c + 2);
+        // (kept here: sunk below the products, the next chunk waited a memory round trip)
+        __builtin_amdgcn_sched_barrier(0);
+        // (stored after the products: a store between them would order every later operand read behind it)
+        float2 val[kMxSeg];
+#pragma unroll
+        for (int kk = 0; kk < kWideK; kk += 2) {
+          float2 an = a, bn = b;
+          if (kk + 2 < kWideK) {
+            an = ea[(kk + 2) * kWideRow];
+            bn = eb[(kk + 2) * kWideRow];
+          }
+          wide_mfma(a, b, p1, p2, p3);
+          val[kk >> 1] = seg_next(sg, kk >> 1);
+          a = an;
+          b = bn;
+          // issue order: products and the value's dependent vector instructions alternate
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
+            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // four VALU
+          }
+        }
+        float2* dst = &fac[(c & 1) ^ 1][y_axis][gk][s0];
+#pragma unroll
+        for (int j = 0; j < kMxSeg; ++j) dst[j] = val[j];
+      } else {
+#pragma unroll
+        for (int kk = 0; kk < kWideK; kk += 2) {
+          float2 an = a, bn = b;
+          if (kk + 2 < kWideK) {
+            an = ea[(kk + 2) * kWideRow];
+            bn = eb[(kk + 2) * kWideRow];
+          }
+          wide_mfma(a, b, p1, p2, p3);
+          a = an;
+          b = bn;
+        }
+      }
+      __syncthreads();  // chunk c + 1 is complete and chunk c read
+    }
+  }
+  // accumulator j of lane l holds row 8 (j / 4) + 4 (l / 32) + j % 4, column l % 32
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const int64_t py = ty0 + mb + 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
+    const int64_t px = tx0 + nb + (lane & 31);
+    if (py < H && px < W)
+      ws[((int64_t)split * H + py) * W + px] =
+          make_float2(ldexpf(p1[j] - p2[j], -scale), ldexpf(p3[j] - (p1[j] + p2[j]), -scale));
+  }
 }
 
 // The slices' sum, in order.  Bound: reading them; four loads in flight hide
@@ -760,21 +957,32 @@ int splits_for(int64_t n, int64_t H, int64_t W) {
   // 212; 131,072 on 1024^2: 16 / 32 / 64 / 128 slices 2.50 / 2.15 / 2.15 /
   // 2.30 ms; 50,000 on 1000 x 300 533 / 468 us.
   const int64_t few = std::min<int64_t>(6LL * tg::cu_count() / ntiles, (int64_t)std::sqrt((double)n));
-  const int64_t sep_tiles = tg::cdiv(H, (int64_t)SepTile::TH) * tg::cdiv(W, (int64_t)SepTile::TW);
+  const int64_t tiles = tg::cdiv(H, (int64_t)SepTile::TH) * tg::cdiv(W, (int64_t)SepTile::TW);
   const int64_t slots = 2LL * tg::cu_count();
-  const int64_t rounds = std::min<int64_t>(4, (int64_t)((double)n * (double)sep_tiles / (600.0 * (double)slots)));
-  int64_t s = std::max(few, rounds * slots / sep_tiles);
+  const int64_t rounds = std::min<int64_t>(4, (int64_t)((double)n * (double)tiles / (600.0 * (double)slots)));
+  int64_t s = std::max(few, rounds * slots / tiles);
   if (s > 128) s = 128;
   if (s < 1) s = 1;
   return (int)s;
 }
 
-template <class M>
-void launch_sep_sum(const SepTables& tab, int64_t n, int64_t H, int64_t W, int nsplit, const int32_t* flags, float2* ws,
-                    hipStream_t s) {
-  const int64_t ntx = tg::cdiv(W, (int64_t)M::TW), ntiles = ntx * tg::cdiv(H, (int64_t)M::TH);
-  hipLaunchKernelGGL(beamlet_sum_sep_kernel<M>, dim3((unsigned)(ntiles * nsplit)), dim3(M::kThreads), 0, s, tab, n, H,
-                     W, (int32_t)ntx, (int32_t)nsplit, flags, ws);
+int64_t sep_tiles(int64_t H, int64_t W) {
+  return tg::cdiv(W, (int64_t)SepTile::TW) * tg::cdiv(H, (int64_t)SepTile::TH);
+}
+
+// The two sums of separable beamlets: the f16 halves, then the f32 products of
+// what they leave.
+int launch_sep_sums(const SepTables& tab, int64_t n, int64_t H, int64_t W, int nsplit, const int32_t* flags,
+                    float2* ws, hipStream_t s) {
+  hipLaunchKernelGGL(beamlet_sum_sep_kernel<SepTile>, dim3((unsigned)(sep_tiles(H, W) * nsplit)),
+                     dim3(SepTile::kThreads), 0, s, tab, n, H, W, (int32_t)tg::cdiv(W, (int64_t)SepTile::TW),
+                     (int32_t)nsplit, flags, ws);
+  TG_LAUNCH_CHECK("beamlet_sum_sep_kernel launch");
+  const int64_t ntx = tg::cdiv(W, (int64_t)kTileW), ntiles = ntx * tg::cdiv(H, (int64_t)kTileH);
+  hipLaunchKernelGGL(beamlet_sum_wide_kernel, dim3((unsigned)(ntiles * nsplit)), dim3(kThreads), 0, s, tab, n, H, W,
+                     (int32_t)ntx, (int32_t)nsplit, flags, ws);
+  TG_LAUNCH_CHECK("beamlet_sum_wide_kernel launch");
+  return TG_OK;
 }
 
 // The recurrence tile sum (beamlet_sum_kernel) for a tile shape
@@ -886,12 +1094,12 @@ extern "C" int tg_beamlet_sum(const tg_beamlet_coef* coef, int64_t n, int64_t he
   int32_t* flags = (int32_t*)((char*)workspace + slices);
   const SepTables tab = sep_tables(flags + kFlagBlocks, n);
   // which tile sum runs is decided on the device (no host round trip, so the
-  // call stays graph-capturable); the other kernel's workgroups exit at once
+  // call stays graph-capturable); the other kernels' workgroups exit at once
   hipLaunchKernelGGL(sep_flag_kernel, dim3(kFlagBlocks), dim3(256), 0, (hipStream_t)stream, coef, n,
                      (int32_t)(path == TG_BEAMLET_PATH_VALU), flags, tab);
   TG_LAUNCH_CHECK("sep_flag_kernel launch");
-  launch_sep_sum<SepTile>(tab, n, height, width, nsplit, flags, (float2*)workspace, (hipStream_t)stream);
-  TG_LAUNCH_CHECK("beamlet_sum_sep_kernel launch");
+  st = launch_sep_sums(tab, n, height, width, nsplit, flags, (float2*)workspace, (hipStream_t)stream);
+  if (st != TG_OK) return st;
   int32_t shape = TG_TILE_64x64_RUN16;
   tg::tune_lookup(TG_TUNE_TILE_SHAPE, key, shape);
   st = launch_recurrence_sum(shape, coef, n, height, width, nsplit, flags, (float2*)workspace, (hipStream_t)stream);
