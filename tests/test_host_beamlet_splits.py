@@ -20,3 +20,16 @@ def test_slices_are_bounded(seed):
             low = slices - 255
             nsplit = [s for s in range(1, 129) if low <= s * h * w * 8 <= slices]
             assert nsplit and nsplit[0] <= max(k, 1)
+
+
+@pytest.mark.parametrize("n,height,width,most", [
+    (1, 600, 612, 1), (30, 1024, 1024, 1), (64, 600, 612, 1), (300, 600, 600, 2), (2000, 1024, 1024, 4),
+    (64, 64, 64, 8), (300, 100, 100, 17),
+])
+def test_a_slice_of_a_large_image_has_beamlets_enough(n, height, width, most):
+    """A slice of ten thousand pixels or fewer: sqrt(n) beamlets and more; of
+    larger images as many more as makes up for its partial image."""
+    lib = _lib.load()
+    autotune.clear()
+    slices = lib.tg_beamlet_sum_workspace(n, height, width) - 256 * 4 - 96 * n
+    assert slices <= -(-most * height * width * 8 // 256) * 256
