@@ -195,7 +195,6 @@ class ColumnMatch:
         # outputs share one allocation, each on a 16-byte boundary
         size = 4 if f32 else 8
         self.row = -(-col.n // (16 // size)) * (16 // size)
-        self.row_bytes = self.row * size
         # immediates rounded once to the ray dtype, as in register programs
         num = (lambda v: float(np.float32(v))) if f32 else float
         col.pathlength = num(path0)

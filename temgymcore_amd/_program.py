@@ -774,7 +774,8 @@ def build_plan(trace: Trace, sym_ray, bin_request=None, extra_rays=(), sym_in=No
         groups.setdefault(bin_shape, [])
         keep = kv
     if column is not None:
-        buf, results = _column_outputs(column, trace.device)
+        results = {v: torch.empty(column.shape, dtype=column.dtype, device=trace.device)
+                   for v in column.out_vids if v is not None}
         programs = lambda: _compile_programs(trace, groups, bin_request, bin_shape, keep, results)[0]  # noqa: E731
     else:
         programs, results = _compile_programs(trace, groups, bin_request, bin_shape, keep)
@@ -827,16 +828,17 @@ def _run_column(lib, col, spec, ws_bytes: int, device, stream) -> int:
     return lib.tg_ray_column_run(ctypes.byref(col), ctypes.byref(spec), ws.data_ptr(), ws_bytes, stream)
 
 
-def _column_outputs(column, device):
-    """One allocation for a column's outputs, every row on a 16-byte boundary
-    (the kernel's wide stores): (buffer [rows, row], value id -> tensor)."""
-    vids = [v for v in column.out_vids if v is not None]
-    n = column.struct.n
-    buf = torch.empty((len(vids), column.row), dtype=column.dtype, device=device)
-    rows = (buf if column.row == n else buf.narrow(1, 0, n)).unbind(0)
-    if len(column.shape) != 1:
-        rows = [r.view(column.shape) for r in rows]
-    return buf, dict(zip(vids, rows))
+def _arrays(count: int, shape: tuple, dtype, device, row: int | None = None) -> list:
+    """`count` fresh arrays of a shape, vectors in one allocation, `row` elements
+    apart.  Each is a tensor of its own to autograd (no views, no common
+    version): a result may be changed in place whatever another was used for."""
+    if len(shape) != 1 or count == 1:
+        return [torch.empty(shape, dtype=dtype, device=device) for _ in range(count)]
+    n = shape[0]
+    if row is None or row == n:
+        return list(torch.unsafe_split_with_sizes(torch.empty(count * n, dtype=dtype, device=device), [n] * count))
+    buf = torch.empty(count * row, dtype=dtype, device=device)
+    return list(torch.unsafe_split_with_sizes(buf, [n, row - n] * count)[::2])
 
 
 def _materialize(trace: Trace, sym_ray, bin_request=None):
@@ -1073,8 +1075,7 @@ class _PlanTemplate:
     def bind(self, leaves: list, acc: torch.Tensor | None):
         """Copies of the programs with this call's arrays and fresh outputs
         bound: ([(Program, BinSpec | None)], output ray, (inputs, outputs)).
-        The outputs of one program that share a shape and dtype are views of
-        one allocation."""
+        The vectors that one program stores in one dtype share an allocation."""
         dev = self.device
         inputs: dict[int, torch.Tensor] = {}
         outs: dict[int, torch.Tensor] = {}
@@ -1093,11 +1094,7 @@ class _PlanTemplate:
             for k, (kind, x) in enumerate(binds):
                 slots[k].ptr = (input_tensor(x) if kind == "leaf" else outs[x]).data_ptr()
             for (shape, dt), members in groups:
-                if len(members) == 1:
-                    views = (torch.empty(shape, dtype=dt, device=dev),)
-                else:
-                    views = torch.empty((len(members),) + shape, dtype=dt, device=dev).unbind(0)
-                for (k, vid), o in zip(members, views):
+                for (k, vid), o in zip(members, _arrays(len(members), shape, dt, dev)):
                     outs[vid] = o
                     prog.out[k] = o.data_ptr()
             spec = None
@@ -1129,12 +1126,11 @@ class _PlanTemplate:
                 ptrs[k] = inputs[i].data_ptr()
         outs = {}
         if match.n_out:
-            buf, outs = _column_outputs(match, dev)
-            at, ptrs = buf.data_ptr(), col.out
+            arrays, ptrs = iter(_arrays(match.n_out, match.shape, match.dtype, dev, match.row)), col.out
             for k, v in enumerate(match.out_vids):
                 if v is not None:
-                    ptrs[k] = at
-                    at += match.row_bytes
+                    outs[v] = o = next(arrays)
+                    ptrs[k] = o.data_ptr()
         spec = None
         if spec_t is not None:
             spec = _lib.BinSpec.from_buffer_copy(spec_t)
