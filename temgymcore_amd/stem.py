@@ -301,9 +301,9 @@ def backproject(model: STEMModel, data4d: torch.Tensor, params: torch.Tensor | N
     if tuple(data4d.shape) != shape or data4d.dtype != torch.float32 or not data4d.is_cuda:
         raise ValueError(f"data4d must be a device float32 tensor of shape {shape}")
     data4d = data4d.contiguous()
-    # (both cleared by one launch)
-    sums = torch.zeros((2 if weights else 1,) + tuple(model.sample_shape), dtype=torch.float64, device=device)
-    image, weight = sums[0], sums[1] if weights else None
+    # (two tensors: halves of one buffer would share its version and its memory)
+    image = torch.zeros(tuple(model.sample_shape), dtype=torch.float64, device=device)
+    weight = torch.zeros_like(image) if weights else None
     g = model.geometry()
     st = _lib.load().tg_stem_backproject(ctypes.byref(g), params.data_ptr(), data4d.data_ptr(), int(cam),
                                          image.data_ptr(), _ptr(weight), _lib.stream_ptr(device))
