@@ -669,11 +669,13 @@ class Plan:
 
     Launching re-runs the same kernels on the same input and output buffers
     (inputs may be refilled in place between launches).  ``launch()`` costs one
-    C call per program, so a plan is also what a HIP graph capture records.
+    C call per program and takes no memory, so a plan is also what a HIP graph
+    capture records, whoever began it.
 
     A model that is a column of standard elements launches its ``column``
-    (tg_ray_column_run); ``programs``, the register programs of the same model,
-    are then compiled when first asked for.
+    (tg_ray_column_run) with the ``workspace`` that its binning takes;
+    ``programs``, the register programs of the same model, are then compiled
+    when first asked for.
     """
 
     def __init__(self, trace: Trace, programs, out_ray, acc=None):
@@ -683,6 +685,7 @@ class Plan:
         self.acc = acc
         self.extra_out: list = []
         self.column = None  # (Column, BinSpec | None, ColumnMatch)
+        self.workspace = None  # (tensor, the stream it was taken on)
 
     @property
     def programs(self) -> list:
@@ -695,8 +698,10 @@ class Plan:
         st = _lib.stream_ptr(self.trace.device) if stream is None else stream
         if self.column is not None:
             col, spec, _ = self.column
-            _lib.check(_run_column(lib, col, spec, _column_workspace(lib, col, spec), self.trace.device, st),
-                       "tg_ray_column_run")
+            ws, home = self.workspace or (None, st)
+            if st != home:  # (a plan may be dropped while another stream still counts)
+                ws.record_stream(torch.cuda.ExternalStream(st, device=self.trace.device))
+            _lib.check(_run_column(lib, col, spec, ws, st), "tg_ray_column_run")
             return self.out_ray
         for prog, spec, _ in self.programs:
             status = lib.tg_ray_program_run(ctypes.byref(prog), ctypes.byref(spec) if spec is not None else None, st)
@@ -806,6 +811,10 @@ def build_plan(trace: Trace, sym_ray, bin_request=None, extra_rays=(), sym_in=No
                 col.out[k] = results[column.out_vids[k]].data_ptr()
         plan.column = (col, None if bin_request is None else bin_request[0], column)
         plan.recipe = (groups, bin_request, bin_shape, keep)
+        if bin_request is not None and trace.device.type == "cuda":
+            size = _column_workspace(_lib.load(), col, plan.column[1])
+            if size:
+                plan.workspace = _column_scratch(size, trace.device), _lib.stream_ptr(trace.device)
     return plan
 
 
@@ -814,18 +823,14 @@ def _column_workspace(lib, col, spec) -> int:
     return 0 if spec is None else lib.tg_ray_column_workspace(col.n, spec.height, spec.width, spec.acc_dtype)
 
 
-def _run_column(lib, col, spec, ws_bytes: int, device, stream) -> int:
-    """Launch a column; its scratch memory comes from torch's stream-ordered
-    allocator (on the launch's stream) and is given back once the launch is
-    enqueued."""
-    if not ws_bytes:
-        return lib.tg_ray_column_run(ctypes.byref(col), None if spec is None else ctypes.byref(spec), None, 0, stream)
-    if stream == _lib.stream_ptr(device):
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
-    else:
-        with torch.cuda.stream(torch.cuda.ExternalStream(stream, device=device)):
-            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
-    return lib.tg_ray_column_run(ctypes.byref(col), ctypes.byref(spec), ws.data_ptr(), ws_bytes, stream)
+def _column_scratch(size: int, device) -> torch.Tensor:
+    return torch.empty(size, dtype=torch.uint8, device=device)
+
+
+def _run_column(lib, col, spec, ws, stream) -> int:
+    """Launch a column with the scratch memory `ws` (None: none)."""
+    return lib.tg_ray_column_run(ctypes.byref(col), None if spec is None else ctypes.byref(spec),
+                                 None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), stream)
 
 
 def _arrays(count: int, shape: tuple, dtype, device, row: int | None = None) -> list:
@@ -1138,7 +1143,16 @@ class _PlanTemplate:
         lib = _lib.load()
         if ws_bytes is None:
             ws_bytes = self.column[3] = _column_workspace(lib, col, spec)
-        st = _run_column(lib, col, spec, ws_bytes, dev, stream)
+        ws = None
+        if ws_bytes:
+            # from torch's stream-ordered allocator, on the launch's stream, and
+            # given back once the launch is enqueued
+            if stream == _lib.stream_ptr(dev):
+                ws = _column_scratch(ws_bytes, dev)
+            else:
+                with torch.cuda.stream(torch.cuda.ExternalStream(stream, device=dev)):
+                    ws = _column_scratch(ws_bytes, dev)
+        st = _run_column(lib, col, spec, ws, stream)
         if st != 0:
             _lib.check(st, "tg_ray_column_run")
         vals = {}
