@@ -664,6 +664,9 @@ def prepare(trace: Trace, comp: Compiled, bin_spec: _lib.BinSpec | None = None, 
     return prog, outs, keep
 
 
+_COMPILE_LOCK = threading.Lock()  # programs compiled when first asked for
+
+
 class Plan:
     """A traced and compiled model application, ready to launch repeatedly.
 
@@ -690,7 +693,9 @@ class Plan:
     @property
     def programs(self) -> list:
         if callable(self._programs):
-            self._programs = self._programs()
+            with _COMPILE_LOCK:  # (the trace takes one compilation)
+                if callable(self._programs):
+                    self._programs = self._programs()
         return self._programs
 
     def launch(self, stream: int | None = None):
@@ -1074,7 +1079,9 @@ class _PlanTemplate:
     @property
     def programs(self) -> list:
         if callable(self._programs):
-            self._programs = self._programs()
+            with _COMPILE_LOCK:  # (the trace takes one compilation)
+                if callable(self._programs):
+                    self._programs = self._programs()
         return self._programs
 
     def bind(self, leaves: list, acc: torch.Tensor | None):
