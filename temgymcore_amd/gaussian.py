@@ -674,6 +674,8 @@ def make_gaussian_image(gaussian_rays: GaussianRay, model, batch_size=128, cutof
     n = int(params.shape[0])
     if mat is not None:
         abcd, stride = mat, 0
+    elif matrix is not None:
+        abcd, stride = torch.from_numpy(matrix[None]).to(device), 0
     elif abcd is None:
         abcd, stride = _abcd_per_beamlet(rays, model, device, n)
     else:
