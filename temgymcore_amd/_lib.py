@@ -169,6 +169,12 @@ def check(status: int, what: str) -> None:
     raise RuntimeError(f"{what}: {msg}")
 
 
+# Lookups without the public functions' checks and objects; those serve where a
+# torch has not got these.
+_get_device = getattr(torch._C, "_cuda_getDevice", None)
+_get_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 @functools.lru_cache(maxsize=None)
 def _device(index: int) -> torch.device:
     return torch.device("cuda", index)
@@ -176,8 +182,8 @@ def _device(index: int) -> torch.device:
 
 def require_device() -> torch.device:
     """The HIP device vectorised work runs on (torch's current device)."""
-    if torch.cuda.is_initialized():
-        return _device(torch._C._cuda_getDevice())
+    if _get_device is not None and torch.cuda.is_initialized():
+        return _device(_get_device())
     if not torch.cuda.is_available():
         raise RuntimeError(
             "temgymcore_amd: vectorised rays run on the MI355X HIP kernels and need a GPU; "
@@ -189,7 +195,7 @@ def require_device() -> torch.device:
 def stream_ptr(device: torch.device | None = None) -> int:
     """Raw hipStream_t of torch's current stream on `device` (without the
     Stream object that torch.cuda.current_stream makes: 0.1 us for 1.8)."""
-    if not torch.cuda.is_initialized():
+    if _get_raw_stream is None or not torch.cuda.is_initialized():
         return torch.cuda.current_stream(device).cuda_stream
     index = None if device is None else device.index
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice() if index is None else index)
+    return _get_raw_stream(torch.cuda.current_device() if index is None else index)

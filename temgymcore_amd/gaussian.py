@@ -274,11 +274,15 @@ _COLUMN_TYPE = {torch.float32: 1, torch.float64: 2, torch.complex64: 1, torch.co
 
 def _no_transform() -> bool:
     """No tracer, vmap, forward-mode level or dispatch mode sees this call:
-    those follow the torch operations of ``pack_params``."""
+    those follow the torch operations of ``pack_params``.  (Asked of torch's
+    internals; a torch without one of them takes those operations too.)"""
     C = torch._C
-    return (C._functorch.peek_interpreter_stack() is None and C._len_torch_dispatch_stack() == 0
-            and C._len_torch_function_stack() == 0 and torch.autograd.forward_ad._current_level < 0
-            and C._get_tracing_state() is None and not torch.compiler.is_compiling())
+    try:
+        return (C._functorch.peek_interpreter_stack() is None and C._len_torch_dispatch_stack() == 0
+                and C._len_torch_function_stack() == 0 and torch.autograd.forward_ad._current_level < 0
+                and C._get_tracing_state() is None and not torch.compiler.is_compiling())
+    except AttributeError:
+        return False
 
 
 def _device_column(v, n: int, device, complex_: bool = False):
