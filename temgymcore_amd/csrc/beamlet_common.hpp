@@ -529,10 +529,8 @@ struct RowTerms {
   double lre, lim, cre, cim;
 };
 
-// The moments of pixels xs .. xs + cnt of a row (cnt < kRun; WHOLE: all kRun)
-// with weights w, added to M: v = row - pcy, ub = xs - pcx.  f32 within the run,
-// f64 across runs.
-template <bool WHOLE>
+// The moments of pixels xs .. xs + cnt of a row (cnt < kRun) with weights w,
+// added to M: v = row - pcy, ub = xs - pcx.  f32 within the run, f64 across runs.
 __device__ __forceinline__ void run_moments(const tg_beamlet_coef& c, const RowTerms& r, int32_t xs, int32_t cnt,
                                             const float2 (&w)[kRun], double ub, double v, double (&M)[kMoments]) {
   const double px = (double)xs, px2 = 2.0 * px + 1.0;
@@ -545,7 +543,7 @@ __device__ __forceinline__ void run_moments(const tg_beamlet_coef& c, const RowT
 #pragma unroll
   for (int k = 0; k < kRun; ++k) {
     float2 P = cmulf(w[k], F);
-    if (!WHOLE && k > 0) {
+    if (k > 0) {
       const bool on = k <= cnt;
       P.x = on ? P.x : 0.0f;
       P.y = on ? P.y : 0.0f;
@@ -585,15 +583,16 @@ __device__ __forceinline__ void run_moments(const tg_beamlet_coef& c, const RowT
 // with E = exp(Phi_c), (u, v) = pixel offsets from centre_pixel(c).  `wbase`
 // needs kRun readable elements past the image (tail padding).
 //
-// Bound: vector issue and the power it draws (18 instructions a pixel of a
-// whole run, 21 of a cut one, about 70 a run).  So a lane keeps a row, whose
-// extent and terms of Phi it makes once, and walks its 16-pixel runs column by
-// column (fewer than 64 rows: the wavefront takes several columns at a time):
-// the runs inside the ellipse are then whole for all lanes at once.
-// 76,000 Gaussians on 256 images of 128^2 to 512^2 pixels: 2.69 ms with the runs
-// dealt to the lanes in turn, 2.34 so; 9,000 beamlets on 600^2 257 / 238 us with
-// the rest of their backward; 4,096 on 600 x 612 with a 4-sigma cut, whose few
-// rows fill the lanes less well, 59 / 68.
+// Bound: vector issue and the power it draws (21 instructions a pixel, about 70
+// a run).  So a lane keeps a row, whose extent and terms of Phi it makes once,
+// and walks its 16-pixel runs column by column (fewer than 64 rows: the
+// wavefront takes several columns at a time).  Runs dealt to the lanes in turn /
+// this: 76,000 Gaussians on 256 images of 128^2 to 512^2 pixels 2.94 / 2.61 ms,
+// 9,000 beamlets on 600^2 246 / 219 us; where few rows fill the lanes less well,
+// 4,096 on 600 x 612 with a 4-sigma cut 32 / 36, 76,800 Gaussians of 1 to 3
+// pixels 161 / 180.  (A second form without selects for runs that are whole in
+// every lane takes 18 instructions a pixel, but 145 registers in place of 124,
+// three wavefronts a SIMD: 2.49 ms for the first, 215 us for the last.)
 template <int WAVES>
 __device__ inline void beamlet_moments(const tg_beamlet_coef& c, int32_t H, int32_t W,
                                        const float2* __restrict__ wbase, int t, double (&M)[kMoments]) {
@@ -647,10 +646,7 @@ __device__ inline void beamlet_moments(const tg_beamlet_coef& c, int32_t H, int3
       // keep all 16 loads ahead of the math: one memory round trip per run
       __builtin_amdgcn_sched_barrier(0);
       const double ub = (double)xs - (double)pcx;
-      if (__ballot(xe - xs != kRun - 1) == 0)
-        run_moments<true>(c, r, xs, kRun - 1, w, ub, v, M);
-      else
-        run_moments<false>(c, r, xs, xe - xs, w, ub, v, M);
+      run_moments(c, r, xs, xe - xs, w, ub, v, M);
     }
   }
 }
@@ -685,11 +681,9 @@ __device__ __forceinline__ void block_moments(const tg_beamlet_coef& c, int32_t 
 
 // Whether four wavefronts share a beamlet's moments: where one each would not
 // give every SIMD four, and the time is that of a beamlet's runs one after the
-// other.  One wavefront / four, backward of 64 beamlets on 500 x 612 pixels 59 /
-// 36 us, 300 on 200^2 53 / 37, 2,048 on 500 x 612 76 / 75, 4,096 on 300^2 122 /
-// 113, 4,096 on 600 x 612 with a 4-sigma cut (few runs each) 68 / 75; a fit of
-// two images, 100 Gaussians, 151 / 89.  Sixteen wavefronts are 1 to 7 us better
-// for the smallest of these and slower from 300 beamlets on.
+// other.  One wavefront / four: 64 beamlets on 500 x 612 pixels 51 / 18 us, 300 on
+// 200^2 40 / 18, 2,048 on 500 x 612 71 / 58; a fit of two images, 100 Gaussians,
+// 197 / 57.
 inline bool share_moments(int64_t n) { return n < 16LL * tg::cu_count(); }
 
 }  // namespace tgb
