@@ -325,7 +325,7 @@ __global__ __launch_bounds__(kThreads) void stem_forward_kernel(const tg_stem_ge
 // the ray rows that can reach the band are visited: the detector row is
 // monotone in the slope row, so they are one range, found from each row's two
 // end columns.  One wavefront sets the position up for all, once for all of
-// the workgroup's bands.  64x64 positions of 256x256 pixels, 64x64 rays:
+// the workgroup's bands (a few positions are shared by several workgroups).  64x64 positions of 256x256 pixels, 64x64 rays:
 // 193 us (5.6 TB/s of writes; 379 us cleared by a fill and deposited with
 // 16.7M global atomics).  The same without any rays takes 189 us: what is left
 // above the 147 us of a plain fill is the set-up at the start of each round of
@@ -333,18 +333,28 @@ __global__ __launch_bounds__(kThreads) void stem_forward_kernel(const tg_stem_ge
 // band a workgroup 288, two 230, four 207 us; bands of 12/16/24/30 KB
 // 214/210/196/198 us; a first band that differs from position to position
 // 207-219 us; non-temporal stores 196 us.
+// Cleared and deposited / this, whole calls: 64x64 positions of 70x201 pixels,
+// 30^2 rays 62 / 50 us, of 128^2 87 / 52; 31x33 of 70x201, 40^2 rays 23 / 23.  LDS
+// adds floats at half a lane a cycle (58 us for 16.7M), memory faster where every
+// ray has a pixel of its own, and far slower where rays share them: 64x64
+// positions, 64^2 rays on 100x130 pixels 107 / 119, 40^2 rays on 64^2 51 / 59, 64^2
+// rays on 64^2 316 / 119.
 constexpr int kBandFloats = 6144;
+
+// float4s of LDS for a band of npix pixels, wherever in its first 16 bytes it begins
+__host__ __device__ inline int band_quads(int npix) { return (npix + 6) / 4; }
 
 __global__ __launch_bounds__(kThreads) void stem_dataset_kernel(const tg_stem_geometry G, const double* __restrict__ P,
                                                                 const float* __restrict__ img, int band_rows,
                                                                 int bands_each, float* __restrict__ image4d) {
-  __shared__ float th[kMaxSide];
+  extern __shared__ __align__(16) float band[];  // band_quads float4s, then the slopes
   __shared__ float tile[kImgTile * kImgTile];
-  __shared__ __align__(16) float band[kBandFloats + 4];
   __shared__ PositionSetup sh;
   __shared__ int sh_lo[2], sh_hi[2];
   const int64_t s = blockIdx.y;
   const int n = G.n_side, W = G.det_w;
+  const int quads = band_quads(band_rows * W);
+  float* th = band + 4 * quads;
   const int row_begin = (int)blockIdx.x * bands_each * band_rows;
   const int row_end = min(row_begin + bands_each * band_rows, G.det_h);
   if (threadIdx.x < 64) {
@@ -355,7 +365,7 @@ __global__ __launch_bounds__(kThreads) void stem_dataset_kernel(const tg_stem_ge
     }
   }
   for (int k = threadIdx.x; k < n; k += kThreads) th[k] = slope_of(G, k);
-  for (int k = threadIdx.x; k < kBandFloats / 4 + 1; k += kThreads) ((float4*)band)[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int k = threadIdx.x; k < quads; k += kThreads) ((float4*)band)[k] = make_float4(0.f, 0.f, 0.f, 0.f);
   __syncthreads();
   const float a = sh.a[0], bx = sh.bx[0], by = sh.by[0];
   const int oy = sh.oy, ox = sh.ox;
@@ -1331,18 +1341,31 @@ extern "C" int tg_stem_dataset(const tg_stem_geometry* g, const double* params, 
   TG_REQUIRE(g->det_h > 0 && g->det_w > 0, "tg_stem_dataset: bad detector shape");
   TG_REQUIRE(g->det_w <= tg_stem_dataset_max_width(), "tg_stem_dataset: detector rows of %d pixels exceed %d", g->det_w,
              tg_stem_dataset_max_width());
-  // whole bands of a few rows; a multiple of four rows keeps every band of an
-  // aligned image aligned
-  int rows = kBandFloats / g->det_w;
-  if (rows > 4) rows -= rows % 4;
-  if (rows > g->det_h) rows = g->det_h;
-  // as many bands a workgroup as still leave four workgroups (what fits) for
-  // every CU: the set-up is paid once for them
-  const int64_t S = (int64_t)g->scan_h * g->scan_w, bands = tg::cdiv(g->det_h, rows);
-  const int64_t groups = std::min(bands, tg::cdiv(4LL * tg::cu_count(), S)), each = tg::cdiv(bands, groups);
+  // As many workgroups a position as run at a time (five a CU): a few positions
+  // are shared by several, and with many the set-up is paid once for all bands.
+  const int64_t S = (int64_t)g->scan_h * g->scan_w, W = g->det_w;
+  const int64_t share = std::min<int64_t>(16, std::max<int64_t>(1, 5LL * tg::cu_count() / S));
+  // Even bands of whole rows, no more than LDS holds and as many for each that
+  // shares them; a multiple of four rows keeps every band of an aligned image
+  // aligned.
+  const int64_t most = std::max<int64_t>(1, kBandFloats / W);
+  const int64_t want = tg::cdiv(tg::cdiv(g->det_h, most), share) * share;
+  int64_t rows = tg::cdiv(g->det_h, want);
+  rows = std::min((rows + 3) / 4 * 4, most > 4 ? most / 4 * 4 : most);
+  rows = std::min<int64_t>(rows, g->det_h);
+  const int64_t bands = tg::cdiv(g->det_h, rows), each = tg::cdiv(bands, std::min(bands, share));
   const dim3 grid((unsigned)tg::cdiv(bands, each), (unsigned)S);
-  hipLaunchKernelGGL(stem_dataset_kernel, grid, dim3(kThreads), 0, (hipStream_t)stream, *g, params, image, rows,
-                     (int)each, image4d);
+  // As much LDS as the detector and the rays take: the workgroups a CU holds at a
+  // time hide the set-up's latency, which is most of a small detector's time.
+  // Of workgroups with many bands no more than make the rounds even: 64x64
+  // positions of 256x256 pixels 193 us four a CU, 200 five a CU.
+  const int64_t own = 4608, all = 160 * 1024;  // the kernel's other LDS, a CU's
+  int64_t lds = (4 * (int64_t)band_quads((int)(rows * W)) + g->n_side) * (int64_t)sizeof(float);
+  const int64_t held = std::min<int64_t>(8, all / (lds + own)), cus = tg::cu_count(), count = (int64_t)grid.x * S;
+  const int64_t even = std::max<int64_t>(3, tg::cdiv(count, tg::cdiv(count, held * cus) * cus));
+  if (each >= 6 && even < held) lds = std::max(lds, all / (even + 1) - own + 1280);
+  hipLaunchKernelGGL(stem_dataset_kernel, grid, dim3(kThreads), (size_t)lds, (hipStream_t)stream, *g, params, image,
+                     (int)rows, (int)each, image4d);
   TG_LAUNCH_CHECK("stem_dataset_kernel launch");
   return TG_OK;
 }
