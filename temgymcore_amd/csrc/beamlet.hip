@@ -947,18 +947,19 @@ int splits_for(int64_t n, int64_t H, int64_t W) {
   const int64_t ntiles = tg::cdiv(H, kTileH) * tg::cdiv(W, kTileW);
   // Few beamlets: about six workgroups of 64x64 pixels a CU, down to where the
   // slices' own cost takes over: a start, and a partial image each, so slices of
-  // sqrt(n) beamlets, and of more above 10,000 pixels.  The sum's kernels, 256
+  // sqrt(n) beamlets, and of more above 60,000 pixels.  The sum's kernels, 256
   // beamlets a slice as a rule / slices of sqrt(n) whatever the pixels / this
-  // one, separable: 30 on 1024^2 24 / 61 / 29 us, 64 on 600 x 612 19 / 48 / 26,
-  // 300 on 600^2 24 / 48 / 31, 300 on 100^2 33 / 25 / 25; rotated: 30 on 1024^2 34 /
-  // 59 / 31, 300 on 600^2 31 / 56 / 31, 4,096 on 600 x 612 72 / 63 / 60, 500 on
-  // 300^2 130 / 39 / 51, 300 on 100^2 177 / 36 / 36, 64 on 64^2 99 / 27 / 27.
+  // one: tilted 64 on 600 x 612 40 / 34 / 27 us, 300 on 600^2 79 / 46 / 38 (with a
+  // 4-sigma cut 39 / 44 / 32), 2,048 on 500 x 612 141 / 75 / 78, 500 on 300^2
+  // 257 / 38 / 42, 300 on 100^2 166 / 27 / 29; separable 30 on 1024^2 24 / 61 / 29,
+  // 64 on 600 x 612 19 / 48 / 27.  (A sixth of that, from 10,000 pixels on: 2,048
+  // tilted ones 120, 500 on 300^2 70.)
   // Many separable ones: whole rounds of the matrix-core kernel's tiles (two
   // workgroups a CU at a time; tiles of uneven weight want some rounds), slices
   // of at least 600.  20,000 on 512^2: 32 slices, a round, 152 us, 39 slices
   // 212; 131,072 on 1024^2: 16 / 32 / 64 / 128 slices 2.50 / 2.15 / 2.15 /
   // 2.30 ms; 50,000 on 1000 x 300 533 / 468 us.
-  const double start = std::max(1.0, (double)H * (double)W * 1e-4);
+  const double start = std::max(1.0, (double)H * (double)W / 60000.0);
   const int64_t few = std::min<int64_t>(6LL * tg::cu_count() / ntiles, (int64_t)std::sqrt((double)n / start));
   const int64_t tiles = tg::cdiv(H, (int64_t)SepTile::TH) * tg::cdiv(W, (int64_t)SepTile::TW);
   const int64_t slots = 2LL * tg::cu_count();

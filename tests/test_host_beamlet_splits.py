@@ -23,12 +23,12 @@ def test_slices_are_bounded(seed):
 
 
 @pytest.mark.parametrize("n,height,width,most", [
-    (1, 600, 612, 1), (30, 1024, 1024, 1), (64, 600, 612, 1), (300, 600, 600, 2), (2000, 1024, 1024, 4),
+    (1, 600, 612, 1), (30, 1024, 1024, 1), (64, 600, 612, 3), (300, 600, 600, 7), (2000, 1024, 1024, 6),
     (64, 64, 64, 8), (300, 100, 100, 17),
 ])
 def test_a_slice_of_a_large_image_has_beamlets_enough(n, height, width, most):
-    """A slice of ten thousand pixels or fewer: sqrt(n) beamlets and more; of
-    larger images as many more as makes up for its partial image."""
+    """A slice of 60,000 pixels or fewer: sqrt(n) beamlets and more; of larger
+    images as many more as makes up for its partial image."""
     lib = _lib.load()
     autotune.clear()
     slices = lib.tg_beamlet_sum_workspace(n, height, width) - 256 * 4 - 96 * n
