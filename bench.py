@@ -716,7 +716,8 @@ def bench_beamlet(steps: int, warmup: int):
                 "event_ms_per_step": kern_ms, "graph_replay_ms_per_step": graph_ms, "beamlet_sum_event_ms": sum_ms,
                 "tile_sum": "matrix cores (separable beamlets)" if matrix else "VALU recurrence",
                 "kernels_per_step": "beamlet_coef_kernel + sep_flag_kernel + beamlet_sum_sep_kernel / "
-                                    "beamlet_sum_kernel (one exits at once) + split_sum_kernel",
+                                    "beamlet_sum_wide_kernel / beamlet_sum_kernel (those without work exit at "
+                                    "once) + split_sum_kernel",
                 "autotune": {"beamlet_path": {1: "auto", 2: "valu"}[tuned_path],
                              "path_candidate_ms": {{1: "auto", 2: "valu"}[k]: v for k, v in path_ms.items()},
                              "beamlet_splits": tuned_splits, "candidate_ms": tune_ms,
@@ -754,11 +755,12 @@ def _tile_pair_count(coef_bytes, n, H, W, tile=128):
     gamma, beta = rec["abg"][:, 2].astype(f32), rec["abg"][:, 1].astype(f32)
     tx0 = (np.arange(-(-W // tile)) * tile).astype(f32)
     ty0 = (np.arange(-(-H // tile)) * tile).astype(f32)
+    tx1, ty1 = np.minimum(tx0 + f32(tile), f32(W)) - f32(1), np.minimum(ty0 + f32(tile), f32(H)) - f32(1)
     total = 0
     for lo in range(0, n, 4096):
         sl = slice(lo, min(n, lo + 4096))
-        du = np.maximum(np.maximum(tx0[None, :] - cx[sl, None], cx[sl, None] - (tx0[None, :] + f32(tile - 1))), f32(0))
-        dv = np.maximum(np.maximum(ty0[None, :] - cy[sl, None], cy[sl, None] - (ty0[None, :] + f32(tile - 1))), f32(0))
+        du = np.maximum(np.maximum(tx0[None, :] - cx[sl, None], cx[sl, None] - tx1[None, :]), f32(0))
+        dv = np.maximum(np.maximum(ty0[None, :] - cy[sl, None], cy[sl, None] - ty1[None, :]), f32(0))
         gv = (gamma[sl, None] * dv).astype(np.float64) * dv  # fma(gamma dv, dv, du^2) in one rounding
         q = (gv[:, :, None] + (du * du).astype(np.float64)[:, None, :]).astype(f32)
         total += int((q <= beta[sl, None, None]).sum())
@@ -840,7 +842,7 @@ def bench_gauss_fit(steps: int, warmup: int):
                   "kernels": "fit_forward_kernel + fit_moment_kernel (whole step timed)",
                   "valu_busy_percent": _profiled("fit_forward_moment_kernels-gauss_fit_256.md", "valu_busy_percent"),
                   "valu_source": "profiles/fit_forward_moment_kernels-gauss_fit_256.md (VALUBusy PMC of the "
-                                 "forward kernel)"},
+                                 "forward kernel; it counts four cycles an instruction, and some take fewer)"},
         cpu_baseline=cpu,
     )
 

@@ -192,7 +192,7 @@ class ColumnMatch:
         f32 = dtype == torch.float32
         col.dtype = _lib.TG_F32 if f32 else _lib.TG_F64
         col.n = math.prod(shape)
-        # outputs share one allocation, each on a 16-byte boundary
+        # a cached call's outputs share one allocation, each on a 16-byte boundary
         size = 4 if f32 else 8
         self.row = -(-col.n // (16 // size)) * (16 // size)
         # immediates rounded once to the ray dtype, as in register programs

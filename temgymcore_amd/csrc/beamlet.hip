@@ -258,8 +258,8 @@ __global__ __launch_bounds__(kThreads) void beamlet_sum_kernel(const tg_beamlet_
 //
 // 131,072 beamlets, 1024^2, 4 sigma, the whole sum: 4.64 ms with f32 products,
 // now 2.17 ms (of which the search for the range is 0.02).  Bound: vector issue
-// (63% of the cycles, 520 instructions a chunk) and the matrix cores (46%)
-// together, at the 1.9 GHz that this mix runs at.
+// (63% of the cycles, 520 instructions a chunk) and the matrix cores (48%)
+// together, at the 1.7 to 1.9 GHz that this mix runs at.
 // ---------------------------------------------------------------------------
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));

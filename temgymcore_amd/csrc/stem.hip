@@ -1174,7 +1174,7 @@ __global__ __launch_bounds__(kThreads) void stem_fit_small_kernel(const tg_stem_
 // Bound: latency.  So the targets' loads come first, N of them a lane (as many
 // as the rays need where they are one tile), and one wavefront makes the
 // constants while the others fill the slopes.  With the terms and sums in one
-// launch, whole fits before / now: 13x21 positions, 62^2 rays, 3 cameras 13.7 /
+// launch, whole fits before / now: 13x21 positions, 46^2 rays, 3 cameras 13.7 /
 // 11.7 us; 7x13, 30^2, 3 12.4 / 9.4; 31x33, 30^2, 8 43.5 / 28.9; 5x5, 16^2, 1 11.5
 // / 8.4.
 template <int N>
